@@ -615,18 +615,17 @@ DVG_DEV void wave_combine_add(bool active, int key, const float (&v)[N], float *
             for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o, 64);
             sum[i] = x;
         }
-        // the destination of this key, as the leader computed it
+        // the destination of this key, as the leader computed it; the N contiguous sums go
+        // out as one atomic instruction of N lanes
         const unsigned long long addr =
             ((unsigned long long)(unsigned)__shfl((int)((unsigned long long)dst_of_key_leader >> 32), leader, 64)
              << 32) |
             (unsigned)__shfl((int)((unsigned long long)dst_of_key_leader & 0xffffffffull), leader, 64);
-        const int nu = __shfl(n_used, leader, 64);
-        if (lane == leader) {
-            float *d = (float *)addr;
+        const int nu = N == 1 ? 1 : __shfl(n_used, leader, 64);
+        float mine_sum = sum[0];
 #pragma unroll
-            for (int i = 0; i < N; i++)
-                if (i < nu) aadd(d + i, sum[i]);
-        }
+        for (int i = 1; i < N; i++) mine_sum = lane == i ? sum[i] : mine_sum;
+        if (lane < nu) aadd((float *)addr + lane, mine_sum);
         pending &= ~m;
     }
 }
@@ -737,6 +736,97 @@ DVG_DEV void accumulate_boundary_gradient_wave(const DevScene &S, bool active, i
     }
 }
 
+// d_sample_paint for a whole wave (every lane calls it; lanes without a paint adjoint pass
+// on = false): lanes that add to the same stops or the same gradient end points add their
+// values together before the atomics.  A drawing's gradient fill covers thousands of samples
+// that all add to its few stops.  A stop offset order that lets one value fall into several
+// intervals of a radial paint (possible only when the offsets are not sorted) adds the later
+// ones per lane.
+DVG_DEV void d_sample_paint_wave(const DevScene &S, bool on, int type, int off, int ns, V2 pt, V4 d_color,
+                                 float *d_translation) {
+    // the colour that receives all of d_color: a constant paint, the first stop before the
+    // first offset, the last stop past the last (and, for radial paints, always)
+    int full = on ? off : -1;
+    const bool grad = on && type != 0;
+    if (__any(grad)) {
+        float geo[4] = {0.f, 0.f, 0.f, 0.f}, offs[2] = {0.f, 0.f}, cols[8];
+#pragma unroll
+        for (int k = 0; k < 8; k++) cols[k] = 0.f;
+        int at = -1;
+        if (grad) {
+            const float *c = S.color + off;
+            const float *offsets = c + 4;
+            const float *colors = c + 4 + ns;
+            const V2 a{c[0], c[1]}, b{c[2], c[3]};
+            V2 normalized_offset{0, 0}, offset{0, 0};
+            float t;
+            if (type == 1) {
+                t = dot(pt - a, b - a) / fmax_r(dot(b - a, b - a), 1e-3f);
+            } else {
+                offset = pt - a;
+                normalized_offset = vdivv(offset, b);
+                t = len(normalized_offset);
+            }
+            full = off + 4 + ns + 4 * (ns - 1);
+            const bool before = t < offsets[0];
+            if (before) full = off + 4 + ns;
+            for (int i = 0; i < ns - 1 && !before; i++) {
+                const float oc = offsets[i], ox = offsets[i + 1];
+                if (!(t >= oc && t < ox)) continue;
+                const V4 cc = stop_color(colors, i), cn = stop_color(colors, i + 1);
+                const float tt = (t - oc) / (ox - oc);
+                const float d_tt = vsum(d_color * (cn - cc));
+                const float d_ox = -d_tt * tt / (ox - oc);
+                const float d_oc = d_tt * ((tt - 1.f) / (ox - oc));
+                const float d_t = d_tt / (ox - oc);
+                const V4 dc = d_color * (1 - tt), dn = d_color * tt;
+                V2 d_a, d_b;
+                if (type == 1) {
+                    const float l = fmax_r(dot(b - a, b - a), 1e-3f);
+                    d_a = vdiv(d_t * (-(pt - a) - (b - a)), l);
+                    d_b = vdiv(d_t * (pt - a), l);
+                    const float d_l = -d_t * t / l;
+                    if (dot(b - a, b - a) > 1e-3f) {
+                        d_a += 2 * d_l * (a - b);
+                        d_b += 2 * d_l * (b - a);
+                    }
+                    if (d_translation) aadd2(d_translation, d_a + d_b);
+                } else {
+                    const V2 d_no = d_length(normalized_offset, d_t);
+                    d_a = -vdivv(d_no, b);
+                    d_b = vdivv((-d_no) * offset, b * b);
+                    if (d_translation) aadd2(d_translation, d_a);
+                }
+                if (at < 0) {
+                    at = i;
+                    geo[0] = d_a.x, geo[1] = d_a.y, geo[2] = d_b.x, geo[3] = d_b.y;
+                    offs[0] = d_oc, offs[1] = d_ox;
+                    cols[0] = dc.x, cols[1] = dc.y, cols[2] = dc.z, cols[3] = dc.w;
+                    cols[4] = dn.x, cols[5] = dn.y, cols[6] = dn.z, cols[7] = dn.w;
+                } else {
+                    float *d = S.d_color + off;
+                    aadd2(d, d_a);
+                    aadd2(d + 2, d_b);
+                    aadd(d + 4 + i, d_oc);
+                    aadd(d + 4 + i + 1, d_ox);
+                    aadd4(d + 4 + ns + 4 * i, dc);
+                    aadd4(d + 4 + ns + 4 * (i + 1), dn);
+                }
+                if (type == 1) {
+                    full = -1;
+                    break;
+                }
+            }
+        }
+        const bool in = at >= 0;
+        wave_combine_add<4>(in, off, geo, S.d_color + (in ? off : 0));
+        wave_combine_add<2>(in, off + 4 + at, offs, S.d_color + (in ? off + 4 + at : 0));
+        wave_combine_add<8>(in, off + 4 + ns + 4 * at, cols, S.d_color + (in ? off + 4 + ns + 4 * at : 0));
+    }
+    float v[4] = {d_color.x, d_color.y, d_color.z, d_color.w};
+    wave_combine_add<4>(full >= 0, full, v, S.d_color + (full >= 0 ? full : 0));
+}
+
 // d_compute_distance for a whole wave (every lane calls it; lanes without a distance
 // adjoint pass active = false): the values of the per-lane version, with the point,
 // shape-parameter and transform adjoints of lanes that share a segment, shape or group
@@ -778,8 +868,8 @@ DVG_DEV void d_compute_distance_wave(const DevScene &S, bool active, int g, int 
 }
 
 // composite_adjoint_prefiltered for a whole wave, lanes in lockstep by fragment position
-// (as composite_adjoint_wave): constant paints, stroke widths and distance adjoints are
-// combined across lanes.  Every lane must call it; lanes without fragments pass nf = 0.
+// (as composite_adjoint_wave): paints, stroke widths and distance adjoints are combined
+// across lanes.  Every lane must call it; lanes without fragments pass nf = 0.
 DVG_DEV V4 composite_adjoint_prefiltered_wave(const DevScene &S, const PFragRec *frags, int nf, V3 final_color,
                                               float final_alpha, V4 d_color, V2 pt, float *d_translation) {
     V3 d_final_color{d_color.x, d_color.y, d_color.z};
@@ -796,7 +886,7 @@ DVG_DEV V4 composite_adjoint_prefiltered_wave(const DevScene &S, const PFragRec 
         const bool on = i < nf;
         PFragRec f{};
         if (on) f = frags[i];
-        int g = 0, s = 0, type = -1, off = 0;
+        int g = 0, s = 0, type = -1, off = 0, ns = 0;
         bool paint_on = false, dist_on = false, sw_on = false;
         float d_d = 0.f, d_sw = 0.f;
         V4 dci{0, 0, 0, 0};
@@ -809,7 +899,6 @@ DVG_DEV V4 composite_adjoint_prefiltered_wave(const DevScene &S, const PFragRec 
             g = f.gid >> 1;
             s = f.shape_id;
             float d = f.distance;
-            int ns = 0;
             if (f.gid & 1) {
                 type = S.stroke_type[g];
                 off = S.stroke_off[g];
@@ -846,15 +935,10 @@ DVG_DEV V4 composite_adjoint_prefiltered_wave(const DevScene &S, const PFragRec 
                     dist_on = fabs((double)d_d) > 1e-10f && f.within;
                 }
             }
-            if (paint_on && type != 0) d_sample_paint(S, type, off, ns, pt, dci, d_translation);
             d_curr_color = d_prev_color;
             d_curr_alpha = d_prev_alpha;
         }
-        {
-            float v[4] = {dci.x, dci.y, dci.z, dci.w};
-            const bool konst = paint_on && type == 0;
-            wave_combine_add<4>(konst, on ? f.gid : 0, v, S.d_color + (konst ? off : 0));
-        }
+        d_sample_paint_wave(S, paint_on, type, off, ns, pt, dci, d_translation);
         d_compute_distance_wave(S, dist_on, g, s, pt, on ? f.closest : pt, f.info, d_d, d_translation);
         {
             float v[1] = {d_sw};
@@ -903,13 +987,10 @@ DVG_DEV V4 composite_adjoint_wave(const DevScene &S, const FragRec *frags, int n
                 off = S.fill_off[g];
                 ns = S.fill_ns[g];
             }
-            if (type != 0) d_sample_paint(S, type, off, ns, pt, dci, d_translation);
             d_curr_color = d_prev_color;
             d_curr_alpha = d_prev_alpha;
         }
-        float v[4] = {dci.x, dci.y, dci.z, dci.w};
-        const bool konst = on && type == 0;
-        wave_combine_add<4>(konst, on ? f.gid : 0, v, S.d_color + (konst ? off : 0));
+        d_sample_paint_wave(S, on, type, off, ns, pt, dci, d_translation);
     }
     return V4{d_curr_color.x, d_curr_color.y, d_curr_color.z, d_curr_alpha};
 }
