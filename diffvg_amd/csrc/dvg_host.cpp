@@ -610,9 +610,13 @@ int build_scene(const dvg_scene_desc &d, int gpu_index, SceneHost &sc) {
     sc.g_xform = sc.g_color + al(d.num_color_params);
     sc.g_filter = sc.g_xform + al(9 * (size_t)ng);
     sc.grad_floats = sc.g_filter + 64;
-    sc.grad = (float *)cache_alloc(sc.device, sc.grad_floats * sizeof(float), &sc.grad_granted);
+    int reps = 1;
+    while (reps < kGradReps && 2 * reps * sc.grad_floats <= kGradRepFloats) reps *= 2;
+    sc.grad = (float *)cache_alloc(sc.device, reps * sc.grad_floats * sizeof(float), &sc.grad_granted);
     if (!sc.grad) return set_error("out of device memory for the gradients");
-    if (int e = clear_device(sc.device, sc.grad, sc.grad_floats * sizeof(float))) return e;
+    if (int e = clear_device(sc.device, sc.grad, reps * sc.grad_floats * sizeof(float))) return e;
+    D.rep_mask = reps - 1;
+    D.rep_stride = (int)sc.grad_floats;
     D.d_params = sc.grad + sc.g_params;
     D.d_points = sc.grad + sc.g_points;
     D.d_thickness = sc.grad + sc.g_thick;

@@ -77,6 +77,13 @@ constexpr int kRefitGroupLane = 64;
 // a workgroup
 constexpr int kRefitSegCap = 512;
 
+// Copies of a scene's gradient block (DevScene::rep_mask): device-scope float atomics to one
+// address are taken one at a time (~12 ns each on an MI355X), so a scene of few parameters,
+// whose every workgroup adds to the same ones, gets up to kGradReps copies while they stay
+// within kGradRepFloats (256 KB); a scene of many parameters spreads its atomics by itself.
+constexpr int kGradReps = 32;
+constexpr size_t kGradRepFloats = size_t(1) << 16;
+
 constexpr int kErrInts = 16;  // ints of SceneHost::err
 
 struct SceneHost {
@@ -90,7 +97,7 @@ struct SceneHost {
     void *block = nullptr;        // scene arrays
     size_t block_bytes = 0, block_granted = 0;
     float *grad = nullptr;        // gradient arrays
-    size_t grad_floats = 0, grad_granted = 0;
+    size_t grad_floats = 0, grad_granted = 0;  // floats of one copy (DevScene::rep_mask)
     size_t g_params = 0, g_points = 0, g_thick = 0, g_sw = 0, g_color = 0, g_xform = 0, g_filter = 0;
     // [0] render conditions, [1] conditions found by dvg_scene_update, [2] parameter
     // version on the device (advanced by every update), [4..9] and [10..15] the key of the

@@ -715,7 +715,7 @@ DVG_DEV void color_bwd_tile(ColorBwdLds &L, const DevScene &S, const Geom &G, in
     if (threadIdx.x == 0) {
         float t = 0.f;
         for (int w = 0; w < kBlock / 64; w++) t += s_red[w];
-        if (t != 0.f) aadd(S.d_filter_radius, t);
+        if (t != 0.f) aadd(S.d_filter_radius + grad_copy(S), t);
     }
     // d_background: a sample without fragments assigns, one with fragments adds
     // (diffvg.cpp:650-656, 700-704); folded per pixel in sample order.
@@ -999,6 +999,37 @@ __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_EDGE
     __shared__ EdgeLds L;
     edge_chunk<BOTH>(L, S, G, blockIdx.x, edges, tile_off, tile_count, chunk_off, ntiles, sorted, bg, weight, d_img,
                      d_translation);
+}
+
+// Adds the gradient copies 1..rep_mask to the block and clears them (DevScene::rep_mask).
+// Exchanges and atomic adds: another render of the scene on another stream may be adding to
+// the copies, and what it adds after the exchange is folded by its own backward.
+// A workgroup folds 64 floats: wave w exchanges copies 1 + w, 5 + w, ... with all exchanges in
+// flight at once (one after another they would cost a memory round trip each), and the four
+// partial sums meet in LDS.
+DVG_DEV void fold_grads(const DevScene &S, float *grad, int base, float (*part)[64]) {
+    constexpr int kEach = kGradReps / 4;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = base + lane;
+    float v[kEach];
+#pragma unroll
+    for (int k = 0; k < kEach; k++) {
+        const int r = 1 + w + 4 * k;
+        v[k] = i < S.rep_stride && r <= S.rep_mask ? atomicExch(grad + (size_t)r * S.rep_stride + i, 0.f) : 0.f;
+    }
+    float sum = 0.f;
+#pragma unroll
+    for (int k = 0; k < kEach; k++) sum += v[k];
+    part[w][lane] = sum;
+    __syncthreads();
+    if (w == 0) {
+        sum = (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+        if (sum != 0.f) aadd(grad + i, sum);
+    }
+    __syncthreads();
+}
+__global__ __launch_bounds__(kBlock) void k_fold_grads(DevScene S, float *grad) {
+    __shared__ float part[4][64];
+    fold_grads(S, grad, blockIdx.x * 64, part);
 }
 
 // SDF (sample_distance, diffvg.cpp:709-775) -- a linear scan over groups, as the
@@ -1737,6 +1768,8 @@ int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
             k_sdf_tiled<<<ntiles, kBlock, 0, st>>>(S, G, a.render_sdf, a.d_render_sdf, a.d_translation);
         }
     }
+    if ((a.d_render_image || a.d_render_sdf) && S.rep_mask)
+        k_fold_grads<<<(unsigned)((S.rep_stride + 63) / 64), kBlock, 0, st>>>(S, sc.grad);
     DVG_CHECK(hipGetLastError());
     // nothing waits here: conditions the kernels flag are reported by scene_status
     return 0;
@@ -1960,6 +1993,15 @@ __global__ __launch_bounds__(kBlock) void kb_zero(const Job *jobs, const int *pr
         for (int i = b * kBlock + threadIdx.x; i < J.ntiles; i += nb * kBlock) J.tile_count[i] = 0;
     if (zero_grads && (J.d_img || J.d_sdf))
         for (int i = b * kBlock + threadIdx.x; i < J.grad_n; i += nb * kBlock) J.grad[i] = 0.f;
+}
+
+// one row of workgroups per job; a workgroup strides over the job's gradient block
+__global__ __launch_bounds__(kBlock) void kb_fold_grads(const Job *jobs) {
+    const Job &J = jobs[blockIdx.y];
+    if (!(J.d_img || J.d_sdf) || !J.S.rep_mask) return;
+    __shared__ float part[4][64];
+    for (int base = blockIdx.x * 64; base < J.S.rep_stride; base += gridDim.x * 64)
+        fold_grads(J.S, J.grad, base, part);
 }
 
 __global__ __launch_bounds__(kBlock) void kb_weight(const Job *jobs, const int *pref, int nj) {
@@ -2236,6 +2278,7 @@ struct BatchHost {
     // classes: [0] colour without prefiltering, [1] colour prefiltered, [2] SDF
     int cls_begin[4] = {0, 0, 0, 0};
     bool any_img[3] = {false, false, false}, any_dimg[3] = {false, false, false};
+    bool fold[3] = {false, false, false};  // some backward job's scene keeps gradient copies
     std::vector<int> pref;         // per class, per stage: (njobs_in_class + 1) entries
     std::vector<size_t> pref_off;  // offset into pref of (class, stage)
     std::vector<int> total;        // workgroups of (class, stage)
@@ -2399,6 +2442,7 @@ int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, i
         for (int k = B->cls_begin[c]; k < B->cls_begin[c + 1]; k++) {
             B->any_img[c] |= B->jobs[k].img != nullptr;
             B->any_dimg[c] |= B->jobs[k].d_img != nullptr;
+            B->fold[c] |= (B->jobs[k].d_img || B->jobs[k].d_sdf) && B->jobs[k].S.rep_mask;
         }
     B->pref_off.assign(3 * kNumStages, 0);
     B->total.assign(3 * kNumStages, 0);
@@ -2554,6 +2598,7 @@ int batch_render(BatchHost &B, hipStream_t st) {
         if (c == 2) {
             DVG_PROF(st, "kb_sdf");
             kb_sdf<<<T(kStSdf), kBlock, 0, st>>>(J, P(kStSdf), nj);
+            if (B.fold[c]) kb_fold_grads<<<dim3(8, (unsigned)nj), kBlock, 0, st>>>(J);
             continue;
         }
         {
@@ -2591,6 +2636,7 @@ int batch_render(BatchHost &B, hipStream_t st) {
                     if (T(kStChunk2)) kb_edge<true><<<T(kStChunk2), kBlock, 0, st>>>(J, P(kStChunk2), nj);
                 }
             }
+            if (B.fold[c]) kb_fold_grads<<<dim3(8, (unsigned)nj), kBlock, 0, st>>>(J);
         }
     }
     hipError_t e = hipGetLastError();

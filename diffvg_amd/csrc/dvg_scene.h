@@ -99,6 +99,10 @@ struct DevScene {
     float *d_color;
     float *d_xform;
     float *d_filter_radius;
+    // Copies of the gradient block, rep_mask + 1 (a power of two) at rep_stride floats: the
+    // first is the block itself, a backward's workgroups add to copy (workgroup & rep_mask)
+    // and the last kernel of the backward folds the others into the first and clears them.
+    int rep_mask, rep_stride;
 };
 
 }  // namespace dvg

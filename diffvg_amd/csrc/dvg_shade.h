@@ -590,6 +590,9 @@ DVG_DEV void accumulate_boundary_gradient(const DevScene &S, int g, int s, float
     for (int i = 0; i < 9; i++) aadd(dx + i, d_s2c.m[i]);
 }
 
+// Offset of the gradient copy this workgroup adds to (DevScene::rep_mask).
+DVG_DEV int grad_copy(const DevScene &S) { return (int)(blockIdx.x & (unsigned)S.rep_mask) * S.rep_stride; }
+
 // ---- wave-combined gradient scatter for boundary samples ----
 // Device-scope float atomics to ordinary device memory are resolved past the XCD's L2,
 // so the ~20 atomics per boundary sample dominate the edge kernel's memory traffic.  A
@@ -660,7 +663,7 @@ DVG_DEV void accumulate_boundary_gradient_wave(const DevScene &S, bool active, i
     }
     {
         float v[1] = {contrib};
-        wave_combine_add<1>(sw_active, s, v, S.d_stroke_width + (sw_active ? s : 0));
+        wave_combine_add<1>(sw_active, s, v, S.d_stroke_width + grad_copy(S) + (sw_active ? s : 0));
     }
     // shape parameters of circles, ellipses and rects go direct (few per scene)
     if (active && type == 0) {
@@ -713,7 +716,7 @@ DVG_DEV void accumulate_boundary_gradient_wave(const DevScene &S, bool active, i
         for (int j = 0; j < 4; j++) {
             bool on = pa && j <= k + 1;
             float v[2] = {w[j] * normal.x * contrib, w[j] * normal.y * contrib};
-            wave_combine_add<2>(on, seg, v, S.d_points + (on ? 2 * ii[j] : 0));
+            wave_combine_add<2>(on, seg, v, S.d_points + grad_copy(S) + (on ? 2 * ii[j] : 0));
         }
     }
     // shape_to_canvas adjoint, combined by group
@@ -732,7 +735,7 @@ DVG_DEV void accumulate_boundary_gradient_wave(const DevScene &S, bool active, i
 #pragma unroll
             for (int i = 0; i < 9; i++) m9[i] = 0.f;
         }
-        wave_combine_add<9>(active, g, m9, S.d_xform + (active ? 9 * g : 0));
+        wave_combine_add<9>(active, g, m9, S.d_xform + grad_copy(S) + (active ? 9 * g : 0));
     }
 }
 
@@ -819,12 +822,12 @@ DVG_DEV void d_sample_paint_wave(const DevScene &S, bool on, int type, int off, 
             }
         }
         const bool in = at >= 0;
-        wave_combine_add<4>(in, off, geo, S.d_color + (in ? off : 0));
-        wave_combine_add<2>(in, off + 4 + at, offs, S.d_color + (in ? off + 4 + at : 0));
-        wave_combine_add<8>(in, off + 4 + ns + 4 * at, cols, S.d_color + (in ? off + 4 + ns + 4 * at : 0));
+        wave_combine_add<4>(in, off, geo, S.d_color + grad_copy(S) + (in ? off : 0));
+        wave_combine_add<2>(in, off + 4 + at, offs, S.d_color + grad_copy(S) + (in ? off + 4 + at : 0));
+        wave_combine_add<8>(in, off + 4 + ns + 4 * at, cols, S.d_color + grad_copy(S) + (in ? off + 4 + ns + 4 * at : 0));
     }
     float v[4] = {d_color.x, d_color.y, d_color.z, d_color.w};
-    wave_combine_add<4>(full >= 0, full, v, S.d_color + (full >= 0 ? full : 0));
+    wave_combine_add<4>(full >= 0, full, v, S.d_color + grad_copy(S) + (full >= 0 ? full : 0));
 }
 
 // d_compute_distance for a whole wave (every lane calls it; lanes without a distance
@@ -856,14 +859,14 @@ DVG_DEV void d_compute_distance_wave(const DevScene &S, bool active, int g, int 
     for (int j = 0; j < 4; j++) {
         const bool on = act && a.pts.use[j];
         float v[2] = {a.pts.d[j].x, a.pts.d[j].y};
-        wave_combine_add<2>(on, a.seg, v, S.d_points + (on ? 2 * a.pts.idx[j] : 0));
+        wave_combine_add<2>(on, a.seg, v, S.d_points + grad_copy(S) + (on ? 2 * a.pts.idx[j] : 0));
     }
     {
         // circle: radius, centre; rect: p_min, p_max -- contiguous at the shape's offset
         const bool on = act && a.npar > 0;
-        wave_combine_add<4>(on, s, a.par, S.d_params + (on ? S.param_off[s] : 0), a.npar);
+        wave_combine_add<4>(on, s, a.par, S.d_params + grad_copy(S) + (on ? S.param_off[s] : 0), a.npar);
     }
-    wave_combine_add<9>(act, g, a.xform, S.d_xform + (act ? 9 * g : 0));
+    wave_combine_add<9>(act, g, a.xform, S.d_xform + grad_copy(S) + (act ? 9 * g : 0));
     if (act && d_translation) aadd2(d_translation, -a.d_pt);
 }
 
@@ -942,7 +945,7 @@ DVG_DEV V4 composite_adjoint_prefiltered_wave(const DevScene &S, const PFragRec 
         d_compute_distance_wave(S, dist_on, g, s, pt, on ? f.closest : pt, f.info, d_d, d_translation);
         {
             float v[1] = {d_sw};
-            wave_combine_add<1>(sw_on, s, v, S.d_stroke_width + (sw_on ? s : 0));
+            wave_combine_add<1>(sw_on, s, v, S.d_stroke_width + grad_copy(S) + (sw_on ? s : 0));
         }
     }
     return V4{d_curr_color.x, d_curr_color.y, d_curr_color.z, d_curr_alpha};
