@@ -48,6 +48,15 @@ constexpr int kFragMaxGroups = 32768;  // group ids 2 g + is_stroke are kept in 
 // shape, signed distance, closest point, path position and whether a distance was found
 constexpr int kPFragSlots = 8;
 constexpr int kPFragWords = 9;
+// Boundary adjoints of circles, ellipses and rects (three or four parameters each) are
+// combined across a wave's lanes, up to this many samples per shape of the scene: 40 shapes
+// at 333x217, 3x2 samples: k_edge 3.34 -> 0.49 ms.  Past it every lane adds its own, as
+// before (~12 ns per sample: 10 ms for one circle and 262,144 samples, 0.9 combined),
+// because there the two forms differ by more than float rounding of one sum: adding N terms
+// of one sign one by one loses up to 2.3e-5 of the sum at 9,000 samples, 5e-5 at 32,000,
+// 3.4e-4 at 262,144 (12-60 seeds), and results of large few-primitive renders are kept as
+// they were.
+constexpr int64_t kPrimDirect = 12288;
 // Waves per SIMD each heavy shading kernel is compiled for, i.e. its register budget
 // (512 / waves VGPRs per lane; beyond it the compiler spills to scratch).  Chosen by
 // measurement on the 300-path and 2,048-stroke scenes: these kernels wait on memory and
@@ -111,6 +120,7 @@ struct Geom {
     float sx_scale, sy_scale;  // canvas / render
     float margin;
     int echunk;  // boundary samples per edge workgroup: kEdgeChunk or kBlock
+    int prim_direct;  // primitives' boundary adjoints are added sample by sample (kPrimDirect)
 };
 
 // Workgroup-shared storage of the tiled stages.  Each stage function takes its own
@@ -985,7 +995,7 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
         }
         BoundaryData bd = active ? es.data : BoundaryData{0, 0, 0.f, 0};
         accumulate_boundary_gradient_wave(S, active, active ? es.group : 0, active ? es.shape : 0, contrib,
-                                          active ? es.t : 0.f, n, bd, active ? V2{es.lx, es.ly} : V2{0, 0});
+                                          active ? es.t : 0.f, n, bd, active ? V2{es.lx, es.ly} : V2{0, 0}, G.prim_direct != 0);
         if (active && d_translation) {
             aadd(d_translation + 2 * (by * G.W + bx) + 0, n.x * contrib);
             aadd(d_translation + 2 * (by * G.W + bx) + 1, n.y * contrib);
@@ -1550,6 +1560,7 @@ static Geom make_geom(const SceneHost &sc, const dvg_render_args &a) {
     G.tw = tw;
     G.th = th;
     G.echunk = sc.edge_spw == 64 ? kBlock : kEdgeChunk;
+    G.prim_direct = (int64_t)G.W * G.H * G.spp > kPrimDirect * sc.num_shapes;
     G.tiles_x = (G.W + tw - 1) / tw;
     G.tiles_y = (G.H + th - 1) / th;
     G.sx_scale = (float)sc.cw / (float)G.W;

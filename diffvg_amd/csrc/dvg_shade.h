@@ -637,7 +637,7 @@ DVG_DEV void wave_combine_add(bool active, int key, const float (&v)[N], float *
 // the per-sample version, with the stroke-width, path-point and transform adjoints of
 // lanes that share a shape, segment or group added together before the atomics.
 DVG_DEV void accumulate_boundary_gradient_wave(const DevScene &S, bool active, int g, int s, float contrib, float t,
-                                               V2 normal, const BoundaryData &bd, V2 local_pt) {
+                                               V2 normal, const BoundaryData &bd, V2 local_pt, bool prim_direct) {
     int type = active ? S.shape_type[s] : -1;
     // strokes: per-point thickness goes direct (rare); stroke width combined by shape
     bool sw_active = active && bd.is_stroke && !(type == 2 && S.has_thick[s]);
@@ -665,27 +665,56 @@ DVG_DEV void accumulate_boundary_gradient_wave(const DevScene &S, bool active, i
         float v[1] = {contrib};
         wave_combine_add<1>(sw_active, s, v, S.d_stroke_width + grad_copy(S) + (sw_active ? s : 0));
     }
-    // shape parameters of circles, ellipses and rects go direct (few per scene)
-    if (active && type == 0) {
-        float *dp = S.d_params + S.param_off[s];
-        aadd2(dp + 1, normal * contrib);
-        aadd(dp, contrib);
-    } else if (active && type == 1) {
-        float *dp = S.d_params + S.param_off[s];
-        const float tp = 2 * (float)kPi;
-        aadd2(dp + 2, normal * contrib);
-        aadd(dp + 0, (float)(cos((double)(tp * t)) * normal.x * contrib));
-        aadd(dp + 1, (float)(sin((double)(tp * t)) * normal.y * contrib));
-    } else if (active && type == 3) {
-        float *dp = S.d_params + S.param_off[s];
-        if (normal == V2{-1, 0})
-            aadd(dp + 0, -contrib);
-        else if (normal == V2{1, 0})
-            aadd(dp + 2, contrib);
-        else if (normal == V2{0, -1})
-            aadd(dp + 1, -contrib);
-        else if (normal == V2{0, 1})
-            aadd(dp + 3, contrib);
+    // shape parameters of circles, ellipses and rects: combined by shape, or (prim_direct,
+    // see kPrimDirect) added by every lane
+    if (prim_direct) {
+        if (active && type == 0) {
+            float *dp = S.d_params + S.param_off[s];
+            aadd2(dp + 1, normal * contrib);
+            aadd(dp, contrib);
+        } else if (active && type == 1) {
+            float *dp = S.d_params + S.param_off[s];
+            const float tp = 2 * (float)kPi;
+            aadd2(dp + 2, normal * contrib);
+            aadd(dp + 0, (float)(cos((double)(tp * t)) * normal.x * contrib));
+            aadd(dp + 1, (float)(sin((double)(tp * t)) * normal.y * contrib));
+        } else if (active && type == 3) {
+            float *dp = S.d_params + S.param_off[s];
+            if (normal == V2{-1, 0})
+                aadd(dp + 0, -contrib);
+            else if (normal == V2{1, 0})
+                aadd(dp + 2, contrib);
+            else if (normal == V2{0, -1})
+                aadd(dp + 1, -contrib);
+            else if (normal == V2{0, 1})
+                aadd(dp + 3, contrib);
+        }
+    } else {
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+        const bool on = active && type != 2;
+        int n = 4;
+        if (on && type == 0) {
+            v[0] = contrib;
+            v[1] = normal.x * contrib;
+            v[2] = normal.y * contrib;
+            n = 3;
+        } else if (on && type == 1) {
+            const float tp = 2 * (float)kPi;
+            v[0] = (float)(cos((double)(tp * t)) * normal.x * contrib);
+            v[1] = (float)(sin((double)(tp * t)) * normal.y * contrib);
+            v[2] = normal.x * contrib;
+            v[3] = normal.y * contrib;
+        } else if (on) {
+            if (normal == V2{-1, 0})
+                v[0] = -contrib;
+            else if (normal == V2{1, 0})
+                v[2] = contrib;
+            else if (normal == V2{0, -1})
+                v[1] = -contrib;
+            else if (normal == V2{0, 1})
+                v[3] = contrib;
+        }
+        wave_combine_add<4>(on, s, v, S.d_params + grad_copy(S) + (on ? S.param_off[s] : 0), n);
     }
     // path control points, combined by segment.  A segment's points are not contiguous
     // (the last point of a closed path's last segment wraps to its first), so each of the
