@@ -615,6 +615,10 @@ int build_scene(const dvg_scene_desc &d, int gpu_index, SceneHost &sc) {
     sc.grad = (float *)cache_alloc(sc.device, reps * sc.grad_floats * sizeof(float), &sc.grad_granted);
     if (!sc.grad) return set_error("out of device memory for the gradients");
     if (int e = clear_device(sc.device, sc.grad, reps * sc.grad_floats * sizeof(float))) return e;
+    D.wave_ok = nseg <= kWaveMaxSegs;
+    for (int g = 0; g < ng; g++) D.wave_ok &= d.group_num_shapes[g] == 1;
+    for (int s = 0; s < ns; s++)
+        if (shape_type[s] == 2) D.wave_ok &= !approx[s] && d.path_num_base_points[s] <= kWaveMaxPathSegs;
     D.rep_mask = reps - 1;
     D.rep_stride = (int)sc.grad_floats;
     D.d_params = sc.grad + sc.g_params;

@@ -85,6 +85,13 @@ constexpr int64_t kPrimDirect = 12288;
 #ifndef DVG_WAVES_EDGE
 #define DVG_WAVES_EDGE 6
 #endif
+// the kernels with the wave-cooperative coverage tests
+#ifndef DVG_WAVES_COLOR_WAVE
+#define DVG_WAVES_COLOR_WAVE 5
+#endif
+#ifndef DVG_WAVES_EDGE_WAVE
+#define DVG_WAVES_EDGE_WAVE 4
+#endif
 // the edge kernel with both sides of a sample per lane keeps two compositors live
 #ifndef DVG_WAVES_EDGE_BOTH
 #define DVG_WAVES_EDGE_BOTH 5
@@ -139,7 +146,14 @@ struct ColorBwdLds {
 struct EdgeLds {
     CandLds c;
     int perm[kBlock];
-    int key[kBlock];
+};
+struct ColorWaveLds {
+    CandLds c;
+    WaveLds<1> w[kBlock / 64];
+};
+struct EdgeWaveLds {
+    EdgeLds e;
+    WaveLds<2> w[kBlock / 64];
 };
 struct SdfLds {
     CandLds c;
@@ -579,6 +593,51 @@ __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_COLOR_PRE : DVG_WAVES_COLOR
     color_tile<PRE>(L, S, G, blockIdx.x, bg, colors, err, frag, pkeep);
 }
 
+// color_tile<0> with the wave-cooperative coverage tests (DevScene::wave_ok): the same
+// fragments in the same order.
+DVG_DEV void color_tile_wave(ColorWaveLds &L, const SceneRef &R, const Geom &G, int tile, const float *bg,
+                             float4 *colors, int *err, uint16_t *frag) {
+    const DevScene S = R.get();
+    if (frag && tile == 0 && threadIdx.x == 0) key_of(G, err + 2, err + 4);
+    const int tx = tile % G.tiles_x, ty = tile / G.tiles_x;
+    int x, y, sx, sy, idx;
+    const bool valid = tile_sample(G, tx, ty, threadIdx.x, x, y, sx, sy, idx);
+    V2 pt{0, 0};
+    if (valid) pt = to_canvas(S, G, sample_pos(G, x, y, sx, sy, idx, false));
+    const bool has_bg = bg != nullptr;
+    const V4 bgc = (valid && has_bg) ? load_bg(bg, y * G.W + x) : V4{0, 0, 0, 0};
+    Compositor comp;
+    comp.init(has_bg, bgc);
+    const float4 tb = tile_box(S, G, tx, ty, 0.f);
+    const size_t nsamp = (size_t)G.W * G.H * G.spp;
+    for (int c0 = 0; c0 < S.ng; c0 += kCandCap) {
+        const int n = __builtin_amdgcn_readfirstlane(
+            build_candidates(S, tb, c0, min(S.ng, c0 + kCandCap), L.c.list, L.c.w));
+        wave_shade<1>(R, L.w[threadIdx.x >> 6], L.c.list, n, valid, pt, pt, pt, 0.f, 0.f,
+                      [&](const DevScene &S, int g, bool stroke, bool on, bool) {
+                          const int type = stroke ? S.stroke_type[g] : S.fill_type[g];
+                          const int off = stroke ? S.stroke_off[g] : S.fill_off[g];
+                          const int ns = stroke ? S.stroke_ns[g] : S.fill_ns[g];
+                          if (on) {
+                              if (frag && comp.nf < kFragSlots)
+                                  frag[(size_t)comp.nf * nsamp + idx] = (uint16_t)(2 * g + (stroke ? 1 : 0));
+                              comp.add(sample_paint(S, type, off, ns, pt), g, -1);
+                          }
+                      });
+        if (c0 + kCandCap < S.ng) __syncthreads();
+    }
+    if (valid) {
+        const V4 c = comp.result(has_bg, bgc);
+        colors[idx] = make_float4(c.x, c.y, c.z, c.w);
+        if (frag) frag[(size_t)kFragSlots * nsamp + idx] = (uint16_t)min(comp.nf, 65535);
+    }
+}
+__global__ __launch_bounds__(kBlock, DVG_WAVES_COLOR_WAVE) void k_color_wave(DevScene S, Geom G, const float *bg,
+                                                                            float4 *colors, int *err, uint16_t *frag) {
+    __shared__ ColorWaveLds L;
+    color_tile_wave(L, scene_argument(), G, blockIdx.x, bg, colors, err, frag);
+}
+
 DVG_DEV void resolve_pixel(const DevScene &S, const Geom &G, int pix, int prefilter, const float *weight,
                            const float4 *colors, float *out) {
     if (pix >= G.W * G.H) return;
@@ -840,11 +899,13 @@ __global__ __launch_bounds__(kBlock) void k_edge_bin(int count, const int *edge_
 // diffvg.cpp:1388-1475, evaluates the inside and the outside point): false -- lanes 2i and
 // 2i + 1 shade the inside and the outside point of sample i (kEdgeChunk samples, less
 // state per lane); true -- one lane shades both points of its sample (kBlock samples).
-template <bool BOTH>
+// WAVE (with BOTH): the wave-cooperative coverage tests (dvg_wave.h, `W`), which test both
+// points of a sample at once where one decision holds for both.
+template <bool BOTH, bool WAVE = false>
 DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk, const EdgeSample *edges,
                         const int *tile_off, const int *tile_count, const int *chunk_off, int ntiles,
                         const int *sorted, const float *bg, const float *weight, const float *d_img,
-                        float *d_translation) {
+                        float *d_translation, SceneRef R = {}, WaveLds<2> *W = nullptr) {
     constexpr int kChunk = BOTH ? kBlock : kEdgeChunk;
     int *s_list = L.c.list;
     int *s_w = L.c.w;
@@ -871,7 +932,7 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
         // The chunk's samples in order of their shape (stable): samples of one boundary
         // share a wave, so fewer waves run the deep part of the winding test for a curve
         // close to one of their points, and the gradient scatter combines more lanes.
-        int *s_key = L.key;
+        int *s_key = s_list;  // free until the first candidate list is built
         const int nvalid = min(kChunk, cnt - b0);
         if (threadIdx.x < kChunk)
             s_key[threadIdx.x] = (int)threadIdx.x < nvalid ? edges[sorted[off + b0 + threadIdx.x]].shape : INT_MAX;
@@ -936,7 +997,7 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
             cin = mine;
             cout = other;
         } else {
-            V2 pin{0, 0}, pout{0, 0};
+            V2 pin{0, 0}, pout{0, 0}, pmid{0, 0};
             Compositor ci, co;
             {
                 EdgeSample es0{};
@@ -945,6 +1006,7 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
                 V2 qi = bp - 1e-4f * n0, qo = bp + 1e-4f * n0;
                 pin = V2{qi.x * S.cw, qi.y * S.ch};
                 pout = V2{qo.x * S.cw, qo.y * S.ch};
+                pmid = V2{bp.x * S.cw, bp.y * S.ch};
                 if (valid) {
                     tgroup = es0.group;
                     tshape = es0.shape;
@@ -954,16 +1016,35 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
                 ci.init(has_bg, bg0);
                 co.init(has_bg, bg0);
             }
-            EdgeQuery qin{tgroup, tshape, false};
-            EdgeQuery qout = qin;
+            // a group of one shape whose shape is hit also adds a fragment, so the hits that
+            // the coverage tests raise themselves only matter for groups of several shapes
             bool hin = false, hout = false;
-            for (int c0 = 0; c0 < S.ng; c0 += kCandCap) {
-                int nc = build_candidates(S, tb, c0, min(S.ng, c0 + kCandCap), s_list, s_w);
-                if (valid) {
-                    shade_list(S, pin, s_list, nc, ci, &qin, hin);
-                    shade_list(S, pout, s_list, nc, co, &qout, hout);
+            if constexpr (WAVE) {
+                for (int c0 = 0; c0 < S.ng; c0 += kCandCap) {
+                    const int nc = __builtin_amdgcn_readfirstlane(
+                        build_candidates(S, tb, c0, min(S.ng, c0 + kCandCap), s_list, s_w));
+                    wave_shade<2>(R, W[threadIdx.x >> 6], s_list, nc, valid, pin, pout, pmid, 1.01e-4f * S.cw,
+                                  1.01e-4f * S.ch, [&](const DevScene &S, int g, bool stroke, bool on_in,
+                                                     bool on_out) {
+                                      const int type = stroke ? S.stroke_type[g] : S.fill_type[g];
+                                      const int off = stroke ? S.stroke_off[g] : S.fill_off[g];
+                                      const int ns = stroke ? S.stroke_ns[g] : S.fill_ns[g];
+                                      if (on_in) ci.add(sample_paint(S, type, off, ns, pin), g, tgroup);
+                                      if (on_out) co.add(sample_paint(S, type, off, ns, pout), g, tgroup);
+                                  });
+                    if (c0 + kCandCap < S.ng) __syncthreads();
                 }
-                if (c0 + kCandCap < S.ng) __syncthreads();
+            } else {
+                EdgeQuery qin{tgroup, tshape, false};
+                EdgeQuery qout = qin;
+                for (int c0 = 0; c0 < S.ng; c0 += kCandCap) {
+                    int nc = build_candidates(S, tb, c0, min(S.ng, c0 + kCandCap), s_list, s_w);
+                    if (valid) {
+                        shade_list(S, pin, s_list, nc, ci, &qin, hin);
+                        shade_list(S, pout, s_list, nc, co, &qout, hout);
+                    }
+                    if (c0 + kCandCap < S.ng) __syncthreads();
+                }
             }
             asm volatile("" ::: "memory");  // read the sample again, do not keep it live
             if (valid) es = edges[eidx];
@@ -1009,6 +1090,14 @@ __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_EDGE
     __shared__ EdgeLds L;
     edge_chunk<BOTH>(L, S, G, blockIdx.x, edges, tile_off, tile_count, chunk_off, ntiles, sorted, bg, weight, d_img,
                      d_translation);
+}
+
+__global__ __launch_bounds__(kBlock, DVG_WAVES_EDGE_WAVE) void k_edge_wave(
+    DevScene S, Geom G, const EdgeSample *edges, const int *tile_off, const int *tile_count, const int *chunk_off,
+    int ntiles, const int *sorted, const float *bg, const float *weight, const float *d_img, float *d_translation) {
+    __shared__ EdgeWaveLds L;
+    edge_chunk<true, true>(L.e, S, G, blockIdx.x, edges, tile_off, tile_count, chunk_off, ntiles, sorted, bg, weight,
+                           d_img, d_translation, scene_argument(), L.w);
 }
 
 // Adds the gradient copies 1..rep_mask to the block and clears them (DevScene::rep_mask).
@@ -1559,7 +1648,7 @@ static Geom make_geom(const SceneHost &sc, const dvg_render_args &a) {
     if (th < 1) th = 1;
     G.tw = tw;
     G.th = th;
-    G.echunk = sc.edge_spw == 64 ? kBlock : kEdgeChunk;
+    G.echunk = sc.dev.wave_ok || sc.edge_spw == 64 ? kBlock : kEdgeChunk;
     G.prim_direct = (int64_t)G.W * G.H * G.spp > kPrimDirect * sc.num_shapes;
     G.tiles_x = (G.W + tw - 1) / tw;
     G.tiles_y = (G.H + th - 1) / th;
@@ -1699,6 +1788,8 @@ int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
                 DVG_PROF(st, "k_color");
                 if (pre)
                     k_color<1><<<ntiles, kBlock, 0, st>>>(S, G, a.background_image, ws.colors, sc.err, nullptr, pkeep);
+                else if (S.wave_ok)
+                    k_color_wave<<<ntiles, kBlock, 0, st>>>(S, G, a.background_image, ws.colors, sc.err, frag);
                 else
                     k_color<0><<<ntiles, kBlock, 0, st>>>(S, G, a.background_image, ws.colors, sc.err, frag, nullptr);
             }
@@ -1755,7 +1846,11 @@ int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
                     DVG_PROF(st, "k_edge");
                     // at most one partial chunk per tile plus nsamp / echunk full ones
                     unsigned grid = (unsigned)(ntiles + (nsamp + G.echunk - 1) / G.echunk);
-                    if (G.echunk == kBlock)
+                    if (S.wave_ok)
+                        k_edge_wave<<<grid, kBlock, 0, st>>>(S, G, ws.edges, ws.tile_off, ws.tile_count, ws.chunk_off,
+                                                             ntiles, ws.edge_sorted, a.background_image, ws.weight,
+                                                             a.d_render_image, a.d_translation);
+                    else if (G.echunk == kBlock)
                         k_edge<true><<<grid, kBlock, 0, st>>>(S, G, ws.edges, ws.tile_off, ws.tile_count,
                                                               ws.chunk_off, ntiles, ws.edge_sorted,
                                                               a.background_image, ws.weight, a.d_render_image,
@@ -1980,8 +2075,10 @@ struct Job {
     int *pkeep;      // its kept prefiltered fragments, or null
 };
 
-// kStChunk / kStChunk2: edge chunks of the jobs with one side / both sides per lane
-enum { kStPix = 0, kStTile, kStSamp, kStChunk, kStSdf, kStZero, kStChunk2, kNumStages };
+// kStChunk / kStChunk2: edge chunks of the jobs with one side / both sides per lane;
+// kStChunkW: of the jobs with wave-cooperative tests; kStTileF / kStTileW: tiles of the
+// colour forward of the others / of those
+enum { kStPix = 0, kStTile, kStSamp, kStChunk, kStSdf, kStZero, kStChunk2, kStChunkW, kStTileF, kStTileW, kNumStages };
 
 // prefix arrays: pref[stage * (nj + 1) + k] = first workgroup of job k in that stage
 DVG_DEV int find_job(const int *pref, int nj, int blk) {
@@ -2029,6 +2126,14 @@ __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_BATCH_COLOR_PRE : DVG_WAVES
     __shared__ CandLds L;
     color_tile<PRE>(L, J.S, J.G, blockIdx.x - pref[j], J.bg, J.colors, J.err, PRE ? nullptr : J.frag,
                     PRE ? J.pkeep : nullptr);
+}
+
+__global__ __launch_bounds__(kBlock, DVG_WAVES_COLOR_WAVE) void kb_color_wave(const Job *jobs, const int *pref, int nj) {
+    int j = find_job(pref, nj, blockIdx.x);
+    const Job &J = jobs[j];
+    if (!J.img) return;
+    __shared__ ColorWaveLds L;
+    color_tile_wave(L, SceneRef{(uint64_t)&J.S}, J.G, blockIdx.x - pref[j], J.bg, J.colors, J.err, J.frag);
 }
 
 __global__ __launch_bounds__(kBlock) void kb_resolve(const Job *jobs, const int *pref, int nj) {
@@ -2082,6 +2187,15 @@ __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_BATC
     __shared__ EdgeLds L;
     edge_chunk<BOTH>(L, J.S, J.G, blockIdx.x - pref[j], J.edges, J.tile_off, J.tile_count, J.chunk_off, J.ntiles,
                      J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr);
+}
+
+__global__ __launch_bounds__(kBlock, DVG_WAVES_EDGE_WAVE) void kb_edge_wave(const Job *jobs, const int *pref, int nj) {
+    int j = find_job(pref, nj, blockIdx.x);
+    const Job &J = jobs[j];
+    if (!J.d_img) return;
+    __shared__ EdgeWaveLds L;
+    edge_chunk<true, true>(L.e, J.S, J.G, blockIdx.x - pref[j], J.edges, J.tile_off, J.tile_count, J.chunk_off,
+                           J.ntiles, J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr, SceneRef{(uint64_t)&J.S}, L.w);
 }
 
 __global__ __launch_bounds__(kBlock, DVG_WAVES_SDF) void kb_sdf(const Job *jobs, const int *pref, int nj) {
@@ -2441,10 +2555,14 @@ int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, i
             case kStPix: return color ? (J.npix + kBlock - 1) / kBlock : 0;
             case kStTile: return color ? J.ntiles : 0;
             case kStSamp: return edges ? (J.nsamp + kBlock - 1) / kBlock : 0;
+            case kStTileF: return J.img && (J.pre || !J.S.wave_ok) ? J.ntiles : 0;
+            case kStTileW: return J.img && !J.pre && J.S.wave_ok ? J.ntiles : 0;
+            case kStChunkW:
+                return edges && J.S.wave_ok ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
             case kStChunk:
                 return edges && J.G.echunk != kBlock ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
             case kStChunk2:
-                return edges && J.G.echunk == kBlock ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
+                return edges && J.G.echunk == kBlock && !J.S.wave_ok ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
             case kStSdf: return sdf ? (J.eval ? (J.num_eval + kBlock - 1) / kBlock : J.ntiles) : 0;
             default: return std::max(1, std::min(64, (std::max(J.grad_n, J.ntiles) + kBlock - 1) / kBlock));
         }
@@ -2620,9 +2738,10 @@ int batch_render(BatchHost &B, hipStream_t st) {
             {
                 DVG_PROF(st, "kb_color");
                 if (c == 1)
-                    kb_color<1><<<T(kStTile), kBlock, 0, st>>>(J, P(kStTile), nj);
-                else
-                    kb_color<0><<<T(kStTile), kBlock, 0, st>>>(J, P(kStTile), nj);
+                    kb_color<1><<<T(kStTileF), kBlock, 0, st>>>(J, P(kStTileF), nj);
+                else if (T(kStTileF))
+                    kb_color<0><<<T(kStTileF), kBlock, 0, st>>>(J, P(kStTileF), nj);
+                if (T(kStTileW)) kb_color_wave<<<T(kStTileW), kBlock, 0, st>>>(J, P(kStTileW), nj);
             }
             kb_resolve<<<T(kStPix), kBlock, 0, st>>>(J, P(kStPix), nj);
         }
@@ -2645,6 +2764,7 @@ int batch_render(BatchHost &B, hipStream_t st) {
                     DVG_PROF(st, "kb_edge");
                     if (T(kStChunk)) kb_edge<false><<<T(kStChunk), kBlock, 0, st>>>(J, P(kStChunk), nj);
                     if (T(kStChunk2)) kb_edge<true><<<T(kStChunk2), kBlock, 0, st>>>(J, P(kStChunk2), nj);
+                    if (T(kStChunkW)) kb_edge_wave<<<T(kStChunkW), kBlock, 0, st>>>(J, P(kStChunkW), nj);
                 }
             }
             if (B.fold[c]) kb_fold_grads<<<dim3(8, (unsigned)nj), kBlock, 0, st>>>(J);
@@ -3393,7 +3513,8 @@ __global__ __launch_bounds__(kBlock) void k_refit_cdf(RefitArgs A) {
 }
 
 // The segment-only parts of the fast cubic tests, one lane per segment, from the scene's
-// current points: wf::cubic_prep in float4 0-2, wf::stroke_prep in float4 3-7.
+// current points: wf::cubic_prep in float4 0-2, wf::stroke_prep in float4 3-7, and the control
+// points in float4 8-9.
 __global__ __launch_bounds__(kBlock) void k_seg_prep(DevScene S) {
     const int seg = blockIdx.x * blockDim.x + threadIdx.x;
     if (seg >= S.nseg) return;
@@ -3412,6 +3533,8 @@ __global__ __launch_bounds__(kBlock) void k_seg_prep(DevScene S) {
     wf::stroke_prep(a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y, poly, mc, dev);
     for (int i = 0; i < 4; i++) dst[3 + i] = make_float4(poly[4 * i], poly[4 * i + 1], poly[4 * i + 2], poly[4 * i + 3]);
     dst[7] = make_float4(mc, dev, 0.f, 0.f);
+    dst[8] = make_float4(a.x, a.y, b.x, b.y);
+    dst[9] = make_float4(c.x, c.y, d.x, d.y);
 }
 
 int prep_segments(SceneHost &sc, hipStream_t st) {

@@ -51,9 +51,38 @@ DVG_DEV V2 ceval(V2 p0, V2 p1, V2 p2, V2 p3, float t) {
     return (tt * tt * tt) * p0 + (3 * tt * tt * t) * p1 + (3 * tt * t * t) * p2 + (t * t * t) * p3;
 }
 
-// Winding contribution of one segment (winding_number.h:58-167)
-// `prep`: the segment's wf::CubicPrep as three float4 (cubic segments only)
-DVG_DEV int segment_winding(int k, const V2 *p, V2 pt, const float4 *prep) {
+// Winding contribution of a cubic by the reference's double solve (winding_number.h:119-157)
+DVG_DEV int cubic_winding_solve(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
+    int w = 0;
+    double t[3] = {0.0, 0.0, 0.0};
+    double ca = (double)(-p0.y + 3 * p1.y - 3 * p2.y + p3.y), cb = (double)(3 * p0.y - 6 * p1.y + 3 * p2.y),
+           cc = (double)(-3 * p0.y + 3 * p1.y), cd = (double)(p0.y - pt.y);
+    int num_sol = solve_cubic_d(ca, cb, cc, cd, t);
+    // a root at a segment end is counted by the side its last bit falls on: take
+    // that bit from correctly rounded libm functions, as the host libm gives it
+    bool edge = false;
+#pragma unroll
+    for (int j = 0; j < 3; j++) edge |= j < num_sol && (fabs(t[j]) < 1e-9 || fabs(t[j] - 1.0) < 1e-9);
+    if (edge) num_sol = solve_cubic_d_cr(ca, cb, cc, cd, t[0], t[1], t[2]);
+    float ax = -p0.x + 3 * p1.x - 3 * p2.x + p3.x;
+    float bx = 3 * p0.x - 6 * p1.x + 3 * p2.x;
+    float cx = -3 * p0.x + 3 * p1.x;
+    float ay3 = 3 * (-p0.y + 3 * p1.y - 3 * p2.y + p3.y);
+    float by2 = 2 * (3 * p0.y - 6 * p1.y + 3 * p2.y);
+    float cy = -3 * p0.y + 3 * p1.y;
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        double tj = t[j];
+        if (j < num_sol && tj >= 0 && tj <= 1) {
+            double tp = ax * tj * tj * tj + bx * tj * tj + cx * tj + p0.x - pt.x;
+            if (tp > 0) w += (ay3 * tj * tj + by2 * tj + cy > 0) ? 1 : -1;
+        }
+    }
+    return w;
+}
+
+// Winding contribution of a line (k = 0) or quadratic (k = 1) segment (winding_number.h:58-118)
+DVG_DEV int segment_winding_lq(int k, const V2 *p, V2 pt) {
     int w = 0;
     if (k == 0) {
         V2 p0 = p[0], p1 = p[1];
@@ -64,7 +93,7 @@ DVG_DEV int segment_winding(int k, const V2 *p, V2 pt, const float4 *prep) {
                 if (tp >= 0) w += (p1.y - p0.y > 0) ? 1 : -1;
             }
         }
-    } else if (k == 1) {
+    } else {
         V2 p0 = p[0], p1 = p[1], p2 = p[2];
         float t[2];
         if (solve_quadratic_f(p0.y - 2 * p1.y + p2.y, -2 * p0.y + 2 * p1.y, p0.y - pt.y, &t[0], &t[1])) {
@@ -76,39 +105,23 @@ DVG_DEV int segment_winding(int k, const V2 *p, V2 pt, const float4 *prep) {
                 }
             }
         }
-    } else {
-        V2 p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
-        // decided in float whenever every decision of the reference is certain
-        // (dvg_winding_fast.h); otherwise the reference's double solve below
-        int wfast = 0;
-        const float4 q0 = prep[0], q1 = prep[1], q2 = prep[2];
-        const wf::CubicPrep q{q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x};
-        if (wf::cubic_winding_fast_prep(q, p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y, pt.x, pt.y, wfast))
-            return wfast;
-        double t[3];
-        double ca = (double)(-p0.y + 3 * p1.y - 3 * p2.y + p3.y), cb = (double)(3 * p0.y - 6 * p1.y + 3 * p2.y),
-               cc = (double)(-3 * p0.y + 3 * p1.y), cd = (double)(p0.y - pt.y);
-        int num_sol = solve_cubic_d(ca, cb, cc, cd, t);
-        // a root at a segment end is counted by the side its last bit falls on: take
-        // that bit from correctly rounded libm functions, as the host libm gives it
-        bool edge = false;
-        for (int j = 0; j < num_sol; j++) edge |= fabs(t[j]) < 1e-9 || fabs(t[j] - 1.0) < 1e-9;
-        if (edge) num_sol = solve_cubic_d_cr(ca, cb, cc, cd, t);
-        float ax = -p0.x + 3 * p1.x - 3 * p2.x + p3.x;
-        float bx = 3 * p0.x - 6 * p1.x + 3 * p2.x;
-        float cx = -3 * p0.x + 3 * p1.x;
-        float ay3 = 3 * (-p0.y + 3 * p1.y - 3 * p2.y + p3.y);
-        float by2 = 2 * (3 * p0.y - 6 * p1.y + 3 * p2.y);
-        float cy = -3 * p0.y + 3 * p1.y;
-        for (int j = 0; j < num_sol; j++) {
-            double tj = t[j];
-            if (tj >= 0 && tj <= 1) {
-                double tp = ax * tj * tj * tj + bx * tj * tj + cx * tj + p0.x - pt.x;
-                if (tp > 0) w += (ay3 * tj * tj + by2 * tj + cy > 0) ? 1 : -1;
-            }
-        }
     }
     return w;
+}
+
+// Winding contribution of one segment (winding_number.h:58-167)
+// `prep`: the segment's wf::CubicPrep as three float4 (cubic segments only)
+DVG_DEV int segment_winding(int k, const V2 *p, V2 pt, const float4 *prep) {
+    if (k != 2) return segment_winding_lq(k, p, pt);
+    V2 p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
+    // decided in float whenever every decision of the reference is certain
+    // (dvg_winding_fast.h); otherwise the reference's double solve
+    int wfast = 0;
+    const float4 q0 = prep[0], q1 = prep[1], q2 = prep[2];
+    const wf::CubicPrep q{q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x};
+    if (wf::cubic_winding_fast_prep(q, p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y, pt.x, pt.y, wfast))
+        return wfast;
+    return cubic_winding_solve(p0, p1, p2, p3, pt);
 }
 
 DVG_DEV int winding_path(const DevScene &S, int s, V2 pt) {
@@ -125,9 +138,8 @@ DVG_DEV int winding_path(const DevScene &S, int s, V2 pt) {
     return wn;
 }
 
-DVG_DEV int winding_shape(const DevScene &S, int s, V2 pt) {
-    int type = S.shape_type[s];
-    if (type == 2) return winding_path(S, s, pt);
+// of a circle, an ellipse or a rect
+DVG_DEV int winding_prim(const DevScene &S, int s, int type, V2 pt) {
     const float *P = S.params + S.param_off[s];
     if (type == 0) {
         float r = P[0];
@@ -137,6 +149,10 @@ DVG_DEV int winding_shape(const DevScene &S, int s, V2 pt) {
         return (dx * dx) / (P[0] * P[0]) + (dy * dy) / (P[1] * P[1]) < 1 ? 1 : 0;
     }
     return (pt.x > P[0] && pt.x < P[2] && pt.y > P[1] && pt.y < P[3]) ? 1 : 0;
+}
+DVG_DEV int winding_shape(const DevScene &S, int s, V2 pt) {
+    int type = S.shape_type[s];
+    return type == 2 ? winding_path(S, s, pt) : winding_prim(S, s, type, pt);
 }
 
 // is_inside (diffvg.cpp:33-87); `local` is canvas_to_shape(pt)
@@ -208,23 +224,34 @@ DVG_DEV double quintic_deriv(const Quintic &q, double t) {
 }
 // Isolating intervals (within_distance.h:195-216); the reference's uninitialised
 // intervals[0] (isolator root outside [0, 1]) is treated as absent.
-DVG_DEV int quintic_intervals(const Quintic &q, float *iv) {
+// All indices are compile-time constants (slots past n are not read as such), so the array
+// stays in registers.
+DVG_DEV int quintic_intervals(const Quintic &q, float (&iv)[4]) {
     double p1A = ((2 / 5.f) * q.C - (4 / 25.f) * q.B * q.B);
     double p1B = ((3 / 5.f) * q.D - (3 / 25.f) * q.B * q.C);
     double p1C = ((4 / 5.f) * q.E - (2 / 25.f) * q.B * q.D);
     double p1D = q.F - q.B * q.E / 25.f;
     double q_root = -q.B / 5.f;
-    double pr[3];
+    double pr[3] = {0.0, 0.0, 0.0};
     int num_sol = solve_cubic_d(p1A, p1B, p1C, p1D, pr);
-    int n = 0;
-    if (q_root >= 0 && q_root <= 1) iv[n++] = (float)q_root;
-    for (int j = 0; j < num_sol; j++) iv[n++] = (float)pr[j];
-    for (int j = 1; j < n; j++)
-        for (int k = j; k > 0 && iv[k - 1] > iv[k]; k--) {
-            float tmp = iv[k];
-            iv[k] = iv[k - 1];
-            iv[k - 1] = tmp;
+    const bool first = q_root >= 0 && q_root <= 1;
+    const int n = num_sol + (first ? 1 : 0);
+    iv[0] = first ? (float)q_root : (float)pr[0];
+    iv[1] = first ? (float)pr[0] : (float)pr[1];
+    iv[2] = first ? (float)pr[1] : (float)pr[2];
+    iv[3] = (float)pr[2];
+    // insertion sort of the first n
+#pragma unroll
+    for (int j = 1; j < 4; j++) {
+        bool go = j < n;
+#pragma unroll
+        for (int k = j; k > 0; k--) {
+            go = go && iv[k - 1] > iv[k];
+            const float lo = go ? iv[k] : iv[k - 1], hi = go ? iv[k - 1] : iv[k];
+            iv[k - 1] = lo;
+            iv[k] = hi;
         }
+    }
     return n;
 }
 DVG_DEV float quintic_root(const Quintic &q, float lb, float ub) {
@@ -260,14 +287,42 @@ DVG_DEV bool cubic_farther_than(const DevScene &S, int seg, V2 p0, V2 pt, float 
     return wf::cubic_certainly_farther_prep(poly, md.x, md.y, p0.x, p0.y, pt.x, pt.y, r);
 }
 
-// One stroke segment test of within_distance (within_distance.h:32-276).
-// Returns 1 (hit), 0 (miss) or -1 (quadratic distance-approximation miss, which ends
-// the whole path query in the reference).
-DVG_DEV int segment_within(const DevScene &S, int s, int seg, V2 pt, float r) {
-    V2 p[4];
-    int4 idx;
-    int k = seg_load(S, seg, p, idx);
-    bool thick = S.has_thick[s] != 0;
+// Whether one of the stationary points of the distance to a cubic that the quintic search
+// finds lies within the stroke's radius there (within_distance.h:119-272 past its end tests).
+DVG_DEV bool cubic_stroke_search(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2, float r3) {
+    Quintic q = cubic_quintic(p0, p1, p2, p3, pt);
+    float iv[4];
+    int niv = quintic_intervals(q, iv);
+    const float e0 = iv[0], e1 = iv[1], e2 = iv[2], e3 = iv[3];
+    float lower = 0.f;
+#pragma nounroll
+    for (int j = 0; j < niv + 1; j++) {
+        const float end = j < 2 ? (j == 0 ? e0 : e1) : (j == 2 ? e2 : e3);
+        if (j < niv && end < 0.f) continue;
+        float upper = j < niv ? fmin_r(end, 1.f) : 1.f;
+        float lb = lower, ub = upper;
+        double lbe = quintic_eval(q, lb), ube = quintic_eval(q, ub);
+        if (lbe * ube > 0) continue;
+        if (lbe > ube) {
+            float tmp = lb;
+            lb = ub;
+            ub = tmp;
+        }
+        float t = quintic_root(q, lb, ub);
+        float tt = 1 - t;
+        float rr = (tt * tt * tt) * r0 + (3 * tt * tt * t) * r1 + (3 * tt * t * t) * r2 + (t * t * t) * r3;
+        if (dist_sq(ceval(p0, p1, p2, p3, t), pt) < rr * rr) return true;
+        if (upper >= 1.f) break;
+        lower = upper;
+    }
+    return false;
+}
+
+// One line (k = 0) or quadratic (k = 1) stroke segment test of within_distance
+// (within_distance.h:32-118).  Returns 1 (hit), 0 (miss) or -1 (quadratic
+// distance-approximation miss, which ends the whole path query in the reference).
+DVG_DEV int segment_within_lq(const DevScene &S, int s, int k, const V2 *p, int4 idx, V2 pt, float r) {
+    const bool thick = S.has_thick[s] != 0;
     if (k == 0) {
         V2 p0 = p[0], p1 = p[1];
         float t = dot(pt - p0, p1 - p0) / dot(p1 - p0, p1 - p0);
@@ -280,35 +335,44 @@ DVG_DEV int segment_within(const DevScene &S, int s, int seg, V2 pt, float r) {
         if (t > 1) return dist_sq(p1, pt) < r1 * r1;
         float rr = r0 + t * (r1 - r0);
         return dist_sq(p0 + t * (p1 - p0), pt) < rr * rr;
-    } else if (k == 1) {
-        V2 p0 = p[0], p1 = p[1], p2 = p[2];
-        if (S.approx[s]) {
-            V2 cp = quadratic_closest_pt_approx(p0, p1, p2, pt);
-            return dist_sq(cp, pt) < r * r ? 1 : -1;
-        }
-        float r0 = r, r1 = r, r2 = r;
-        if (thick) {
-            r0 = S.thickness[idx.x];
-            r1 = S.thickness[idx.y];
-            r2 = S.thickness[idx.z];
-        }
-        if (dist_sq(qeval(p0, p1, p2, 0), pt) < r0 * r0) return 1;
-        if (dist_sq(qeval(p0, p1, p2, 1), pt) < r2 * r2) return 1;
-        float A = vsum((p0 - 2 * p1 + p2) * (p0 - 2 * p1 + p2));
-        float B = vsum(3 * (p0 - 2 * p1 + p2) * (-p0 + p1));
-        float C = vsum(2 * (-p0 + p1) * (-p0 + p1) + (p0 - 2 * p1 + p2) * (p0 - pt));
-        float D = vsum((-p0 + p1) * (p0 - pt));
-        float t[3];
-        int num_sol = solve_cubic_f(A, B, C, D, t);
-        for (int j = 0; j < num_sol; j++) {
-            if (t[j] >= 0 && t[j] <= 1) {
-                float tt = 1 - t[j];
-                float rr = (tt * tt) * r0 + (2 * tt * t[j]) * r1 + (t[j] * t[j]) * r2;
-                if (dist_sq(qeval(p0, p1, p2, t[j]), pt) < rr * rr) return 1;
-            }
-        }
-        return 0;
     }
+    V2 p0 = p[0], p1 = p[1], p2 = p[2];
+    if (S.approx[s]) {
+        V2 cp = quadratic_closest_pt_approx(p0, p1, p2, pt);
+        return dist_sq(cp, pt) < r * r ? 1 : -1;
+    }
+    float r0 = r, r1 = r, r2 = r;
+    if (thick) {
+        r0 = S.thickness[idx.x];
+        r1 = S.thickness[idx.y];
+        r2 = S.thickness[idx.z];
+    }
+    if (dist_sq(qeval(p0, p1, p2, 0), pt) < r0 * r0) return 1;
+    if (dist_sq(qeval(p0, p1, p2, 1), pt) < r2 * r2) return 1;
+    float A = vsum((p0 - 2 * p1 + p2) * (p0 - 2 * p1 + p2));
+    float B = vsum(3 * (p0 - 2 * p1 + p2) * (-p0 + p1));
+    float C = vsum(2 * (-p0 + p1) * (-p0 + p1) + (p0 - 2 * p1 + p2) * (p0 - pt));
+    float D = vsum((-p0 + p1) * (p0 - pt));
+    float t[3] = {0.f, 0.f, 0.f};
+    int num_sol = solve_cubic_f(A, B, C, D, t);
+#pragma unroll
+    for (int j = 0; j < 3; j++) {
+        if (j < num_sol && t[j] >= 0 && t[j] <= 1) {
+            float tt = 1 - t[j];
+            float rr = (tt * tt) * r0 + (2 * tt * t[j]) * r1 + (t[j] * t[j]) * r2;
+            if (dist_sq(qeval(p0, p1, p2, t[j]), pt) < rr * rr) return 1;
+        }
+    }
+    return 0;
+}
+
+// One stroke segment test of within_distance (within_distance.h:32-276); results as above.
+DVG_DEV int segment_within(const DevScene &S, int s, int seg, V2 pt, float r) {
+    V2 p[4];
+    int4 idx;
+    int k = seg_load(S, seg, p, idx);
+    if (k != 2) return segment_within_lq(S, s, k, p, idx, pt, r);
+    bool thick = S.has_thick[s] != 0;
     V2 p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
     float r0 = r, r1 = r, r2 = r, r3 = r;
     if (thick) {
@@ -336,29 +400,7 @@ DVG_DEV int segment_within(const DevScene &S, int s, int seg, V2 pt, float r) {
                                              fmaxf(fmaxf(fabsf(r0), fabsf(r1)), fmaxf(fabsf(r2), fabsf(r3)))))
             return 0;
     }
-    Quintic q = cubic_quintic(p0, p1, p2, p3, pt);
-    float iv[4];
-    int niv = quintic_intervals(q, iv);
-    float lower = 0.f;
-    for (int j = 0; j < niv + 1; j++) {
-        if (j < niv && iv[j] < 0.f) continue;
-        float upper = j < niv ? fmin_r(iv[j], 1.f) : 1.f;
-        float lb = lower, ub = upper;
-        double lbe = quintic_eval(q, lb), ube = quintic_eval(q, ub);
-        if (lbe * ube > 0) continue;
-        if (lbe > ube) {
-            float tmp = lb;
-            lb = ub;
-            ub = tmp;
-        }
-        float t = quintic_root(q, lb, ub);
-        float tt = 1 - t;
-        float rr = (tt * tt * tt) * r0 + (3 * tt * tt * t) * r1 + (3 * tt * t * t) * r2 + (t * t * t) * r3;
-        if (dist_sq(ceval(p0, p1, p2, p3, t), pt) < rr * rr) return 1;
-        if (upper >= 1.f) break;
-        lower = upper;
-    }
-    return 0;
+    return cubic_stroke_search(p0, p1, p2, p3, pt, r0, r1, r2, r3);
 }
 
 DVG_DEV bool within_distance_path(const DevScene &S, int s, V2 pt, float r) {
@@ -372,9 +414,8 @@ DVG_DEV bool within_distance_path(const DevScene &S, int s, V2 pt, float r) {
     return false;
 }
 
-DVG_DEV bool within_distance_shape(const DevScene &S, int s, V2 pt, float r) {
-    int type = S.shape_type[s];
-    if (type == 2) return within_distance_path(S, s, pt, r);
+// of a circle, an ellipse or a rect
+DVG_DEV bool within_distance_prim(const DevScene &S, int s, int type, V2 pt, float r) {
     const float *P = S.params + S.param_off[s];
     if (type == 0) return fabs((double)(dist(V2{P[1], P[2]}, pt) - P[0])) < r;
     if (type == 1) return false;  // the reference asserts on stroked ellipses
@@ -386,6 +427,10 @@ DVG_DEV bool within_distance_shape(const DevScene &S, int s, V2 pt, float r) {
         return dist_sq(p0 + t * (p1 - p0), pt) < r * r;
     };
     return test(lt, lb) || test(lt, rt) || test(rt, rb) || test(lb, rb);
+}
+DVG_DEV bool within_distance_shape(const DevScene &S, int s, V2 pt, float r) {
+    int type = S.shape_type[s];
+    return type == 2 ? within_distance_path(S, s, pt, r) : within_distance_prim(S, s, type, pt, r);
 }
 
 // within_distance for a group (within_distance.h:355-446)
@@ -488,10 +533,13 @@ DVG_DEV float cubic_closest(const DevScene &S, int seg, V2 pt, V2 &cp, float &t_
     Quintic q = cubic_quintic(p0, p1, p2, p3, pt);
     float iv[4];
     int niv = quintic_intervals(q, iv);
+    const float e0 = iv[0], e1 = iv[1], e2 = iv[2], e3 = iv[3];
     float lower = 0.f;
+#pragma nounroll
     for (int j = 0; j < niv + 1; j++) {
-        if (j < niv && iv[j] < 0.f) continue;
-        float upper = j < niv ? fmin_r(iv[j], 1.f) : 1.f;
+        const float end = j < 2 ? (j == 0 ? e0 : e1) : (j == 2 ? e2 : e3);
+        if (j < niv && end < 0.f) continue;
+        float upper = j < niv ? fmin_r(end, 1.f) : 1.f;
         float lb = lower, ub = upper;
         double lbe = quintic_eval(q, lb), ube = quintic_eval(q, ub);
         if (lbe * ube > 0) continue;

@@ -32,8 +32,16 @@ struct BNode {  // BVHNode (reference scene.h:12-16), padded to 32 bytes
     int pad;
 };
 
-// float4 per segment of DevScene::seg_wf: wf::CubicPrep (3), wf::stroke_prep (5)
-constexpr int kSegPrep = 8;
+// float4 per segment of DevScene::seg_wf: wf::CubicPrep (3), wf::stroke_prep (5), the four
+// control points (2)
+constexpr int kSegPrep = 10;
+
+// What the wave-cooperative coverage tests (dvg_wave.h) take: every group has one shape, no
+// path uses the approximate quadratic distance (its first miss ends the path's query, so its
+// segments cannot be tested in any order), segment numbers fit their queue entries and the
+// winding sums of a path fit 16 bits (a cubic adds at most 3).
+constexpr int kWaveMaxSegs = 1 << 20;
+constexpr int kWaveMaxPathSegs = 10000;
 
 struct DevScene {
     int cw, ch;
@@ -103,6 +111,7 @@ struct DevScene {
     // first is the block itself, a backward's workgroups add to copy (workgroup & rep_mask)
     // and the last kernel of the backward folds the others into the first and clears them.
     int rep_mask, rep_stride;
+    int wave_ok;  // the wave-cooperative coverage tests apply (kWaveMaxSegs)
 };
 
 }  // namespace dvg

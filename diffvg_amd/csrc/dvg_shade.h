@@ -13,6 +13,7 @@
 #pragma once
 
 #include "dvg_query.h"
+#include "dvg_wave.h"
 
 namespace dvg {
 

@@ -63,10 +63,19 @@ DVG_WF void halve(float c0, float c1, float c2, float c3, bool rising, float &lo
 // Over the bracket [lo, hi] of a crossing, each value lies within (derivative bound) x
 // (half width) of its value at the midpoint: returns +1 / -1 when y' keeps the crossing's
 // sign with margin ed and x(t) - pt.x is certainly positive / negative (margin ex), else 0.
+// With hy > 0 the same for every ray height within hy of the point's: the crossing then lies
+// up to hy / min |y'| outside the bracket, so the bracket grows by 2 hy / |y'(m)| and |y'|
+// must stay above half of |y'(m)| over it.
 DVG_WF int crossing_side(float p0x, float p1x, float p2x, float p3x, float d0, float d1, float d2, float ptx,
-                         bool rising, float lo, float hi, float ddmax, float xdmax, float ed, float ex) {
-    const float m = 0.5f * (lo + hi), half = 0.5f * (hi - lo);
+                         bool rising, float lo, float hi, float ddmax, float xdmax, float ed, float ex,
+                         float hy = 0.f) {
+    const float m = 0.5f * (lo + hi);
+    float half = 0.5f * (hi - lo);
     const float yd = 3.f * bern2(d0, d1, d2, m);
+    if (hy > 0.f) {
+        half += 2.02f * hy / fabsf(yd);
+        if (!(fabsf(yd) - 3.f * ddmax * half >= 0.5f * fabsf(yd))) return 0;
+    }
     if ((yd > 0.f) != rising || !(fabsf(yd) - 3.f * ddmax * half > ed)) return 0;
     const float xm = bern3(p0x, p1x, p2x, p3x, m) - ptx, xv = xdmax * half + ex;
     if (xm - xv > 0.f) return 1;
@@ -145,17 +154,19 @@ DVG_WF CubicPrep cubic_prep(float p0x, float p0y, float p1x, float p1y, float p2
 }
 
 // Returns true and sets `w` when the contribution is decided; `q` is the segment's
-// cubic_prep.
+// cubic_prep.  With hx, hy > 0 it decides for every point within hx, hy of (ptx, pty) at
+// once (the two sides of a boundary sample): every margin grows by that much.
 DVG_WF bool cubic_winding_fast_prep(const CubicPrep &q, float p0x, float p0y, float p1x, float p1y, float p2x,
-                                    float p2y, float p3x, float p3y, float ptx, float pty, int &w) {
-    const float M = fmaxf(q.my, fabsf(pty)) + 1.f;
-    const float Mx = fmaxf(q.mx, fabsf(ptx)) + 1.f;
+                                    float p2y, float p3x, float p3y, float ptx, float pty, int &w, float hx = 0.f,
+                                    float hy = 0.f) {
+    const float M = fmaxf(q.my, fabsf(pty) + hy) + 1.f;
+    const float Mx = fmaxf(q.mx, fabsf(ptx) + hx) + 1.f;
     const float E = q.E;
     if (!(E < 1e-3f)) return false;
     // value margins: the reference's coefficients are within ~2e-6 M of the curve's, and
     // its roots within E of the true ones
-    const float ey = 1e-5f * M + 3.f * E * q.ddy;
-    const float ex = 1e-5f * Mx + 3.f * E * q.ddx;
+    const float ey = 1e-5f * M + 3.f * E * q.ddy + hy;
+    const float ex = 1e-5f * Mx + 3.f * E * q.ddx + hx;
     const float c0 = p0y - pty, c1 = p1y - pty, c2 = p2y - pty, c3 = p3y - pty;
     // hull above or below the ray
     if ((c0 > ey && c1 > ey && c2 > ey && c3 > ey) || (c0 < -ey && c1 < -ey && c2 < -ey && c3 < -ey)) {
@@ -168,38 +179,46 @@ DVG_WF bool cubic_winding_fast_prep(const CubicPrep &q, float p0x, float p0y, fl
         return true;
     }
     if (q.br1 != q.br1) return false;  // y nearly constant
-    // breakpoints: 0, critical points of y in (0, 1), 1
-    float br[4];
-    int nb = 0;
-    br[nb++] = 0.f;
-    if (q.br1 > 0.f) br[nb++] = q.br1;
-    if (q.br2 > 0.f) br[nb++] = q.br2;
-    br[nb++] = 1.f;
-    float fv[4];
-    for (int i = 0; i < nb; i++) {
-        fv[i] = i == 0 ? c0 : (i == nb - 1 ? c3 : bern3(c0, c1, c2, c3, br[i]));
-        if (!(fabsf(fv[i]) > ey)) return false;
+    // breakpoints: 0, critical points of y in (0, 1) (br2 only beside br1), 1
+    const bool has1 = q.br1 > 0.f, has2 = q.br2 > 0.f;
+    if (!(fabsf(c0) > ey) || !(fabsf(c3) > ey)) return false;
+    float f1 = c3, f2 = c3;
+    if (has1) {
+        f1 = bern3(c0, c1, c2, c3, q.br1);
+        if (!(fabsf(f1) > ey)) return false;
+    }
+    if (has2) {
+        f2 = bern3(c0, c1, c2, c3, q.br2);
+        if (!(fabsf(f2) > ey)) return false;
     }
     // bounds for the bracket tests
     const float d0 = p1y - p0y, d1 = p2y - p1y, d2 = p3y - p2y;
     const float ddmax = q.ddmax, xdmax = q.xdmax;
     const float ed = 1e-4f * M * 3.f + 1e-6f + 6.f * E * ddmax;  // derivative margin
     int acc = 0;
-    for (int i = 0; i + 1 < nb; i++) {
-        const float fa = fv[i], fb = fv[i + 1];
-        if ((fa > 0.f) == (fb > 0.f)) continue;  // no crossing on this monotone piece
-        // Bisection to a bracket of width (b - a) / 65536 at most, in two unrolled runs:
-        // after the first 4 halvings a crossing far from pt is usually decided already.
-        float lo = br[i], hi = br[i + 1];
-        const bool rising = fb > 0.f;
-        halve<4>(c0, c1, c2, c3, rising, lo, hi);
-        int xs = crossing_side(p0x, p1x, p2x, p3x, d0, d1, d2, ptx, rising, lo, hi, ddmax, xdmax, ed, ex);
-        if (xs == 0) {
-            halve<12>(c0, c1, c2, c3, rising, lo, hi);
-            xs = crossing_side(p0x, p1x, p2x, p3x, d0, d1, d2, ptx, rising, lo, hi, ddmax, xdmax, ed, ex);
+    float from = 0.f, fa = c0;
+#pragma nounroll
+    for (int i = 0; i < 3; i++) {
+        // the piece [from, to] and its end values; past the last breakpoint nothing is left
+        const bool last = i == 0 ? !has1 : (i == 1 ? !has2 : true);
+        const float to = last ? 1.f : (i == 0 ? q.br1 : q.br2), fb = last ? c3 : (i == 0 ? f1 : f2);
+        if ((fa > 0.f) != (fb > 0.f)) {
+            // Bisection to a bracket of width (to - from) / 65536 at most, in two unrolled
+            // runs: after the first 4 halvings a crossing far from pt is usually decided.
+            float lo = from, hi = to;
+            const bool rising = fb > 0.f;
+            halve<4>(c0, c1, c2, c3, rising, lo, hi);
+            int xs = crossing_side(p0x, p1x, p2x, p3x, d0, d1, d2, ptx, rising, lo, hi, ddmax, xdmax, ed, ex, hy);
+            if (xs == 0) {
+                halve<12>(c0, c1, c2, c3, rising, lo, hi);
+                xs = crossing_side(p0x, p1x, p2x, p3x, d0, d1, d2, ptx, rising, lo, hi, ddmax, xdmax, ed, ex, hy);
+            }
+            if (xs == 0) return false;
+            if (xs > 0) acc += rising ? 1 : -1;
         }
-        if (xs == 0) return false;
-        if (xs > 0) acc += rising ? 1 : -1;
+        if (last) break;
+        from = to;
+        fa = fb;
     }
     w = acc;
     return true;

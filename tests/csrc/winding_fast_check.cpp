@@ -98,6 +98,56 @@ void wf_fuzz(int mode, int64_t n, uint64_t seed, int64_t *out, float *bad) {
 }
 }
 
+extern "C" {
+// The test with a widened margin (one decision for all points within hx, hy of the middle):
+// whenever it decides, the oracle must agree at the corners and at random points of that box.
+// near: the middle lies on the curve's normal within a few half widths of it, as boundary
+// samples of other curves do; else anywhere in the control box.  out, bad as wf_fuzz.
+void wf_fuzz_box(int near, int64_t n, uint64_t seed, int64_t *out, float *bad) {
+    std::mt19937_64 g(seed);
+    std::uniform_real_distribution<float> U(0.f, 1.f);
+    std::normal_distribution<float> N(0.f, 1.f);
+    int64_t decided = 0, mism = 0;
+    for (int64_t i = 0; i < n; i++) {
+        const float canvas = 32.f * std::pow(32.f, U(g));
+        const float h = 1.01e-4f * canvas, hx = h * (0.2f + 0.8f * U(g)), hy = h * (0.2f + 0.8f * U(g));
+        const float sp = canvas * (0.005f + 0.1f * U(g));
+        const float cx = canvas * U(g), cy = canvas * U(g);
+        orc::V2 p[4];
+        for (int k = 0; k < 4; k++) p[k] = orc::V2{cx + sp * N(g), cy + sp * N(g)};
+        const float t = U(g), s = 1.f - t;
+        const float bx = s * s * s * p[0].x + 3 * s * s * t * p[1].x + 3 * s * t * t * p[2].x + t * t * t * p[3].x;
+        const float by = s * s * s * p[0].y + 3 * s * s * t * p[1].y + 3 * s * t * t * p[2].y + t * t * t * p[3].y;
+        orc::V2 m{bx + 4.f * hx * N(g), by + 4.f * hy * N(g)};
+        if (!near) m = orc::V2{cx + 1.5f * sp * N(g), cy + 1.5f * sp * N(g)};
+        const dvg::wf::CubicPrep q = dvg::wf::cubic_prep(p[0].x, p[0].y, p[1].x, p[1].y, p[2].x, p[2].y, p[3].x, p[3].y);
+        int w = 0;
+        if (!dvg::wf::cubic_winding_fast_prep(q, p[0].x, p[0].y, p[1].x, p[1].y, p[2].x, p[2].y, p[3].x, p[3].y, m.x,
+                                              m.y, w, hx, hy))
+            continue;
+        decided++;
+        for (int k = 0; k < 8; k++) {
+            const float fx = k < 4 ? (k & 1 ? 1.f : -1.f) : 2.f * U(g) - 1.f;
+            const float fy = k < 4 ? (k & 2 ? 1.f : -1.f) : 2.f * U(g) - 1.f;
+            const orc::V2 pt{m.x + fx * hx, m.y + fy * hy};
+            if (orc::segment_winding(2, p, pt) == w) continue;
+            if (mism == 0) {
+                for (int j = 0; j < 4; j++) {
+                    bad[2 * j] = p[j].x;
+                    bad[2 * j + 1] = p[j].y;
+                }
+                bad[8] = pt.x;
+                bad[9] = pt.y;
+            }
+            mism++;
+        }
+    }
+    out[0] = decided;
+    out[1] = mism;
+    out[2] = n;
+}
+}
+
 #include "../../oracle/oracle.h"
 
 extern "C" {

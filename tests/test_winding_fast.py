@@ -43,3 +43,19 @@ def test_fast_cubic_stroke_rejection_never_disagrees(mode, min_decided):
     L.wf_within_fuzz(mode, 200000, 77 + mode, out, bad)
     assert out[1] == 0, ('mismatch', list(bad))
     assert out[0] / out[2] >= min_decided
+
+
+@pytest.mark.parametrize('near, min_decided', [(0, 0.9), (1, 0.25)])
+def test_fast_cubic_winding_holds_over_a_box(near, min_decided):
+    """With half widths the test decides for every point of a box at once (the two sides of a
+    boundary sample): the oracle agrees at the box's corners and at points inside it."""
+    if not os.path.exists(SO):
+        pytest.skip('tests/csrc not built (make -C tests/csrc)')
+    L = ctypes.CDLL(SO)
+    L.wf_fuzz_box.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_uint64, ctypes.POINTER(ctypes.c_int64),
+                              ctypes.POINTER(ctypes.c_float)]
+    out = (ctypes.c_int64 * 3)()
+    bad = (ctypes.c_float * 10)()
+    L.wf_fuzz_box(near, 300000, 500 + near, out, bad)
+    assert out[1] == 0, ('mismatch', list(bad))
+    assert out[0] / out[2] >= min_decided
