@@ -512,6 +512,7 @@ DVG_DEV void weight_pixel(const DevScene &S, const Geom &G, int pix, float *weig
     weight[pix] = acc;
 }
 __global__ __launch_bounds__(kBlock) void k_weight(DevScene S, Geom G, float *weight) {
+    mark(S);
     weight_pixel(S, G, blockIdx.x * blockDim.x + threadIdx.x, weight);
 }
 
@@ -589,6 +590,7 @@ DVG_DEV void color_tile(CandLds &L, const DevScene &S, const Geom &G, int tile, 
 template <int PRE>
 __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_COLOR_PRE : DVG_WAVES_COLOR) void k_color(DevScene S, Geom G, const float *bg, float4 *colors, int *err,
                                                   uint16_t *frag, int *pkeep) {
+    mark(S);
     __shared__ CandLds L;
     color_tile<PRE>(L, S, G, blockIdx.x, bg, colors, err, frag, pkeep);
 }
@@ -668,6 +670,7 @@ DVG_DEV void resolve_pixel(const DevScene &S, const Geom &G, int pix, int prefil
 }
 __global__ __launch_bounds__(kBlock) void k_resolve(DevScene S, Geom G, int prefilter, const float *weight,
                                                     const float4 *colors, float *out) {
+    mark(S);
     resolve_pixel(S, G, blockIdx.x * blockDim.x + threadIdx.x, prefilter, weight, colors, out);
 }
 
@@ -811,6 +814,7 @@ template <int PRE>
 __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_COLOR_BWD_PRE : DVG_WAVES_COLOR_BWD) void k_color_bwd(DevScene S, Geom G, const float *bg, const float *weight,
                                                       const float *d_img, float *d_bg, float *d_translation,
                                                       int *err, const uint16_t *frag, const int *pkeep) {
+    mark(S);
     __shared__ ColorBwdLds L;
     color_bwd_tile<PRE>(L, S, G, blockIdx.x, bg, weight, d_img, d_bg, d_translation, err, frag, pkeep);
 }
@@ -835,6 +839,7 @@ DVG_DEV void edge_sample_one(const DevScene &S, const Geom &G, int idx, int coun
 }
 __global__ __launch_bounds__(kBlock) void k_edge_sample(DevScene S, Geom G, int count, EdgeSample *edges,
                                                         int *edge_tile, int *edge_rank, int *tile_count) {
+    mark(S);
     edge_sample_one(S, G, blockIdx.x * blockDim.x + threadIdx.x, count, edges, edge_tile, edge_rank, tile_count);
 }
 
@@ -1087,6 +1092,7 @@ template <bool BOTH>
 __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_EDGE) void k_edge(
     DevScene S, Geom G, const EdgeSample *edges, const int *tile_off, const int *tile_count, const int *chunk_off,
     int ntiles, const int *sorted, const float *bg, const float *weight, const float *d_img, float *d_translation) {
+    mark(S);
     __shared__ EdgeLds L;
     edge_chunk<BOTH>(L, S, G, blockIdx.x, edges, tile_off, tile_count, chunk_off, ntiles, sorted, bg, weight, d_img,
                      d_translation);
@@ -1095,6 +1101,7 @@ __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_EDGE
 __global__ __launch_bounds__(kBlock, DVG_WAVES_EDGE_WAVE) void k_edge_wave(
     DevScene S, Geom G, const EdgeSample *edges, const int *tile_off, const int *tile_count, const int *chunk_off,
     int ntiles, const int *sorted, const float *bg, const float *weight, const float *d_img, float *d_translation) {
+    mark(S);
     __shared__ EdgeWaveLds L;
     edge_chunk<true, true>(L.e, S, G, blockIdx.x, edges, tile_off, tile_count, chunk_off, ntiles, sorted, bg, weight,
                            d_img, d_translation, scene_argument(), L.w);
@@ -1308,11 +1315,13 @@ DVG_DEV void sdf_tile(SdfLds &L, const DevScene &S, const Geom &G, int tile, flo
 }
 __global__ __launch_bounds__(kBlock, DVG_WAVES_SDF) void k_sdf_tiled(DevScene S, Geom G, float *sdf, const float *d_sdf,
                                                       float *d_translation) {
+    mark(S);
     __shared__ SdfLds L;
     sdf_tile(L, S, G, blockIdx.x, sdf, d_sdf, d_translation);
 }
 __global__ __launch_bounds__(kBlock) void k_sdf(DevScene S, Geom G, const float *eval_positions, int num_eval,
                                                 float *sdf, const float *d_sdf, float *d_translation) {
+    mark(S);
     sdf_sample(S, G, blockIdx.x * blockDim.x + threadIdx.x, eval_positions, num_eval, sdf, d_sdf, d_translation);
 }
 
@@ -2080,6 +2089,20 @@ struct Job {
 // colour forward of the others / of those
 enum { kStPix = 0, kStTile, kStSamp, kStChunk, kStSdf, kStZero, kStChunk2, kStChunkW, kStTileF, kStTileW, kNumStages };
 
+// What the kernels read through a job is constant while they run, except the buffers that
+// one stage hands to the next (written and read by different launches of one stream, so
+// constant within each) and the images and gradients, marked global.
+DVG_DEV void mark(Job &J) {
+    mark(J.S);
+    mark_constant(J.bg), mark_constant(J.d_img), mark_constant(J.d_sdf), mark_constant(J.eval);
+    mark_global(J.img), mark_global(J.d_bg), mark_global(J.d_tr), mark_global(J.sdf);
+    mark_global(J.weight), mark_global(J.colors), mark_global(J.edges);
+    mark_global(J.edge_tile), mark_global(J.edge_sorted), mark_global(J.edge_rank);
+    mark_global(J.tile_count), mark_global(J.tile_off), mark_global(J.chunk_off);
+    mark_global(J.err), mark_global(J.grad), mark_global(J.frag), mark_global(J.pkeep);
+}
+DVG_DEV Job load_job(const Job *job) { return load_constant<Job>((uint64_t)job); }
+
 // prefix arrays: pref[stage * (nj + 1) + k] = first workgroup of job k in that stage
 DVG_DEV int find_job(const int *pref, int nj, int blk) {
     int lo = 0, hi = nj - 1;
@@ -2095,7 +2118,7 @@ DVG_DEV int find_job(const int *pref, int nj, int blk) {
 
 __global__ __launch_bounds__(kBlock) void kb_zero(const Job *jobs, const int *pref, int nj, int zero_grads) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     int b = blockIdx.x - pref[j], nb = pref[j + 1] - pref[j];
     if (J.d_img && J.tile_count)
         for (int i = b * kBlock + threadIdx.x; i < J.ntiles; i += nb * kBlock) J.tile_count[i] = 0;
@@ -2105,7 +2128,7 @@ __global__ __launch_bounds__(kBlock) void kb_zero(const Job *jobs, const int *pr
 
 // one row of workgroups per job; a workgroup strides over the job's gradient block
 __global__ __launch_bounds__(kBlock) void kb_fold_grads(const Job *jobs) {
-    const Job &J = jobs[blockIdx.y];
+    const Job J = load_job(jobs + blockIdx.y);
     if (!(J.d_img || J.d_sdf) || !J.S.rep_mask) return;
     __shared__ float part[4][64];
     for (int base = blockIdx.x * 64; base < J.S.rep_stride; base += gridDim.x * 64)
@@ -2114,14 +2137,14 @@ __global__ __launch_bounds__(kBlock) void kb_fold_grads(const Job *jobs) {
 
 __global__ __launch_bounds__(kBlock) void kb_weight(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     weight_pixel(J.S, J.G, (blockIdx.x - pref[j]) * kBlock + threadIdx.x, J.weight);
 }
 
 template <int PRE>
 __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_BATCH_COLOR_PRE : DVG_WAVES_BATCH_COLOR) void kb_color(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     if (!J.img) return;
     __shared__ CandLds L;
     color_tile<PRE>(L, J.S, J.G, blockIdx.x - pref[j], J.bg, J.colors, J.err, PRE ? nullptr : J.frag,
@@ -2130,15 +2153,15 @@ __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_BATCH_COLOR_PRE : DVG_WAVES
 
 __global__ __launch_bounds__(kBlock, DVG_WAVES_COLOR_WAVE) void kb_color_wave(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     if (!J.img) return;
     __shared__ ColorWaveLds L;
-    color_tile_wave(L, SceneRef{(uint64_t)&J.S}, J.G, blockIdx.x - pref[j], J.bg, J.colors, J.err, J.frag);
+    color_tile_wave(L, SceneRef{(uint64_t)&jobs[j].S}, J.G, blockIdx.x - pref[j], J.bg, J.colors, J.err, J.frag);
 }
 
 __global__ __launch_bounds__(kBlock) void kb_resolve(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     if (!J.img) return;
     resolve_pixel(J.S, J.G, (blockIdx.x - pref[j]) * kBlock + threadIdx.x, J.pre, J.weight, J.colors, J.img);
 }
@@ -2146,7 +2169,7 @@ __global__ __launch_bounds__(kBlock) void kb_resolve(const Job *jobs, const int 
 template <int PRE>
 __global__ __launch_bounds__(kBlock, DVG_WAVES_BATCH_COLOR_BWD) void kb_color_bwd(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     if (!J.d_img) return;
     __shared__ ColorBwdLds L;
     color_bwd_tile<PRE>(L, J.S, J.G, blockIdx.x - pref[j], J.bg, J.weight, J.d_img, J.d_bg, J.d_tr, J.err,
@@ -2155,14 +2178,14 @@ __global__ __launch_bounds__(kBlock, DVG_WAVES_BATCH_COLOR_BWD) void kb_color_bw
 
 __global__ __launch_bounds__(kBlock) void kb_edge_sample(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     if (!J.d_img) return;
     edge_sample_one(J.S, J.G, (blockIdx.x - pref[j]) * kBlock + threadIdx.x, J.nsamp, J.edges, J.edge_tile,
                     J.edge_rank, J.tile_count);
 }
 
 __global__ __launch_bounds__(1024) void kb_scan(const Job *jobs, int j0) {
-    const Job &J = jobs[j0 + blockIdx.x];
+    const Job J = load_job(jobs + j0 + blockIdx.x);
     if (!J.d_img) return;
     __shared__ ScanLds<1024> L;
     scan_tiles<1024>(L, J.tile_count, J.tile_off, J.chunk_off, J.ntiles, J.G.echunk);
@@ -2170,7 +2193,7 @@ __global__ __launch_bounds__(1024) void kb_scan(const Job *jobs, int j0) {
 
 __global__ __launch_bounds__(kBlock) void kb_edge_bin(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     if (!J.d_img) return;
     edge_bin_one((blockIdx.x - pref[j]) * kBlock + threadIdx.x, J.nsamp, J.edge_tile, J.edge_rank, J.tile_off,
                  J.edge_sorted);
@@ -2182,7 +2205,7 @@ template <bool BOTH>
 __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_BATCH_EDGE) void kb_edge(
     const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     if (!J.d_img) return;
     __shared__ EdgeLds L;
     edge_chunk<BOTH>(L, J.S, J.G, blockIdx.x - pref[j], J.edges, J.tile_off, J.tile_count, J.chunk_off, J.ntiles,
@@ -2191,17 +2214,17 @@ __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_BATC
 
 __global__ __launch_bounds__(kBlock, DVG_WAVES_EDGE_WAVE) void kb_edge_wave(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     if (!J.d_img) return;
     __shared__ EdgeWaveLds L;
     edge_chunk<true, true>(L.e, J.S, J.G, blockIdx.x - pref[j], J.edges, J.tile_off, J.tile_count, J.chunk_off,
-                           J.ntiles, J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr, SceneRef{(uint64_t)&J.S}, L.w);
+                           J.ntiles, J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr, SceneRef{(uint64_t)&jobs[j].S}, L.w);
 }
 
 __global__ __launch_bounds__(kBlock, DVG_WAVES_SDF) void kb_sdf(const Job *jobs, const int *pref, int nj) {
     __shared__ SdfLds L;
     int j = find_job(pref, nj, blockIdx.x);
-    const Job &J = jobs[j];
+    const Job J = load_job(jobs + j);
     if (J.eval)
         sdf_sample(J.S, J.G, (blockIdx.x - pref[j]) * kBlock + threadIdx.x, J.eval, J.num_eval, J.sdf, J.d_sdf,
                    J.d_tr);

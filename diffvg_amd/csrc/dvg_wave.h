@@ -27,6 +27,7 @@
 // Scenes that qualify: DevScene::wave_ok.
 #pragma once
 
+#include "dvg_memory.h"
 #include "dvg_query.h"
 
 namespace dvg {
@@ -55,10 +56,7 @@ struct SceneRef {
     DVG_DEV DevScene get() const {
         uint64_t p = at;
         asm volatile("" : "+s"(p));
-        typedef const __attribute__((address_space(4))) DevScene *Const;
-        DevScene S;
-        __builtin_memcpy(&S, (const void *)(Const)p, sizeof(S));
-        return S;
+        return load_constant<DevScene>(p);
     }
 };
 // of a kernel whose first argument is the DevScene
