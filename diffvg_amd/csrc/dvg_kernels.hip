@@ -87,10 +87,10 @@ constexpr int64_t kPrimDirect = 12288;
 #endif
 // the kernels with the wave-cooperative coverage tests
 #ifndef DVG_WAVES_COLOR_WAVE
-#define DVG_WAVES_COLOR_WAVE 5
+#define DVG_WAVES_COLOR_WAVE 6
 #endif
 #ifndef DVG_WAVES_EDGE_WAVE
-#define DVG_WAVES_EDGE_WAVE 4
+#define DVG_WAVES_EDGE_WAVE 5
 #endif
 // the edge kernel with both sides of a sample per lane keeps two compositors live
 #ifndef DVG_WAVES_EDGE_BOTH
@@ -126,7 +126,7 @@ struct Geom {
     int tw, th, tiles_x, tiles_y;
     float sx_scale, sy_scale;  // canvas / render
     float margin;
-    int echunk;  // boundary samples per edge workgroup: kEdgeChunk or kBlock
+    int echunk;  // boundary samples per edge workgroup: 64 (wave-cooperative), kEdgeChunk or kBlock
     int prim_direct;  // primitives' boundary adjoints are added sample by sample (kPrimDirect)
 };
 
@@ -146,14 +146,6 @@ struct ColorBwdLds {
 struct EdgeLds {
     CandLds c;
     int perm[kBlock];
-};
-struct ColorWaveLds {
-    CandLds c;
-    WaveLds<1> w[kBlock / 64];
-};
-struct EdgeWaveLds {
-    EdgeLds e;
-    WaveLds<2> w[kBlock / 64];
 };
 struct SdfLds {
     CandLds c;
@@ -595,49 +587,60 @@ __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_COLOR_PRE : DVG_WAVES_COLOR
     color_tile<PRE>(L, S, G, blockIdx.x, bg, colors, err, frag, pkeep);
 }
 
+// Samples of a tile in quarters of it, so that the 64 samples of a wave lie in a smaller box:
+// tile_sample with the pixel order changed (where both sides of the tile are even).
+DVG_DEV bool tile_sample_quarters(const Geom &G, int tx, int ty, int si, int &x, int &y, int &sx, int &sy, int &idx) {
+    if ((G.tw | G.th) & 1) return tile_sample(G, tx, ty, si, x, y, sx, sy, idx);
+    const int tile_px = G.tw * G.th;
+    if (si >= tile_px * G.spp) return false;
+    const int p = si / G.spp, sub = si - p * G.spp;
+    const int qw = G.tw >> 1, qh = G.th >> 1, q = p / (qw * qh), i = p - q * (qw * qh);
+    x = tx * G.tw + (q & 1) * qw + i % qw;
+    y = ty * G.th + (q >> 1) * qh + i / qw;
+    if (x >= G.W || y >= G.H) return false;
+    sx = sub % G.nsx;
+    sy = sub / G.nsx;
+    idx = ((y * G.W + x) * G.nsy + sy) * G.nsx + sx;
+    return true;
+}
+
 // color_tile<0> with the wave-cooperative coverage tests (DevScene::wave_ok): the same
-// fragments in the same order.
-DVG_DEV void color_tile_wave(ColorWaveLds &L, const SceneRef &R, const Geom &G, int tile, const float *bg,
+// fragments in the same order.  One wave per workgroup: wave `part` of the tile.
+constexpr int kTileWaves = kBlock / 64;
+DVG_DEV void color_tile_wave(WaveLds<1> &L, const SceneRef &R, const Geom &G, int tile, int part, const float *bg,
                              float4 *colors, int *err, uint16_t *frag) {
-    const DevScene S = R.get();
-    if (frag && tile == 0 && threadIdx.x == 0) key_of(G, err + 2, err + 4);
+    if (frag && tile == 0 && part == 0 && threadIdx.x == 0) key_of(G, err + 2, err + 4);
     const int tx = tile % G.tiles_x, ty = tile / G.tiles_x;
     int x, y, sx, sy, idx;
-    const bool valid = tile_sample(G, tx, ty, threadIdx.x, x, y, sx, sy, idx);
+    const bool valid = tile_sample_quarters(G, tx, ty, 64 * part + threadIdx.x, x, y, sx, sy, idx);
+    if (!__any(valid)) return;
     V2 pt{0, 0};
-    if (valid) pt = to_canvas(S, G, sample_pos(G, x, y, sx, sy, idx, false));
+    if (valid) pt = to_canvas(R.get(), G, sample_pos(G, x, y, sx, sy, idx, false));
     const bool has_bg = bg != nullptr;
     const V4 bgc = (valid && has_bg) ? load_bg(bg, y * G.W + x) : V4{0, 0, 0, 0};
     Compositor comp;
     comp.init(has_bg, bgc);
-    const float4 tb = tile_box(S, G, tx, ty, 0.f);
     const size_t nsamp = (size_t)G.W * G.H * G.spp;
-    for (int c0 = 0; c0 < S.ng; c0 += kCandCap) {
-        const int n = __builtin_amdgcn_readfirstlane(
-            build_candidates(S, tb, c0, min(S.ng, c0 + kCandCap), L.c.list, L.c.w));
-        wave_shade<1>(R, L.w[threadIdx.x >> 6], L.c.list, n, valid, pt, pt, pt, 0.f, 0.f,
-                      [&](const DevScene &S, int g, bool stroke, bool on, bool) {
-                          const int type = stroke ? S.stroke_type[g] : S.fill_type[g];
-                          const int off = stroke ? S.stroke_off[g] : S.fill_off[g];
-                          const int ns = stroke ? S.stroke_ns[g] : S.fill_ns[g];
-                          if (on) {
-                              if (frag && comp.nf < kFragSlots)
-                                  frag[(size_t)comp.nf * nsamp + idx] = (uint16_t)(2 * g + (stroke ? 1 : 0));
-                              comp.add(sample_paint(S, type, off, ns, pt), g, -1);
-                          }
-                      });
-        if (c0 + kCandCap < S.ng) __syncthreads();
-    }
+    wave_shade<1>(R, L, valid, pt, pt, pt, 0.f, 0.f, [&](const DevScene &S, int g, bool stroke, bool on, bool) {
+        const int type = stroke ? S.stroke_type[g] : S.fill_type[g];
+        const int off = stroke ? S.stroke_off[g] : S.fill_off[g];
+        const int ns = stroke ? S.stroke_ns[g] : S.fill_ns[g];
+        if (on) {
+            if (frag && comp.nf < kFragSlots)
+                frag[(size_t)comp.nf * nsamp + idx] = (uint16_t)(2 * g + (stroke ? 1 : 0));
+            comp.add(sample_paint(S, type, off, ns, pt), g, -1);
+        }
+    });
     if (valid) {
         const V4 c = comp.result(has_bg, bgc);
         colors[idx] = make_float4(c.x, c.y, c.z, c.w);
         if (frag) frag[(size_t)kFragSlots * nsamp + idx] = (uint16_t)min(comp.nf, 65535);
     }
 }
-__global__ __launch_bounds__(kBlock, DVG_WAVES_COLOR_WAVE) void k_color_wave(DevScene S, Geom G, const float *bg,
-                                                                            float4 *colors, int *err, uint16_t *frag) {
-    __shared__ ColorWaveLds L;
-    color_tile_wave(L, scene_argument(), G, blockIdx.x, bg, colors, err, frag);
+__global__ __launch_bounds__(64, DVG_WAVES_COLOR_WAVE) void k_color_wave(DevScene S, Geom G, const float *bg,
+                                                                        float4 *colors, int *err, uint16_t *frag) {
+    __shared__ WaveLds<1> L;
+    color_tile_wave(L, scene_argument(), G, blockIdx.x / kTileWaves, blockIdx.x % kTileWaves, bg, colors, err, frag);
 }
 
 DVG_DEV void resolve_pixel(const DevScene &S, const Geom &G, int pix, int prefilter, const float *weight,
@@ -897,26 +900,45 @@ __global__ __launch_bounds__(kBlock) void k_edge_bin(int count, const int *edge_
     edge_bin_one(blockIdx.x * blockDim.x + threadIdx.x, count, edge_tile, edge_rank, tile_off, sorted);
 }
 
-// One workgroup per chunk of up to G.echunk boundary samples of one tile (the grid is an
-// upper bound on the chunk count; workgroups past the total exit at once), so a tile on a
-// busy boundary is spread over many workgroups instead of looping inside one.  BOTH
-// selects how lanes share the two colour queries of a sample (render_edge_kernel,
-// diffvg.cpp:1388-1475, evaluates the inside and the outside point): false -- lanes 2i and
-// 2i + 1 shade the inside and the outside point of sample i (kEdgeChunk samples, less
-// state per lane); true -- one lane shades both points of its sample (kBlock samples).
-// WAVE (with BOTH): the wave-cooperative coverage tests (dvg_wave.h, `W`), which test both
-// points of a sample at once where one decision holds for both.
-template <bool BOTH, bool WAVE = false>
-DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk, const EdgeSample *edges,
-                        const int *tile_off, const int *tile_count, const int *chunk_off, int ntiles,
-                        const int *sorted, const float *bg, const float *weight, const float *d_img,
-                        float *d_translation, SceneRef R = {}, WaveLds<2> *W = nullptr) {
-    constexpr int kChunk = BOTH ? kBlock : kEdgeChunk;
-    int *s_list = L.c.list;
-    int *s_w = L.c.w;
-    int *s_perm = L.perm;
-    if (chunk >= chunk_off[ntiles]) return;
-    // tile = the last t with chunk_off[t] <= chunk (chunk_off is non-decreasing)
+// Adjoint of a wave's boundary samples (render_edge_kernel, diffvg.cpp:1430-1475) from the
+// colours and edge hits of their two sides; every lane calls it, lanes without a sample pass
+// on = false.
+DVG_DEV void edge_scatter(const DevScene &S, const Geom &G, bool on, const EdgeSample &es, bool in_hit, bool out_hit,
+                          V4 cin, V4 cout, const float *weight, const float *d_img, float *d_translation) {
+    V2 n{es.nx, es.ny};
+    int bx = (int)(es.px * G.W), by = (int)(es.py * G.H);
+    // every lane stays to the end: the gradient scatter combines lanes of a wave
+    bool active = on && (in_hit || out_hit);
+    float contrib = 0.f;
+    if (active) {
+        if (!in_hit) {
+            n = -n;
+            V4 tmp = cin;
+            cin = cout;
+            cout = tmp;
+        }
+        V2 sb{es.px * G.W, es.py * G.H};
+        V4 d_color = gather_d_color(S.filter_type, S.filter_radius, d_img, weight, G.W, G.H, sb);
+        d_color = vdiv(d_color, (float)(S.cw * S.ch));
+        contrib = dot(cin - cout, d_color) / es.pdf;
+    }
+    BoundaryData bd = active ? es.data : BoundaryData{0, 0, 0.f, 0};
+    accumulate_boundary_gradient_wave(S, active, active ? es.group : 0, active ? es.shape : 0, contrib,
+                                      active ? es.t : 0.f, n, bd, active ? V2{es.lx, es.ly} : V2{0, 0}, G.prim_direct != 0);
+    if (active && d_translation) {
+        aadd(d_translation + 2 * (by * G.W + bx) + 0, n.x * contrib);
+        aadd(d_translation + 2 * (by * G.W + bx) + 1, n.y * contrib);
+    }
+}
+
+// edge_chunk with the wave-cooperative coverage tests (dvg_wave.h), which test both points of
+// a sample at once where one decision holds for both: one wave, G.echunk = 64 samples of one
+// tile.  A chunk of 256 left a third of the lanes without a sample (a tile of the 300-path
+// scene holds 256 on average, so its second chunk is mostly empty).  A group of one shape
+// whose shape is hit also adds a fragment, so the hits that the coverage tests raise
+// themselves (EdgeQuery), which matter for groups of several shapes, are not needed.
+DVG_DEV int find_tile(const int *chunk_off, int ntiles, int chunk) {
+    // the last t with chunk_off[t] <= chunk (chunk_off is non-decreasing)
     int lo = 0, hi = ntiles - 1;
     while (lo < hi) {
         int mid = (lo + hi + 1) >> 1;
@@ -925,7 +947,80 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
         else
             hi = mid - 1;
     }
-    const int tile = lo;
+    return lo;
+}
+DVG_DEV void edge_chunk_wave(WaveLds<2> &L, const SceneRef &R, const Geom &G, int chunk, const EdgeSample *edges,
+                             const int *tile_off, const int *tile_count, const int *chunk_off, int ntiles,
+                             const int *sorted, const float *bg, const float *weight, const float *d_img,
+                             float *d_translation) {
+    if (chunk >= chunk_off[ntiles]) return;
+    const int lane = threadIdx.x;
+    const int tile = find_tile(chunk_off, ntiles, chunk);
+    const int b0 = (chunk - chunk_off[tile]) * 64, cnt = min(64, tile_count[tile] - b0);
+    const bool valid = lane < cnt;
+    const int eidx = valid ? sorted[tile_off[tile] + b0 + lane] : 0;
+    const bool has_bg = bg != nullptr;
+    V2 pin{0, 0}, pout{0, 0}, pmid{0, 0};
+    int tgroup = -1;
+    Compositor ci, co;
+    float cw, ch;
+    {
+        const DevScene S = R.get();
+        cw = (float)S.cw;
+        ch = (float)S.ch;
+        EdgeSample es{};
+        if (valid) es = edges[eidx];
+        const V2 bp{es.px, es.py}, n0{es.nx, es.ny};
+        const V2 qi = bp - 1e-4f * n0, qo = bp + 1e-4f * n0;
+        pin = V2{qi.x * S.cw, qi.y * S.ch};
+        pout = V2{qo.x * S.cw, qo.y * S.ch};
+        pmid = V2{bp.x * S.cw, bp.y * S.ch};
+        if (valid) tgroup = es.group;
+        const int bx = (int)(es.px * G.W), by = (int)(es.py * G.H);
+        const V4 bg0 = (valid && has_bg) ? load_bg(bg, by * G.W + bx) : V4{0, 0, 0, 0};
+        ci.init(has_bg, bg0);
+        co.init(has_bg, bg0);
+    }
+    wave_shade<2>(R, L, valid, pin, pout, pmid, 1.01e-4f * cw, 1.01e-4f * ch,
+                  [&](const DevScene &S, int g, bool stroke, bool on_in, bool on_out) {
+                      const int type = stroke ? S.stroke_type[g] : S.fill_type[g];
+                      const int off = stroke ? S.stroke_off[g] : S.fill_off[g];
+                      const int ns = stroke ? S.stroke_ns[g] : S.fill_ns[g];
+                      if (on_in) ci.add(sample_paint(S, type, off, ns, pin), g, tgroup);
+                      if (on_out) co.add(sample_paint(S, type, off, ns, pout), g, tgroup);
+                  });
+    const DevScene S = R.get();
+    EdgeSample es{};
+    if (valid) es = edges[eidx];
+    const int bx = (int)(es.px * G.W), by = (int)(es.py * G.H);
+    const V4 bgc = (valid && has_bg) ? load_bg(bg, by * G.W + bx) : V4{0, 0, 0, 0};
+    V4 cin{0, 0, 0, 0}, cout{0, 0, 0, 0};
+    if (valid) {
+        cin = ci.result(has_bg, bgc);
+        cout = co.result(has_bg, bgc);
+    }
+    edge_scatter(S, G, valid, es, valid && ci.edge_hit(false), valid && co.edge_hit(false), cin, cout, weight, d_img,
+                 d_translation);
+}
+
+// One workgroup per chunk of up to G.echunk boundary samples of one tile (the grid is an
+// upper bound on the chunk count; workgroups past the total exit at once), so a tile on a
+// busy boundary is spread over many workgroups instead of looping inside one.  BOTH
+// selects how lanes share the two colour queries of a sample (render_edge_kernel,
+// diffvg.cpp:1388-1475, evaluates the inside and the outside point): false -- lanes 2i and
+// 2i + 1 shade the inside and the outside point of sample i (kEdgeChunk samples, less
+// state per lane); true -- one lane shades both points of its sample (kBlock samples).
+template <bool BOTH>
+DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk, const EdgeSample *edges,
+                        const int *tile_off, const int *tile_count, const int *chunk_off, int ntiles,
+                        const int *sorted, const float *bg, const float *weight, const float *d_img,
+                        float *d_translation) {
+    constexpr int kChunk = BOTH ? kBlock : kEdgeChunk;
+    int *s_list = L.c.list;
+    int *s_w = L.c.w;
+    int *s_perm = L.perm;
+    if (chunk >= chunk_off[ntiles]) return;
+    const int tile = find_tile(chunk_off, ntiles, chunk);
     const int cnt = tile_count[tile];
     int tx = tile % G.tiles_x, ty = tile / G.tiles_x;
     float ext = 1e-4f * (float)max(S.cw, S.ch) * 1.01f;
@@ -1002,7 +1097,7 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
             cin = mine;
             cout = other;
         } else {
-            V2 pin{0, 0}, pout{0, 0}, pmid{0, 0};
+            V2 pin{0, 0}, pout{0, 0};
             Compositor ci, co;
             {
                 EdgeSample es0{};
@@ -1011,7 +1106,6 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
                 V2 qi = bp - 1e-4f * n0, qo = bp + 1e-4f * n0;
                 pin = V2{qi.x * S.cw, qi.y * S.ch};
                 pout = V2{qo.x * S.cw, qo.y * S.ch};
-                pmid = V2{bp.x * S.cw, bp.y * S.ch};
                 if (valid) {
                     tgroup = es0.group;
                     tshape = es0.shape;
@@ -1021,35 +1115,16 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
                 ci.init(has_bg, bg0);
                 co.init(has_bg, bg0);
             }
-            // a group of one shape whose shape is hit also adds a fragment, so the hits that
-            // the coverage tests raise themselves only matter for groups of several shapes
+            EdgeQuery qin{tgroup, tshape, false};
+            EdgeQuery qout = qin;
             bool hin = false, hout = false;
-            if constexpr (WAVE) {
-                for (int c0 = 0; c0 < S.ng; c0 += kCandCap) {
-                    const int nc = __builtin_amdgcn_readfirstlane(
-                        build_candidates(S, tb, c0, min(S.ng, c0 + kCandCap), s_list, s_w));
-                    wave_shade<2>(R, W[threadIdx.x >> 6], s_list, nc, valid, pin, pout, pmid, 1.01e-4f * S.cw,
-                                  1.01e-4f * S.ch, [&](const DevScene &S, int g, bool stroke, bool on_in,
-                                                     bool on_out) {
-                                      const int type = stroke ? S.stroke_type[g] : S.fill_type[g];
-                                      const int off = stroke ? S.stroke_off[g] : S.fill_off[g];
-                                      const int ns = stroke ? S.stroke_ns[g] : S.fill_ns[g];
-                                      if (on_in) ci.add(sample_paint(S, type, off, ns, pin), g, tgroup);
-                                      if (on_out) co.add(sample_paint(S, type, off, ns, pout), g, tgroup);
-                                  });
-                    if (c0 + kCandCap < S.ng) __syncthreads();
+            for (int c0 = 0; c0 < S.ng; c0 += kCandCap) {
+                int nc = build_candidates(S, tb, c0, min(S.ng, c0 + kCandCap), s_list, s_w);
+                if (valid) {
+                    shade_list(S, pin, s_list, nc, ci, &qin, hin);
+                    shade_list(S, pout, s_list, nc, co, &qout, hout);
                 }
-            } else {
-                EdgeQuery qin{tgroup, tshape, false};
-                EdgeQuery qout = qin;
-                for (int c0 = 0; c0 < S.ng; c0 += kCandCap) {
-                    int nc = build_candidates(S, tb, c0, min(S.ng, c0 + kCandCap), s_list, s_w);
-                    if (valid) {
-                        shade_list(S, pin, s_list, nc, ci, &qin, hin);
-                        shade_list(S, pout, s_list, nc, co, &qout, hout);
-                    }
-                    if (c0 + kCandCap < S.ng) __syncthreads();
-                }
+                if (c0 + kCandCap < S.ng) __syncthreads();
             }
             asm volatile("" ::: "memory");  // read the sample again, do not keep it live
             if (valid) es = edges[eidx];
@@ -1062,30 +1137,7 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
                 cout = co.result(has_bg, bgc);
             }
         }
-        V2 n{es.nx, es.ny};
-        int bx = (int)(es.px * G.W), by = (int)(es.py * G.H);
-        // every lane stays to the end: the gradient scatter combines lanes of a wave
-        bool active = valid && side == 0 && (in_hit || out_hit);
-        float contrib = 0.f;
-        if (active) {
-            if (!in_hit) {
-                n = -n;
-                V4 tmp = cin;
-                cin = cout;
-                cout = tmp;
-            }
-            V2 sb{es.px * G.W, es.py * G.H};
-            V4 d_color = gather_d_color(S.filter_type, S.filter_radius, d_img, weight, G.W, G.H, sb);
-            d_color = vdiv(d_color, (float)(S.cw * S.ch));
-            contrib = dot(cin - cout, d_color) / es.pdf;
-        }
-        BoundaryData bd = active ? es.data : BoundaryData{0, 0, 0.f, 0};
-        accumulate_boundary_gradient_wave(S, active, active ? es.group : 0, active ? es.shape : 0, contrib,
-                                          active ? es.t : 0.f, n, bd, active ? V2{es.lx, es.ly} : V2{0, 0}, G.prim_direct != 0);
-        if (active && d_translation) {
-            aadd(d_translation + 2 * (by * G.W + bx) + 0, n.x * contrib);
-            aadd(d_translation + 2 * (by * G.W + bx) + 1, n.y * contrib);
-        }
+        edge_scatter(S, G, valid && side == 0, es, in_hit, out_hit, cin, cout, weight, d_img, d_translation);
     }
 }
 template <bool BOTH>
@@ -1098,13 +1150,12 @@ __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_EDGE
                      d_translation);
 }
 
-__global__ __launch_bounds__(kBlock, DVG_WAVES_EDGE_WAVE) void k_edge_wave(
+__global__ __launch_bounds__(64, DVG_WAVES_EDGE_WAVE) void k_edge_wave(
     DevScene S, Geom G, const EdgeSample *edges, const int *tile_off, const int *tile_count, const int *chunk_off,
     int ntiles, const int *sorted, const float *bg, const float *weight, const float *d_img, float *d_translation) {
-    mark(S);
-    __shared__ EdgeWaveLds L;
-    edge_chunk<true, true>(L.e, S, G, blockIdx.x, edges, tile_off, tile_count, chunk_off, ntiles, sorted, bg, weight,
-                           d_img, d_translation, scene_argument(), L.w);
+    __shared__ WaveLds<2> L;
+    edge_chunk_wave(L, scene_argument(), G, blockIdx.x, edges, tile_off, tile_count, chunk_off, ntiles, sorted, bg,
+                    weight, d_img, d_translation);
 }
 
 // Adds the gradient copies 1..rep_mask to the block and clears them (DevScene::rep_mask).
@@ -1657,7 +1708,7 @@ static Geom make_geom(const SceneHost &sc, const dvg_render_args &a) {
     if (th < 1) th = 1;
     G.tw = tw;
     G.th = th;
-    G.echunk = sc.dev.wave_ok || sc.edge_spw == 64 ? kBlock : kEdgeChunk;
+    G.echunk = sc.dev.wave_ok ? 64 : (sc.edge_spw == 64 ? kBlock : kEdgeChunk);
     G.prim_direct = (int64_t)G.W * G.H * G.spp > kPrimDirect * sc.num_shapes;
     G.tiles_x = (G.W + tw - 1) / tw;
     G.tiles_y = (G.H + th - 1) / th;
@@ -1798,7 +1849,7 @@ int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
                 if (pre)
                     k_color<1><<<ntiles, kBlock, 0, st>>>(S, G, a.background_image, ws.colors, sc.err, nullptr, pkeep);
                 else if (S.wave_ok)
-                    k_color_wave<<<ntiles, kBlock, 0, st>>>(S, G, a.background_image, ws.colors, sc.err, frag);
+                    k_color_wave<<<kTileWaves * ntiles, 64, 0, st>>>(S, G, a.background_image, ws.colors, sc.err, frag);
                 else
                     k_color<0><<<ntiles, kBlock, 0, st>>>(S, G, a.background_image, ws.colors, sc.err, frag, nullptr);
             }
@@ -1856,7 +1907,7 @@ int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
                     // at most one partial chunk per tile plus nsamp / echunk full ones
                     unsigned grid = (unsigned)(ntiles + (nsamp + G.echunk - 1) / G.echunk);
                     if (S.wave_ok)
-                        k_edge_wave<<<grid, kBlock, 0, st>>>(S, G, ws.edges, ws.tile_off, ws.tile_count, ws.chunk_off,
+                        k_edge_wave<<<grid, 64, 0, st>>>(S, G, ws.edges, ws.tile_off, ws.tile_count, ws.chunk_off,
                                                              ntiles, ws.edge_sorted, a.background_image, ws.weight,
                                                              a.d_render_image, a.d_translation);
                     else if (G.echunk == kBlock)
@@ -2151,12 +2202,14 @@ __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_BATCH_COLOR_PRE : DVG_WAVES
                     PRE ? J.pkeep : nullptr);
 }
 
-__global__ __launch_bounds__(kBlock, DVG_WAVES_COLOR_WAVE) void kb_color_wave(const Job *jobs, const int *pref, int nj) {
+__global__ __launch_bounds__(64, DVG_WAVES_COLOR_WAVE) void kb_color_wave(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
     const Job J = load_job(jobs + j);
     if (!J.img) return;
-    __shared__ ColorWaveLds L;
-    color_tile_wave(L, SceneRef{(uint64_t)&jobs[j].S}, J.G, blockIdx.x - pref[j], J.bg, J.colors, J.err, J.frag);
+    __shared__ WaveLds<1> L;
+    const int b = blockIdx.x - pref[j];
+    color_tile_wave(L, SceneRef{(uint64_t)&jobs[j].S}, J.G, b / kTileWaves, b % kTileWaves, J.bg, J.colors, J.err,
+                    J.frag);
 }
 
 __global__ __launch_bounds__(kBlock) void kb_resolve(const Job *jobs, const int *pref, int nj) {
@@ -2212,13 +2265,13 @@ __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_BATC
                      J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr);
 }
 
-__global__ __launch_bounds__(kBlock, DVG_WAVES_EDGE_WAVE) void kb_edge_wave(const Job *jobs, const int *pref, int nj) {
+__global__ __launch_bounds__(64, DVG_WAVES_EDGE_WAVE) void kb_edge_wave(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
     const Job J = load_job(jobs + j);
     if (!J.d_img) return;
-    __shared__ EdgeWaveLds L;
-    edge_chunk<true, true>(L.e, J.S, J.G, blockIdx.x - pref[j], J.edges, J.tile_off, J.tile_count, J.chunk_off,
-                           J.ntiles, J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr, SceneRef{(uint64_t)&jobs[j].S}, L.w);
+    __shared__ WaveLds<2> L;
+    edge_chunk_wave(L, SceneRef{(uint64_t)&jobs[j].S}, J.G, blockIdx.x - pref[j], J.edges, J.tile_off, J.tile_count,
+                    J.chunk_off, J.ntiles, J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr);
 }
 
 __global__ __launch_bounds__(kBlock, DVG_WAVES_SDF) void kb_sdf(const Job *jobs, const int *pref, int nj) {
@@ -2579,11 +2632,11 @@ int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, i
             case kStTile: return color ? J.ntiles : 0;
             case kStSamp: return edges ? (J.nsamp + kBlock - 1) / kBlock : 0;
             case kStTileF: return J.img && (J.pre || !J.S.wave_ok) ? J.ntiles : 0;
-            case kStTileW: return J.img && !J.pre && J.S.wave_ok ? J.ntiles : 0;
+            case kStTileW: return J.img && !J.pre && J.S.wave_ok ? kTileWaves * J.ntiles : 0;
             case kStChunkW:
                 return edges && J.S.wave_ok ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
             case kStChunk:
-                return edges && J.G.echunk != kBlock ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
+                return edges && J.G.echunk == kEdgeChunk ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
             case kStChunk2:
                 return edges && J.G.echunk == kBlock && !J.S.wave_ok ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
             case kStSdf: return sdf ? (J.eval ? (J.num_eval + kBlock - 1) / kBlock : J.ntiles) : 0;
@@ -2764,7 +2817,7 @@ int batch_render(BatchHost &B, hipStream_t st) {
                     kb_color<1><<<T(kStTileF), kBlock, 0, st>>>(J, P(kStTileF), nj);
                 else if (T(kStTileF))
                     kb_color<0><<<T(kStTileF), kBlock, 0, st>>>(J, P(kStTileF), nj);
-                if (T(kStTileW)) kb_color_wave<<<T(kStTileW), kBlock, 0, st>>>(J, P(kStTileW), nj);
+                if (T(kStTileW)) kb_color_wave<<<T(kStTileW), 64, 0, st>>>(J, P(kStTileW), nj);
             }
             kb_resolve<<<T(kStPix), kBlock, 0, st>>>(J, P(kStPix), nj);
         }
@@ -2787,7 +2840,7 @@ int batch_render(BatchHost &B, hipStream_t st) {
                     DVG_PROF(st, "kb_edge");
                     if (T(kStChunk)) kb_edge<false><<<T(kStChunk), kBlock, 0, st>>>(J, P(kStChunk), nj);
                     if (T(kStChunk2)) kb_edge<true><<<T(kStChunk2), kBlock, 0, st>>>(J, P(kStChunk2), nj);
-                    if (T(kStChunkW)) kb_edge_wave<<<T(kStChunkW), kBlock, 0, st>>>(J, P(kStChunkW), nj);
+                    if (T(kStChunkW)) kb_edge_wave<<<T(kStChunkW), 64, 0, st>>>(J, P(kStChunkW), nj);
                 }
             }
             if (B.fold[c]) kb_fold_grads<<<dim3(8, (unsigned)nj), kBlock, 0, st>>>(J);

@@ -32,7 +32,8 @@
 
 namespace dvg {
 
-constexpr int kWaveSlots = 8;  // at most 16 (queue entries, hit masks)
+constexpr int kWaveSlots = 8;   // at most 16 (queue entries, hit masks)
+constexpr int kWaveList = 256;  // candidates listed at a time
 
 template <int SIDES>
 struct WaveLds {
@@ -42,6 +43,7 @@ struct WaveLds {
     int q1[128];                // screen queue: segment << 10 | slot << 6 | lane
     float q1x[128], q1y[128];   // and the point in the group's space
     int q2[64 + 64 * SIDES];    // exact queue: segment << 11 | side << 10 | slot << 6 | lane
+    int list[kWaveList];        // candidate groups, in increasing order
     int group[kWaveSlots], shape[kWaveSlots];
     float hx[kWaveSlots], hy[kWaveSlots];  // how far the sides lie from the middle, in the group's space
 };
@@ -343,29 +345,12 @@ DVG_DEV void wave_paths(const SceneRef &R, WaveLds<SIDES> &W, unsigned todo, uns
     }
 }
 
-// Coverage of the wave's points by the groups of `list`, in its order: emit(S, g, stroke, a, b)
-// for every group and paint that covers some lane's point (stroke before fill of a group),
-// a and b whether it covers this lane's first and second point.  Every lane of the wave calls
-// it; lanes without a point pass valid = false.  pm: the point the screen uses (SIDES = 1:
-// pa itself); cx, cy: bounds on |pa - pm| and |pb - pm| per canvas coordinate.
+// Coverage of the wave's points by the listed candidates, in their order (wave_shade).
 template <int SIDES, class Emit>
-DVG_DEV void wave_shade(const SceneRef &R, WaveLds<SIDES> &W, const int *list, int n, bool valid, V2 pa, V2 pb, V2 pm,
-                        float cx, float cy, const Emit &emit) {
+DVG_DEV void wave_candidates(const SceneRef &R, WaveLds<SIDES> &W, int n, bool valid, V2 pa, V2 pb, V2 pm, float cx,
+                             float cy, float4 wbox, const Emit &emit) {
     const int lane = threadIdx.x & 63;
-    W.pt[0][lane] = make_float2(pa.x, pa.y);
-    if constexpr (SIDES == 2) W.pt[1][lane] = make_float2(pb.x, pb.y);
-    W.hit[lane] = 0;
-#pragma unroll
-    for (int k = 0; k < kWaveSlots; k++) W.wn[k][lane] = 0;
     const float inf = __builtin_huge_valf();
-    float4 wbox = valid ? make_float4(pm.x, pm.y, pm.x, pm.y) : make_float4(inf, inf, -inf, -inf);
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        wbox.x = fminf(wbox.x, __shfl_xor(wbox.x, o, 64));
-        wbox.y = fminf(wbox.y, __shfl_xor(wbox.y, o, 64));
-        wbox.z = fmaxf(wbox.z, __shfl_xor(wbox.z, o, 64));
-        wbox.w = fmaxf(wbox.w, __shfl_xor(wbox.w, o, 64));
-    }
     for (int base = 0; base < n; base += kWaveSlots) {
         const int cnt = min(kWaveSlots, n - base);
         // which points each candidate's boxes hold (bit slot + 16 side), and shapes without
@@ -373,7 +358,7 @@ DVG_DEV void wave_shade(const SceneRef &R, WaveLds<SIDES> &W, const int *list, i
         unsigned in_s = 0, in_f = 0, paths_s = 0, paths_f = 0;
         for (int k = 0; k < cnt; k++) {
             const DevScene S = R.get();
-            const int g = __builtin_amdgcn_readfirstlane(list[base + k]);
+            const int g = __builtin_amdgcn_readfirstlane(W.list[base + k]);
             const float4 b = S.g_box[g];
             const float mr = S.g_maxr[g];
             const bool a0 = valid && (S.ng == 1 || in_box(b, pa, mr));
@@ -452,6 +437,58 @@ DVG_DEV void wave_shade(const SceneRef &R, WaveLds<SIDES> &W, const int *list, i
         }
         wave_sync();
     }
+}
+
+// Coverage of the wave's points by the scene's groups, in increasing order: emit(S, g, stroke,
+// a, b) for every group and paint that covers some lane's point (stroke before fill of a
+// group), a and b whether it covers this lane's first and second point.  Every lane of the
+// wave calls it; lanes without a point pass valid = false.  pm: the point the screen uses
+// (SIDES = 1: pa itself); cx, cy: bounds on |pa - pm| and |pb - pm| per canvas coordinate.
+// Each wave lists its own candidates, the groups whose inflated top-level box meets the box
+// of its points, so waves do not wait for each other and a wave of 64 samples tests a
+// smaller box than a tile of 256.
+template <int SIDES, class Emit>
+DVG_DEV void wave_shade(const SceneRef &R, WaveLds<SIDES> &W, bool valid, V2 pa, V2 pb, V2 pm, float cx, float cy,
+                        const Emit &emit) {
+    const int lane = threadIdx.x & 63;
+    W.pt[0][lane] = make_float2(pa.x, pa.y);
+    if constexpr (SIDES == 2) W.pt[1][lane] = make_float2(pb.x, pb.y);
+    W.hit[lane] = 0;
+#pragma unroll
+    for (int k = 0; k < kWaveSlots; k++) W.wn[k][lane] = 0;
+    const float inf = __builtin_huge_valf();
+    float4 wbox = valid ? make_float4(pm.x, pm.y, pm.x, pm.y) : make_float4(inf, inf, -inf, -inf);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        wbox.x = fminf(wbox.x, __shfl_xor(wbox.x, o, 64));
+        wbox.y = fminf(wbox.y, __shfl_xor(wbox.y, o, 64));
+        wbox.z = fmaxf(wbox.z, __shfl_xor(wbox.z, o, 64));
+        wbox.w = fmaxf(wbox.w, __shfl_xor(wbox.w, o, 64));
+    }
+    int g0 = 0, ng;
+    do {
+        int n = 0;
+        {
+            const DevScene S = R.get();
+            ng = S.ng;
+            for (; g0 < ng && n <= kWaveList - 64; g0 += 64) {
+                const int g = g0 + lane;
+                bool hit = false;
+                if (g < ng) {
+                    const float4 b = S.g_box[g];
+                    const float r = S.g_maxr[g];
+                    // a single group is the root of the top-level BVH and is visited untested
+                    hit = ng == 1 || !(b.x - r > wbox.z + cx || b.z + r < wbox.x - cx || b.y - r > wbox.w + cy ||
+                                       b.w + r < wbox.y - cy);
+                }
+                const uint64_t m = __ballot(hit);
+                if (hit) W.list[n + rank_below(m)] = g;
+                n += __popcll(m);
+            }
+        }
+        wave_sync();
+        wave_candidates<SIDES>(R, W, n, valid, pa, pb, pm, cx, cy, wbox, emit);
+    } while (g0 < ng);
 }
 
 }  // namespace dvg
