@@ -3589,8 +3589,7 @@ __global__ __launch_bounds__(kBlock) void k_refit_cdf(RefitArgs A) {
 }
 
 // The segment-only parts of the fast cubic tests, one lane per segment, from the scene's
-// current points: wf::cubic_prep in float4 0-2, wf::stroke_prep in float4 3-7, and the control
-// points in float4 8-9.
+// current points: wf::CubicPrep, wf::StrokePrep and the control points (kSegPrep).
 __global__ __launch_bounds__(kBlock) void k_seg_prep(DevScene S) {
     const int seg = blockIdx.x * blockDim.x + threadIdx.x;
     if (seg >= S.nseg) return;
@@ -3602,15 +3601,14 @@ __global__ __launch_bounds__(kBlock) void k_seg_prep(DevScene S) {
     const int4 idx = S.seg_idx[seg];
     const float2 a = S.points[idx.x], b = S.points[idx.y], c = S.points[idx.z], d = S.points[idx.w];
     const wf::CubicPrep q = wf::cubic_prep(a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y);
-    dst[0] = make_float4(q.my, q.mx, q.E, q.ddy);
-    dst[1] = make_float4(q.ddx, q.ddmax, q.xdmax, q.br1);
-    dst[2] = make_float4(q.br2, 0.f, 0.f, 0.f);
-    float poly[16], mc, dev;
-    wf::stroke_prep(a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y, poly, mc, dev);
-    for (int i = 0; i < 4; i++) dst[3 + i] = make_float4(poly[4 * i], poly[4 * i + 1], poly[4 * i + 2], poly[4 * i + 3]);
-    dst[7] = make_float4(mc, dev, 0.f, 0.f);
-    dst[8] = make_float4(a.x, a.y, b.x, b.y);
-    dst[9] = make_float4(c.x, c.y, d.x, d.y);
+    const wf::StrokePrep t = wf::stroke_prep(a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y);
+    float4 v[kSegPoints];
+    __builtin_memcpy(v, &q, sizeof(q));
+    __builtin_memcpy(v + kSegStroke, &t, sizeof(t));
+#pragma unroll
+    for (int i = 0; i < kSegPoints; i++) dst[i] = v[i];
+    dst[kSegPoints] = make_float4(a.x, a.y, b.x, b.y);
+    dst[kSegPoints + 1] = make_float4(c.x, c.y, d.x, d.y);
 }
 
 int prep_segments(SceneHost &sc, hipStream_t st) {

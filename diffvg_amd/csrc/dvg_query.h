@@ -42,6 +42,34 @@ DVG_DEV int seg_load(const DevScene &S, int seg, V2 *p, int4 &idx) {
     if (k >= 2) p[3] = ld_pt(S, idx.w);
     return k;
 }
+// The per-segment tables of the fast cubic tests (cubic segments only)
+DVG_DEV wf::CubicPrep cubic_prep_of(const DevScene &S, int seg) {
+    const float4 *src = S.seg_wf + kSegPrep * (size_t)seg;
+    float4 v[wf::kPrepFloats / 4];
+#pragma unroll
+    for (int i = 0; i < wf::kPrepFloats / 4; i++) v[i] = src[i];
+    wf::CubicPrep q;
+    __builtin_memcpy(&q, v, sizeof(q));
+    return q;
+}
+DVG_DEV wf::StrokePrep stroke_prep_of(const DevScene &S, int seg) {
+    const float4 *src = S.seg_wf + kSegPrep * (size_t)seg + kSegStroke;
+    float4 v[wf::kStrokeFloats / 4];
+#pragma unroll
+    for (int i = 0; i < wf::kStrokeFloats / 4; i++) v[i] = src[i];
+    wf::StrokePrep q;
+    __builtin_memcpy(&q, v, sizeof(q));
+    return q;
+}
+struct CubicPoints {
+    V2 p0, p1, p2, p3;
+};
+DVG_DEV CubicPoints cubic_points_of(const DevScene &S, int seg) {
+    const float4 *src = S.seg_wf + kSegPrep * (size_t)seg + kSegPoints;
+    const float4 a = src[0], b = src[1];
+    return CubicPoints{V2{a.x, a.y}, V2{a.z, a.w}, V2{b.x, b.y}, V2{b.z, b.w}};
+}
+
 DVG_DEV V2 qeval(V2 p0, V2 p1, V2 p2, float t) {
     float tt = 1 - t;
     return (tt * tt) * p0 + (2 * tt * t) * p1 + (t * t) * p2;
@@ -109,19 +137,21 @@ DVG_DEV int segment_winding_lq(int k, const V2 *p, V2 pt) {
     return w;
 }
 
-// Winding contribution of one segment (winding_number.h:58-167)
-// `prep`: the segment's wf::CubicPrep as three float4 (cubic segments only)
-DVG_DEV int segment_winding(int k, const V2 *p, V2 pt, const float4 *prep) {
-    if (k != 2) return segment_winding_lq(k, p, pt);
-    V2 p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
+// Winding contribution of segment `seg` (winding_number.h:58-167)
+DVG_DEV int segment_winding(const DevScene &S, int seg, V2 pt) {
+    const int k = S.seg_kind[seg];
+    if (k != 2) {
+        V2 p[4];
+        int4 idx;
+        seg_load(S, seg, p, idx);
+        return segment_winding_lq(k, p, pt);
+    }
     // decided in float whenever every decision of the reference is certain
     // (dvg_winding_fast.h); otherwise the reference's double solve
-    int wfast = 0;
-    const float4 q0 = prep[0], q1 = prep[1], q2 = prep[2];
-    const wf::CubicPrep q{q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x};
-    if (wf::cubic_winding_fast_prep(q, p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y, pt.x, pt.y, wfast))
-        return wfast;
-    return cubic_winding_solve(p0, p1, p2, p3, pt);
+    int w = 0;
+    if (wf::cubic_winding_test<true>(cubic_prep_of(S, seg), pt.x, pt.y, w)) return w;
+    const CubicPoints c = cubic_points_of(S, seg);
+    return cubic_winding_solve(c.p0, c.p1, c.p2, c.p3, pt);
 }
 
 DVG_DEV int winding_path(const DevScene &S, int s, V2 pt) {
@@ -130,10 +160,7 @@ DVG_DEV int winding_path(const DevScene &S, int s, V2 pt) {
     for (int i = 0; i < n; i++) {
         int seg = b + i;  // the winding sum is order independent
         if (n > 1 && !ray_box(S.seg_box[seg], pt)) continue;
-        V2 p[4];
-        int4 idx;
-        int k = seg_load(S, seg, p, idx);
-        wn += segment_winding(k, p, pt, S.seg_wf + kSegPrep * (size_t)seg);
+        wn += segment_winding(S, seg, pt);
     }
     return wn;
 }
@@ -273,18 +300,8 @@ DVG_DEV float quintic_root(const Quintic &q, float lb, float ub) {
 // Every point of cubic segment `seg` is certainly farther than r from pt (the chords of an
 // 8-step polyline, the chords' deviation bound and a rounding margin, from the segment's
 // prep); false for r = inf.
-DVG_DEV bool cubic_farther_than(const DevScene &S, int seg, V2 p0, V2 pt, float r) {
-    const float4 *q = S.seg_wf + kSegPrep * (size_t)seg + 3;
-    float poly[16];
-    for (int i = 0; i < 4; i++) {
-        const float4 v = q[i];
-        poly[4 * i] = v.x;
-        poly[4 * i + 1] = v.y;
-        poly[4 * i + 2] = v.z;
-        poly[4 * i + 3] = v.w;
-    }
-    const float4 md = q[4];
-    return wf::cubic_certainly_farther_prep(poly, md.x, md.y, p0.x, p0.y, pt.x, pt.y, r);
+DVG_DEV bool cubic_farther_than(const DevScene &S, int seg, V2 pt, float r) {
+    return wf::stroke_farther(stroke_prep_of(S, seg), pt.x, pt.y, r);
 }
 
 // Whether one of the stationary points of the distance to a cubic that the quintic search
@@ -318,37 +335,18 @@ DVG_DEV bool cubic_stroke_search(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, fl
     return false;
 }
 
-// One line (k = 0) or quadratic (k = 1) stroke segment test of within_distance
-// (within_distance.h:32-118).  Returns 1 (hit), 0 (miss) or -1 (quadratic
-// distance-approximation miss, which ends the whole path query in the reference).
-DVG_DEV int segment_within_lq(const DevScene &S, int s, int k, const V2 *p, int4 idx, V2 pt, float r) {
-    const bool thick = S.has_thick[s] != 0;
-    if (k == 0) {
-        V2 p0 = p[0], p1 = p[1];
-        float t = dot(pt - p0, p1 - p0) / dot(p1 - p0, p1 - p0);
-        float r0 = r, r1 = r;
-        if (thick) {
-            r0 = S.thickness[idx.x];
-            r1 = S.thickness[idx.y];
-        }
-        if (t < 0) return dist_sq(p0, pt) < r0 * r0;
-        if (t > 1) return dist_sq(p1, pt) < r1 * r1;
-        float rr = r0 + t * (r1 - r0);
-        return dist_sq(p0 + t * (p1 - p0), pt) < rr * rr;
-    }
-    V2 p0 = p[0], p1 = p[1], p2 = p[2];
-    if (S.approx[s]) {
-        V2 cp = quadratic_closest_pt_approx(p0, p1, p2, pt);
-        return dist_sq(cp, pt) < r * r ? 1 : -1;
-    }
-    float r0 = r, r1 = r, r2 = r;
-    if (thick) {
-        r0 = S.thickness[idx.x];
-        r1 = S.thickness[idx.y];
-        r2 = S.thickness[idx.z];
-    }
-    if (dist_sq(qeval(p0, p1, p2, 0), pt) < r0 * r0) return 1;
-    if (dist_sq(qeval(p0, p1, p2, 1), pt) < r2 * r2) return 1;
+// Stroke test of a line and of a quadratic segment (within_distance.h:32-118), radius r0, r1
+// (r2) at the points.
+DVG_DEV bool line_within(V2 p0, V2 p1, V2 pt, float r0, float r1) {
+    float t = dot(pt - p0, p1 - p0) / dot(p1 - p0, p1 - p0);
+    if (t < 0) return dist_sq(p0, pt) < r0 * r0;
+    if (t > 1) return dist_sq(p1, pt) < r1 * r1;
+    float rr = r0 + t * (r1 - r0);
+    return dist_sq(p0 + t * (p1 - p0), pt) < rr * rr;
+}
+DVG_DEV bool quad_within(V2 p0, V2 p1, V2 p2, V2 pt, float r0, float r1, float r2) {
+    if (dist_sq(qeval(p0, p1, p2, 0), pt) < r0 * r0) return true;
+    if (dist_sq(qeval(p0, p1, p2, 1), pt) < r2 * r2) return true;
     float A = vsum((p0 - 2 * p1 + p2) * (p0 - 2 * p1 + p2));
     float B = vsum(3 * (p0 - 2 * p1 + p2) * (-p0 + p1));
     float C = vsum(2 * (-p0 + p1) * (-p0 + p1) + (p0 - 2 * p1 + p2) * (p0 - pt));
@@ -360,10 +358,26 @@ DVG_DEV int segment_within_lq(const DevScene &S, int s, int k, const V2 *p, int4
         if (j < num_sol && t[j] >= 0 && t[j] <= 1) {
             float tt = 1 - t[j];
             float rr = (tt * tt) * r0 + (2 * tt * t[j]) * r1 + (t[j] * t[j]) * r2;
-            if (dist_sq(qeval(p0, p1, p2, t[j]), pt) < rr * rr) return 1;
+            if (dist_sq(qeval(p0, p1, p2, t[j]), pt) < rr * rr) return true;
         }
     }
-    return 0;
+    return false;
+}
+// One line (k = 0) or quadratic (k = 1) stroke segment test of within_distance
+// (within_distance.h:32-118).  Returns 1 (hit), 0 (miss) or -1 (quadratic
+// distance-approximation miss, which ends the whole path query in the reference).
+DVG_DEV int segment_within_lq(const DevScene &S, int s, int k, const V2 *p, int4 idx, V2 pt, float r) {
+    if (k == 1 && S.approx[s]) {
+        V2 cp = quadratic_closest_pt_approx(p[0], p[1], p[2], pt);
+        return dist_sq(cp, pt) < r * r ? 1 : -1;
+    }
+    float r0 = r, r1 = r, r2 = r;
+    if (S.has_thick[s]) {
+        r0 = S.thickness[idx.x];
+        r1 = S.thickness[idx.y];
+        if (k == 1) r2 = S.thickness[idx.z];
+    }
+    return k == 0 ? line_within(p[0], p[1], pt, r0, r1) : quad_within(p[0], p[1], p[2], pt, r0, r1, r2);
 }
 
 // One stroke segment test of within_distance (within_distance.h:32-276); results as above.
@@ -385,21 +399,7 @@ DVG_DEV int segment_within(const DevScene &S, int s, int seg, V2 pt, float r) {
     if (dist_sq(ceval(p0, p1, p2, p3, 1), pt) < r3 * r3) return 1;
     // every curve point certainly farther than the largest radius magnitude (the radius
     // at t is a convex combination of r0..r3): the quintic search below would find nothing
-    {
-        const float4 *q = S.seg_wf + kSegPrep * (size_t)seg + 3;
-        float poly[16];
-        for (int i = 0; i < 4; i++) {
-            const float4 v = q[i];
-            poly[4 * i] = v.x;
-            poly[4 * i + 1] = v.y;
-            poly[4 * i + 2] = v.z;
-            poly[4 * i + 3] = v.w;
-        }
-        const float4 md = q[4];
-        if (wf::cubic_certainly_farther_prep(poly, md.x, md.y, p0.x, p0.y, pt.x, pt.y,
-                                             fmaxf(fmaxf(fabsf(r0), fabsf(r1)), fmaxf(fabsf(r2), fabsf(r3)))))
-            return 0;
-    }
+    if (cubic_farther_than(S, seg, pt, fmaxf(fmaxf(fabsf(r0), fabsf(r1)), fmaxf(fabsf(r2), fabsf(r3))))) return 0;
     return cubic_stroke_search(p0, p1, p2, p3, pt, r0, r1, r2, r3);
 }
 
@@ -579,7 +579,7 @@ DVG_DEV bool closest_point_path(const DevScene &S, int s, V2 pt, float max_radiu
         float tr;
         float dd;
         if (S.seg_kind[seg] == 2) {
-            if (cubic_farther_than(S, seg, ld_pt(S, S.seg_idx[seg].x), pt, min_dist)) continue;
+            if (cubic_farther_than(S, seg, pt, min_dist)) continue;
             dd = cubic_closest(S, seg, pt, cp, tr);
         } else {
             dd = segment_closest_lq(S, s, seg, pt, cp, tr);

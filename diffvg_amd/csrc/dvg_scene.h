@@ -32,9 +32,10 @@ struct BNode {  // BVHNode (reference scene.h:12-16), padded to 32 bytes
     int pad;
 };
 
-// float4 per segment of DevScene::seg_wf: wf::CubicPrep (3), wf::stroke_prep (5), the four
+// float4 per segment of DevScene::seg_wf: wf::CubicPrep (6), wf::StrokePrep (7), the four
 // control points (2)
-constexpr int kSegPrep = 10;
+constexpr int kSegPrep = 15;
+constexpr int kSegStroke = 6, kSegPoints = 13;
 
 // What the wave-cooperative coverage tests (dvg_wave.h) take: every group has one shape, no
 // path uses the approximate quadratic distance (its first miss ends the path's query, so its

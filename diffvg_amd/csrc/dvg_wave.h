@@ -74,6 +74,24 @@ static __device__ __noinline__ int wave_winding_solve(V2 p0, V2 p1, V2 p2, V2 p3
     return cubic_winding_solve(p0, p1, p2, p3, pt);
 }
 
+static __device__ __noinline__ bool wave_quad_within(V2 p0, V2 p1, V2 p2, V2 pt, float r0, float r1, float r2) {
+    return quad_within(p0, p1, p2, pt, r0, r1, r2);
+}
+// segment_within_lq for paths without the approximate quadratic distance
+DVG_DEV bool wave_within_lq(const DevScene &S, int s, int seg, int k, V2 pt, float r) {
+    V2 p[4];
+    int4 idx;
+    seg_load(S, seg, p, idx);
+    float r0 = r, r1 = r, r2 = r;
+    if (S.has_thick[s]) {
+        r0 = S.thickness[idx.x];
+        r1 = S.thickness[idx.y];
+        if (k == 1) r2 = S.thickness[idx.z];
+    }
+    if (k == 0) return line_within(p[0], p[1], pt, r0, r1);
+    return wave_quad_within(p[0], p[1], p[2], pt, r0, r1, r2);
+}
+
 // Orders the wave's LDS accesses (a wave's LDS instructions execute in order; this keeps the
 // compiler from moving them).
 DVG_DEV void wave_sync() {
@@ -109,14 +127,13 @@ DVG_DEV void wave_exact(const SceneRef &R, WaveLds<SIDES> &W, int &n2, int cnt) 
         const V2 p = xform_pt(m3_load(S.c2s + 9 * g), V2{c.x, c.y});
         const bool one = S.nsegs[s] == 1;
         const int k = S.seg_kind[seg];
-        const float4 *prep = S.seg_wf + kSegPrep * (size_t)seg;
         if constexpr (STROKE) {
             const int bit = 1 << (slot + 16 * side);
             if (!(W.hit[owner] & bit) && (one || in_box(S.seg_box[seg], p, S.seg_maxr[seg]))) {
                 const float r = S.stroke_width[s];
                 bool hit;
                 if (k == 2) {
-                    const float4 a = prep[8], b = prep[9];
+                    const CubicPoints c = cubic_points_of(S, seg);
                     float r0 = r, r1 = r, r2 = r, r3 = r;
                     if (S.has_thick[s]) {
                         const int4 idx = S.seg_idx[seg];
@@ -125,25 +142,20 @@ DVG_DEV void wave_exact(const SceneRef &R, WaveLds<SIDES> &W, int &n2, int cnt) 
                         r2 = S.thickness[idx.z];
                         r3 = S.thickness[idx.w];
                     }
-                    const V2 p0{a.x, a.y}, p3{b.z, b.w};
-                    hit = dist_sq(p0, p) < r0 * r0 || dist_sq(p3, p) < r3 * r3;
-                    if (!hit) hit = wave_stroke_search(p0, V2{a.z, a.w}, V2{b.x, b.y}, p3, p, r0, r1, r2, r3);
+                    hit = dist_sq(c.p0, p) < r0 * r0 || dist_sq(c.p3, p) < r3 * r3;
+                    if (!hit) hit = wave_stroke_search(c.p0, c.p1, c.p2, c.p3, p, r0, r1, r2, r3);
                 } else {
-                    V2 q[4];
-                    int4 idx;
-                    seg_load(S, seg, q, idx);
-                    hit = segment_within_lq(S, s, k, q, idx, p, r) > 0;
+                    hit = wave_within_lq(S, s, seg, k, p, r);
                 }
                 if (hit) atomicOr(&W.hit[owner], bit);
             }
         } else if (one || ray_box(S.seg_box[seg], p)) {
             int w = 0;
             if (k == 2) {
-                const float4 q0 = prep[0], q1 = prep[1], q2 = prep[2], a = prep[8], b = prep[9];
-                const wf::CubicPrep q{q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x};
-                // one point: the screen has tried the float test with it
-                if (SIDES == 1 || !wf::cubic_winding_fast_prep(q, a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, p.x, p.y, w))
-                    w = wave_winding_solve(V2{a.x, a.y}, V2{a.z, a.w}, V2{b.x, b.y}, V2{b.z, b.w}, p);
+                if (!wf::cubic_winding_test<true>(cubic_prep_of(S, seg), p.x, p.y, w)) {
+                    const CubicPoints c = cubic_points_of(S, seg);
+                    w = wave_winding_solve(c.p0, c.p1, c.p2, c.p3, p);
+                }
             } else {
                 V2 q[4];
                 int4 idx;
@@ -170,7 +182,6 @@ DVG_DEV void wave_screen(const SceneRef &R, WaveLds<SIDES> &W, int &n1, int &n2,
         const V2 pt{W.q1x[n1 + lane], W.q1y[n1 + lane]};
         const int owner = id & 63, slot = (id >> 6) & 15, seg = id >> 10;
         const float hx = SIDES == 2 ? W.hx[slot] : 0.f, hy = SIDES == 2 ? W.hy[slot] : 0.f;
-        const float4 *prep = S.seg_wf + kSegPrep * (size_t)seg;
         const int k = S.seg_kind[seg];
         if constexpr (STROKE) {
             const int s = W.shape[slot];
@@ -178,7 +189,7 @@ DVG_DEV void wave_screen(const SceneRef &R, WaveLds<SIDES> &W, int &n1, int &n2,
             if ((W.hit[owner] & (both << slot)) != (both << slot)) {
                 const float r = S.stroke_width[s];
                 if (k == 2) {
-                    const float4 a = prep[8], b = prep[9], md = prep[7];
+                    const wf::StrokePrep q = stroke_prep_of(S, seg);
                     float r0 = r, r3 = r, rmax = fabsf(r);
                     if (S.has_thick[s]) {
                         const int4 idx = S.seg_idx[seg];
@@ -187,14 +198,14 @@ DVG_DEV void wave_screen(const SceneRef &R, WaveLds<SIDES> &W, int &n1, int &n2,
                         rmax = fmaxf(fmaxf(fabsf(r0), fabsf(S.thickness[idx.y])),
                                      fmaxf(fabsf(S.thickness[idx.z]), fabsf(r3)));
                     }
-                    const V2 p0{a.x, a.y}, p3{b.z, b.w};
+                    const V2 p0{q.x[0], q.y[0]}, p3{q.x[8], q.y[8]};
                     bool hit;
                     float reach = 0.f;
                     if constexpr (SIDES == 2) {
                         // within both points' reach of an end of the curve, with a margin for
                         // rounding
                         reach = hx + hy;
-                        const float less = reach + 1e-4f * (fmaxf(md.x, fmaxf(fabsf(pt.x), fabsf(pt.y))) + 1.f);
+                        const float less = reach + 1e-4f * (fmaxf(q.mc, fmaxf(fabsf(pt.x), fabsf(pt.y))) + 1.f);
                         const float c0 = r0 - less, c3 = r3 - less;
                         hit = (c0 > 0.f && dist_sq(p0, pt) < c0 * c0) || (c3 > 0.f && dist_sq(p3, pt) < c3 * c3);
                     } else {
@@ -203,22 +214,10 @@ DVG_DEV void wave_screen(const SceneRef &R, WaveLds<SIDES> &W, int &n1, int &n2,
                     if (hit) {
                         atomicOr(&W.hit[owner], both << slot);
                     } else {
-                        float poly[16];
-#pragma unroll
-                        for (int i = 0; i < 4; i++) {
-                            const float4 v = prep[3 + i];
-                            poly[4 * i] = v.x;
-                            poly[4 * i + 1] = v.y;
-                            poly[4 * i + 2] = v.z;
-                            poly[4 * i + 3] = v.w;
-                        }
-                        open = !wf::cubic_certainly_farther_prep(poly, md.x, md.y, p0.x, p0.y, pt.x, pt.y, rmax + reach);
+                        open = !wf::stroke_farther(q, pt.x, pt.y, rmax + reach);
                     }
                 } else if constexpr (SIDES == 1) {
-                    V2 p[4];
-                    int4 idx;
-                    seg_load(S, seg, p, idx);
-                    if (segment_within_lq(S, s, k, p, idx, pt, r) > 0) atomicOr(&W.hit[owner], both << slot);
+                    if (wave_within_lq(S, s, seg, k, pt, r)) atomicOr(&W.hit[owner], both << slot);
                 } else {
                     open = true;
                 }
@@ -226,9 +225,7 @@ DVG_DEV void wave_screen(const SceneRef &R, WaveLds<SIDES> &W, int &n1, int &n2,
         } else {
             int w = 0;
             if (k == 2) {
-                const float4 q0 = prep[0], q1 = prep[1], q2 = prep[2], a = prep[8], b = prep[9];
-                const wf::CubicPrep q{q0.x, q0.y, q0.z, q0.w, q1.x, q1.y, q1.z, q1.w, q2.x};
-                open = !wf::cubic_winding_fast_prep(q, a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w, pt.x, pt.y, w, hx, hy);
+                open = !wf::cubic_winding_test<false>(cubic_prep_of(S, seg), pt.x, pt.y, w, hx, hy);
             } else if constexpr (SIDES == 1) {
                 V2 p[4];
                 int4 idx;

@@ -122,8 +122,8 @@ void wf_fuzz_box(int near, int64_t n, uint64_t seed, int64_t *out, float *bad) {
         if (!near) m = orc::V2{cx + 1.5f * sp * N(g), cy + 1.5f * sp * N(g)};
         const dvg::wf::CubicPrep q = dvg::wf::cubic_prep(p[0].x, p[0].y, p[1].x, p[1].y, p[2].x, p[2].y, p[3].x, p[3].y);
         int w = 0;
-        if (!dvg::wf::cubic_winding_fast_prep(q, p[0].x, p[0].y, p[1].x, p[1].y, p[2].x, p[2].y, p[3].x, p[3].y, m.x,
-                                              m.y, w, hx, hy))
+        if (!(seed & 1 ? dvg::wf::cubic_winding_test<true>(q, m.x, m.y, w, hx, hy)
+                       : dvg::wf::cubic_winding_test<false>(q, m.x, m.y, w, hx, hy)))
             continue;
         decided++;
         for (int k = 0; k < 8; k++) {
