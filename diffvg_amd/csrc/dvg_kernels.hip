@@ -58,23 +58,50 @@ constexpr int kPFragWords = 9;
 // they were.
 constexpr int64_t kPrimDirect = 12288;
 // Waves per SIMD each heavy shading kernel is compiled for, i.e. its register budget
-// (512 / waves VGPRs per lane; beyond it the compiler spills to scratch).  Chosen by
-// measurement on the 300-path and 2,048-stroke scenes: these kernels wait on memory and
-// on long FP64 dependency chains, and 4-6 waves hide that better than 2 waves without
-// spills (k_edge 5.03 -> 3.16 ms, k_color 1.45 -> 0.92 ms, k_color_bwd 1.90 -> 1.33 ms);
-// the colour backward, which mostly replays kept fragment lists, is best at 4.
+// (512 / waves VGPRs per lane; beyond it the compiler spills to scratch), chosen by
+// measurement (MI355X; 300 paths and 2,048 strokes at 512x512, 256 uneven scenes as a batch).
+// the kernels with the wave-cooperative coverage tests, one wave per workgroup: the single
+// forward takes 793 / 348 us at 5 waves, 813 / 350 at 6; the batched one 6.54 ms at 6, 6.77 at
+// 5, 7.3 at 7; the edge kernel 1477 / 875 us and 12.3 ms at 5, 1572 / 917 and 13.0 at 4
+#ifndef DVG_WAVES_COLOR_WAVE
+#define DVG_WAVES_COLOR_WAVE 5
+#endif
+#ifndef DVG_WAVES_BATCH_COLOR_WAVE
+#define DVG_WAVES_BATCH_COLOR_WAVE 6
+#endif
+#ifndef DVG_WAVES_EDGE_WAVE
+#define DVG_WAVES_EDGE_WAVE 5
+#endif
+// the per-lane tests (scenes with groups of several shapes): as measured before the
+// double-precision searches were called rather than inlined
 #ifndef DVG_WAVES_COLOR
 #define DVG_WAVES_COLOR 5
 #endif
+#ifndef DVG_WAVES_BATCH_COLOR
+#define DVG_WAVES_BATCH_COLOR 3
+#endif
+#ifndef DVG_WAVES_EDGE
+#define DVG_WAVES_EDGE 6
+#endif
+#ifndef DVG_WAVES_BATCH_EDGE
+#define DVG_WAVES_BATCH_EDGE 5
+#endif
+// the edge kernel with both sides of a sample per lane keeps two compositors live
+#ifndef DVG_WAVES_EDGE_BOTH
+#define DVG_WAVES_EDGE_BOTH 5
+#endif
+// the colour backward, which mostly replays kept fragment lists: 339 us (300 paths) and 5.26
+// ms (batch) at 4 waves, 374 / 6.23 at 3, 408 / 6.09 at 5
 #ifndef DVG_WAVES_COLOR_BWD
 #define DVG_WAVES_COLOR_BWD 4
 #endif
-// the prefiltered instantiations keep more state per lane: on the 300-path scene
-// k_color<1> takes 3.69 ms at 3 waves, 3.75 at 5, and k_color_bwd<1> 1.71 at 3, 1.69 at 4
-// (the same within run-to-run spread); the batched forward stays at 5 (serving stream:
-// 1.91 ms at 5, 2.16 at 4)
+#ifndef DVG_WAVES_BATCH_COLOR_BWD
+#define DVG_WAVES_BATCH_COLOR_BWD 4
+#endif
+// prefiltered: forward 1.02 ms at 5 waves, 1.08 at 4, 1.19 at 3, 1.10 at 6 (300 paths);
+// backward 0.74 at 3 and 4, 0.89 at 2
 #ifndef DVG_WAVES_COLOR_PRE
-#define DVG_WAVES_COLOR_PRE 3
+#define DVG_WAVES_COLOR_PRE 5
 #endif
 #ifndef DVG_WAVES_BATCH_COLOR_PRE
 #define DVG_WAVES_BATCH_COLOR_PRE 5
@@ -82,37 +109,10 @@ constexpr int64_t kPrimDirect = 12288;
 #ifndef DVG_WAVES_COLOR_BWD_PRE
 #define DVG_WAVES_COLOR_BWD_PRE 3
 #endif
-#ifndef DVG_WAVES_EDGE
-#define DVG_WAVES_EDGE 6
-#endif
-// the kernels with the wave-cooperative coverage tests
-#ifndef DVG_WAVES_COLOR_WAVE
-#define DVG_WAVES_COLOR_WAVE 6
-#endif
-#ifndef DVG_WAVES_EDGE_WAVE
-#define DVG_WAVES_EDGE_WAVE 5
-#endif
-// the edge kernel with both sides of a sample per lane keeps two compositors live
-#ifndef DVG_WAVES_EDGE_BOTH
-#define DVG_WAVES_EDGE_BOTH 5
-#endif
-// the batched edge kernel (job lookup and per-job fields live across its loop) measured
-// fastest at 5 (256 uneven scenes: 31.1 ms at 5, 33.1 at 4, 46.2 at 6, 46.6 at 7)
-// the batched forward (job lookup live across its loop) measured fastest at 3 (256 uneven
-// scenes: 13.2 ms at 3, 14.3 at 4, 20.7 at 5)
-#ifndef DVG_WAVES_BATCH_COLOR
-#define DVG_WAVES_BATCH_COLOR 3
-#endif
-#ifndef DVG_WAVES_BATCH_EDGE
-#define DVG_WAVES_BATCH_EDGE 5
-#endif
+// distance field of 300 paths at 256x256, forward + backward: 1.31 ms at 4 waves, 1.34 at 5,
+// 1.43 at 6
 #ifndef DVG_WAVES_SDF
-#define DVG_WAVES_SDF 5
-#endif
-// the batched backward (job lookup live across its loop; it mostly replays kept fragment
-// lists) measured fastest at 4 (256 uneven scenes: 15.0 ms at 4, 16.3 at 3, 18.1 at 2)
-#ifndef DVG_WAVES_BATCH_COLOR_BWD
-#define DVG_WAVES_BATCH_COLOR_BWD 4
+#define DVG_WAVES_SDF 4
 #endif
 // the persistent batch kernel runs every stage in one launch, so one setting for all
 #ifndef DVG_WAVES_PERSIST
@@ -2202,7 +2202,7 @@ __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_BATCH_COLOR_PRE : DVG_WAVES
                     PRE ? J.pkeep : nullptr);
 }
 
-__global__ __launch_bounds__(64, DVG_WAVES_COLOR_WAVE) void kb_color_wave(const Job *jobs, const int *pref, int nj) {
+__global__ __launch_bounds__(64, DVG_WAVES_BATCH_COLOR_WAVE) void kb_color_wave(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
     const Job J = load_job(jobs + j);
     if (!J.img) return;

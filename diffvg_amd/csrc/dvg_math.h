@@ -287,18 +287,6 @@ DVG_DEV int solve_cubic_d(double a, double b, double c, double d, double t[3]) {
     }
 }
 
-// Out of line, so that the rarely taken correctly rounded solve does not add to the
-// register budget of the kernels that inline the fast one.
-static __device__ inline int solve_cubic_d_cr(double a, double b, double c, double d, double &t0, double &t1,
-                                              double &t2) {
-    double t[3] = {0.0, 0.0, 0.0};
-    const int n = solve_cubic_d<true>(a, b, c, d, t);
-    t0 = t[0];
-    t1 = t[1];
-    t2 = t[2];
-    return n;
-}
-
 // ---- pixel filters (reference filter.h:22-106) and the Gaussian extension ----
 enum { kBox = 0, kTent = 1, kParabolic = 2, kHann = 3, kGaussian = 4 };
 

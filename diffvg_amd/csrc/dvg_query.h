@@ -79,19 +79,21 @@ DVG_DEV V2 ceval(V2 p0, V2 p1, V2 p2, V2 p3, float t) {
     return (tt * tt * tt) * p0 + (3 * tt * tt * t) * p1 + (3 * tt * t * t) * p2 + (t * t * t) * p3;
 }
 
-// Winding contribution of a cubic by the reference's double solve (winding_number.h:119-157)
-DVG_DEV int cubic_winding_solve(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
-    int w = 0;
+// The searches in double precision are called, not inlined: their constants and intermediates
+// then stay out of the register allocation of the loops around them.  They make no calls
+// themselves where that can be had: a value kept across a call takes a higher register, and a
+// kernel needs as many registers as the highest of what it calls.
+struct CubicRoots {
+    double t0, t1, t2;
+    int n;
+};
+static __device__ __noinline__ CubicRoots cubic_roots_cr(double a, double b, double c, double d) {
     double t[3] = {0.0, 0.0, 0.0};
-    double ca = (double)(-p0.y + 3 * p1.y - 3 * p2.y + p3.y), cb = (double)(3 * p0.y - 6 * p1.y + 3 * p2.y),
-           cc = (double)(-3 * p0.y + 3 * p1.y), cd = (double)(p0.y - pt.y);
-    int num_sol = solve_cubic_d(ca, cb, cc, cd, t);
-    // a root at a segment end is counted by the side its last bit falls on: take
-    // that bit from correctly rounded libm functions, as the host libm gives it
-    bool edge = false;
-#pragma unroll
-    for (int j = 0; j < 3; j++) edge |= j < num_sol && (fabs(t[j]) < 1e-9 || fabs(t[j] - 1.0) < 1e-9);
-    if (edge) num_sol = solve_cubic_d_cr(ca, cb, cc, cd, t[0], t[1], t[2]);
+    const int n = solve_cubic_d<true>(a, b, c, d, t);
+    return CubicRoots{t[0], t[1], t[2], n};
+}
+DVG_DEV int winding_at_roots(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, const CubicRoots &r) {
+    int w = 0;
     float ax = -p0.x + 3 * p1.x - 3 * p2.x + p3.x;
     float bx = 3 * p0.x - 6 * p1.x + 3 * p2.x;
     float cx = -3 * p0.x + 3 * p1.x;
@@ -100,13 +102,35 @@ DVG_DEV int cubic_winding_solve(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
     float cy = -3 * p0.y + 3 * p1.y;
 #pragma unroll
     for (int j = 0; j < 3; j++) {
-        double tj = t[j];
-        if (j < num_sol && tj >= 0 && tj <= 1) {
+        double tj = j == 0 ? r.t0 : (j == 1 ? r.t1 : r.t2);
+        if (j < r.n && tj >= 0 && tj <= 1) {
             double tp = ax * tj * tj * tj + bx * tj * tj + cx * tj + p0.x - pt.x;
             if (tp > 0) w += (ay3 * tj * tj + by2 * tj + cy > 0) ? 1 : -1;
         }
     }
     return w;
+}
+// Winding contribution of a cubic by the reference's double solve (winding_number.h:119-157),
+// times two, plus one when some root lies at a segment end
+static __device__ __noinline__ int cubic_winding_libm(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
+    double t[3] = {0.0, 0.0, 0.0};
+    double ca = (double)(-p0.y + 3 * p1.y - 3 * p2.y + p3.y), cb = (double)(3 * p0.y - 6 * p1.y + 3 * p2.y),
+           cc = (double)(-3 * p0.y + 3 * p1.y), cd = (double)(p0.y - pt.y);
+    const int n = solve_cubic_d(ca, cb, cc, cd, t);
+    bool edge = false;
+#pragma unroll
+    for (int j = 0; j < 3; j++) edge |= j < n && (fabs(t[j]) < 1e-9 || fabs(t[j] - 1.0) < 1e-9);
+    return 2 * winding_at_roots(p0, p1, p2, p3, pt, CubicRoots{t[0], t[1], t[2], n}) + (edge ? 1 : 0);
+}
+DVG_DEV int cubic_winding_solve(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
+    const int code = cubic_winding_libm(p0, p1, p2, p3, pt);
+    if (!(code & 1)) return code >> 1;
+    // a root at a segment end is counted by the side its last bit falls on: take that bit
+    // from correctly rounded libm functions, as the host libm gives it
+    return winding_at_roots(p0, p1, p2, p3, pt,
+                            cubic_roots_cr((double)(-p0.y + 3 * p1.y - 3 * p2.y + p3.y),
+                                           (double)(3 * p0.y - 6 * p1.y + 3 * p2.y), (double)(-3 * p0.y + 3 * p1.y),
+                                           (double)(p0.y - pt.y)));
 }
 
 // Winding contribution of a line (k = 0) or quadratic (k = 1) segment (winding_number.h:58-118)
@@ -221,8 +245,16 @@ DVG_DEV V2 quadratic_closest_pt_approx(V2 b0, V2 b1, V2 b2, V2 pt, float *t_ = n
     return (tt * tt) * b0 + (2 * tt * t) * b1 + (t * t) * b2 + pt;
 }
 
+// The stationary points of the distance to a cubic: roots of a quintic, isolated by the roots
+// of a cubic and a linear factor (within_distance.h:119-272, compute_distance.h:127-280).  The
+// arithmetic is double; next to the reference's, divisions by one number are products with
+// its reciprocal, polynomials are evaluated by Horner's rule with fused multiply-adds and the
+// trigonometric roots come from one sine and cosine: roundings of the last bit or two, in
+// interval ends and iterates that are then stored as floats.  (A point's coverage by its 2,048
+// strokes took half of the edge kernel: 17 double divisions, three cosines, a power and 45
+// double operations a Newton step for each.)
 struct Quintic {
-    double A, B, C, D, E, F;
+    double A, B, C, D, E, F;  // leading coefficient, and the others divided by it
 };
 DVG_DEV Quintic cubic_quintic(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
     V2 a = -p0 + 3 * p1 - 3 * p2 + p3;
@@ -231,36 +263,84 @@ DVG_DEV Quintic cubic_quintic(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
     V2 d = p0 - pt;
     Quintic q;
     q.A = 3 * vsum(a * a);
-    q.B = 5 * vsum(a * b);
-    q.C = 4 * vsum(a * c) + 2 * vsum(b * b);
-    q.D = 3 * (vsum(b * c) + vsum(a * d));
-    q.E = vsum(c * c) + 2 * vsum(d * b);
-    q.F = vsum(d * c);
-    q.B /= q.A;
-    q.C /= q.A;
-    q.D /= q.A;
-    q.E /= q.A;
-    q.F /= q.A;
+    const double inv = 1.0 / q.A;
+    q.B = (double)(5 * vsum(a * b)) * inv;
+    q.C = (double)(4 * vsum(a * c) + 2 * vsum(b * b)) * inv;
+    q.D = (double)(3 * (vsum(b * c) + vsum(a * d))) * inv;
+    q.E = (double)(vsum(c * c) + 2 * vsum(d * b)) * inv;
+    q.F = (double)vsum(d * c) * inv;
     return q;
 }
 DVG_DEV double quintic_eval(const Quintic &q, double t) {
-    return t * t * t * t * t + q.B * t * t * t * t + q.C * t * t * t + q.D * t * t + q.E * t + q.F;
+    return __builtin_fma(__builtin_fma(__builtin_fma(__builtin_fma(t + q.B, t, q.C), t, q.D), t, q.E), t, q.F);
 }
 DVG_DEV double quintic_deriv(const Quintic &q, double t) {
-    return 5 * t * t * t * t + 4 * q.B * t * t * t + 3 * q.C * t * t + 2 * q.D * t + q.E;
+    return __builtin_fma(__builtin_fma(__builtin_fma(__builtin_fma(5.0, t, 4 * q.B), t, 3 * q.C), t, 2 * q.D), t, q.E);
+}
+// sin and cos of x in [0, pi / 3] by their Taylor series (to x^21 and x^20; the next terms are
+// below 1e-20)
+DVG_DEV void sincos_third(double x, double &s, double &c) {
+    const double z = x * x;
+    double p = 1.0 / 51090942171709440000.0, r = 1.0 / 2432902008176640000.0;
+    p = __builtin_fma(p, z, -1.0 / 121645100408832000.0);
+    r = __builtin_fma(r, z, -1.0 / 6402373705728000.0);
+    p = __builtin_fma(p, z, 1.0 / 355687428096000.0);
+    r = __builtin_fma(r, z, 1.0 / 20922789888000.0);
+    p = __builtin_fma(p, z, -1.0 / 1307674368000.0);
+    r = __builtin_fma(r, z, -1.0 / 87178291200.0);
+    p = __builtin_fma(p, z, 1.0 / 6227020800.0);
+    r = __builtin_fma(r, z, 1.0 / 479001600.0);
+    p = __builtin_fma(p, z, -1.0 / 39916800.0);
+    r = __builtin_fma(r, z, -1.0 / 3628800.0);
+    p = __builtin_fma(p, z, 1.0 / 362880.0);
+    r = __builtin_fma(r, z, 1.0 / 40320.0);
+    p = __builtin_fma(p, z, -1.0 / 5040.0);
+    r = __builtin_fma(r, z, -1.0 / 720.0);
+    p = __builtin_fma(p, z, 1.0 / 120.0);
+    r = __builtin_fma(r, z, 1.0 / 24.0);
+    p = __builtin_fma(p, z, -1.0 / 6.0);
+    r = __builtin_fma(r, z, -0.5);
+    s = __builtin_fma(p * z, x, x);
+    c = __builtin_fma(r, z, 1.0);
+}
+// Roots of a t^3 + b t^2 + c t + d as solve_cubic_d returns them (solve.h:29-64).
+DVG_DEV int isolating_cubic(double a, double b, double c, double d, double (&t)[3]) {
+    if (fabs(a) < 1e-6f) return solve_quadratic_d(b, c, d, &t[0], &t[1]) ? 2 : 0;
+    const double inv = 1.0 / a, third = 1.0 / 3.0;
+    b *= inv;
+    c *= inv;
+    d *= inv;
+    const double Q = (b * b - 3 * c) * (1.0 / 9.0);
+    const double R = (2 * b * b * b - 9 * b * c + 27 * d) * (1.0 / 54.0);
+    const double Q3 = Q * Q * Q, b3 = b * third;
+    if (R * R < Q3) {
+        double s, co;
+        sincos_third(acos(R / sqrt(Q3)) * third, s, co);
+        const double h = 0.86602540378443864676 * s, m = -2.0 * __builtin_sqrt(Q);
+        t[0] = m * co - b3;
+        t[1] = m * (-0.5 * co - h) - b3;
+        t[2] = m * (-0.5 * co + h) - b3;
+        return 3;
+    }
+    const double root = cbrt(fabs(R) + __builtin_sqrt(R * R - Q3));
+    const double A = R > 0 ? -root : root;
+    const double B = fabs(A) > 1e-6f ? Q / A : 0.0;
+    t[0] = (A + B) - b3;
+    return 1;
 }
 // Isolating intervals (within_distance.h:195-216); the reference's uninitialised
 // intervals[0] (isolator root outside [0, 1]) is treated as absent.
 // All indices are compile-time constants (slots past n are not read as such), so the array
 // stays in registers.
 DVG_DEV int quintic_intervals(const Quintic &q, float (&iv)[4]) {
-    double p1A = ((2 / 5.f) * q.C - (4 / 25.f) * q.B * q.B);
-    double p1B = ((3 / 5.f) * q.D - (3 / 25.f) * q.B * q.C);
-    double p1C = ((4 / 5.f) * q.E - (2 / 25.f) * q.B * q.D);
-    double p1D = q.F - q.B * q.E / 25.f;
-    double q_root = -q.B / 5.f;
+    // the reference's float fractions
+    const double p1A = (2 / 5.f) * q.C - (4 / 25.f) * q.B * q.B;
+    const double p1B = (3 / 5.f) * q.D - (3 / 25.f) * q.B * q.C;
+    const double p1C = (4 / 5.f) * q.E - (2 / 25.f) * q.B * q.D;
+    const double p1D = q.F - q.B * q.E * (1.0 / 25.0);
+    const double q_root = q.B * -0.2;
     double pr[3] = {0.0, 0.0, 0.0};
-    int num_sol = solve_cubic_d(p1A, p1B, p1C, p1D, pr);
+    const int num_sol = isolating_cubic(p1A, p1B, p1C, p1D, pr);
     const bool first = q_root >= 0 && q_root <= 1;
     const int n = num_sol + (first ? 1 : 0);
     iv[0] = first ? (float)q_root : (float)pr[0];
@@ -281,20 +361,65 @@ DVG_DEV int quintic_intervals(const Quintic &q, float (&iv)[4]) {
     }
     return n;
 }
+// Newton's iteration kept in its bracket (within_distance.h:232-262)
 DVG_DEV float quintic_root(const Quintic &q, float lb, float ub) {
     float t = 0.5f * (lb + ub);
+#pragma nounroll
     for (int it = 0; it < 20; it++) {
         if (!(t >= lb && t <= ub)) t = 0.5f * (lb + ub);
-        double value = quintic_eval(q, t);
+        const double td = t;
+        const double value = quintic_eval(q, td);
         if (fabs(value) < 1e-5f || it == 19) break;
         if (value > 0.f)
             ub = t;
         else
             lb = t;
-        double derivative = quintic_deriv(q, t);
-        t = (float)((double)t - value / derivative);
+        const double deriv = quintic_deriv(q, td);
+        double r = __builtin_amdgcn_rcp(deriv);
+        r = __builtin_fma(__builtin_fma(-deriv, r, 1.0), r, r);
+        r = __builtin_fma(__builtin_fma(-deriv, r, 1.0), r, r);
+        t = (float)__builtin_fma(-value, r, td);
     }
     return t;
+}
+// Calls visit(t) for the root in each interval with a sign change, in order, until it
+// returns true.  The brackets are found first, so that the lanes of a wave run their first
+// searches together, then their second ones, whichever intervals those are.
+template <class Visit>
+DVG_DEV void quintic_search(const Quintic &q, const Visit &visit) {
+    float iv[4];
+    const int n = quintic_intervals(q, iv);
+    float lo[5], hi[5];
+    unsigned found = 0;
+    float lower = 0.f;
+    double at_lower = quintic_eval(q, 0.0);
+    bool more = true;
+#pragma unroll
+    for (int j = 0; j < 5; j++) {
+        const bool inner = j < 4 && j < n;
+        const float end = j < 4 ? iv[j < 4 ? j : 3] : 1.f;
+        const bool use = more && j <= n && !(inner && end < 0.f);
+        const float upper = inner ? fmin_r(end, 1.f) : 1.f;
+        const double at_upper = quintic_eval(q, upper);
+        const bool change = use && !(at_lower * at_upper > 0);
+        const bool falls = at_lower > at_upper;
+        lo[j] = falls ? upper : lower;
+        hi[j] = falls ? lower : upper;
+        if (change) {
+            found |= 1u << j;
+            more = !(upper >= 1.f);
+            lower = upper;
+            at_lower = at_upper;
+        }
+    }
+#pragma nounroll
+    while (found) {
+        const int j = __ffs(found) - 1;
+        found &= found - 1;
+        const float lb = j < 2 ? (j == 0 ? lo[0] : lo[1]) : (j == 2 ? lo[2] : (j == 3 ? lo[3] : lo[4]));
+        const float ub = j < 2 ? (j == 0 ? hi[0] : hi[1]) : (j == 2 ? hi[2] : (j == 3 ? hi[3] : hi[4]));
+        if (visit(quintic_root(q, lb, ub))) break;
+    }
 }
 
 // Every point of cubic segment `seg` is certainly farther than r from pt (the chords of an
@@ -306,33 +431,16 @@ DVG_DEV bool cubic_farther_than(const DevScene &S, int seg, V2 pt, float r) {
 
 // Whether one of the stationary points of the distance to a cubic that the quintic search
 // finds lies within the stroke's radius there (within_distance.h:119-272 past its end tests).
-DVG_DEV bool cubic_stroke_search(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2, float r3) {
-    Quintic q = cubic_quintic(p0, p1, p2, p3, pt);
-    float iv[4];
-    int niv = quintic_intervals(q, iv);
-    const float e0 = iv[0], e1 = iv[1], e2 = iv[2], e3 = iv[3];
-    float lower = 0.f;
-#pragma nounroll
-    for (int j = 0; j < niv + 1; j++) {
-        const float end = j < 2 ? (j == 0 ? e0 : e1) : (j == 2 ? e2 : e3);
-        if (j < niv && end < 0.f) continue;
-        float upper = j < niv ? fmin_r(end, 1.f) : 1.f;
-        float lb = lower, ub = upper;
-        double lbe = quintic_eval(q, lb), ube = quintic_eval(q, ub);
-        if (lbe * ube > 0) continue;
-        if (lbe > ube) {
-            float tmp = lb;
-            lb = ub;
-            ub = tmp;
-        }
-        float t = quintic_root(q, lb, ub);
+static __device__ __noinline__ bool cubic_stroke_search(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2,
+                                                        float r3) {
+    bool hit = false;
+    quintic_search(cubic_quintic(p0, p1, p2, p3, pt), [&](float t) {
         float tt = 1 - t;
         float rr = (tt * tt * tt) * r0 + (3 * tt * tt * t) * r1 + (3 * tt * t * t) * r2 + (t * t * t) * r3;
-        if (dist_sq(ceval(p0, p1, p2, p3, t), pt) < rr * rr) return true;
-        if (upper >= 1.f) break;
-        lower = upper;
-    }
-    return false;
+        hit = dist_sq(ceval(p0, p1, p2, p3, t), pt) < rr * rr;
+        return hit;
+    });
+    return hit;
 }
 
 // Stroke test of a line and of a quadratic segment (within_distance.h:32-118), radius r0, r1
@@ -344,7 +452,7 @@ DVG_DEV bool line_within(V2 p0, V2 p1, V2 pt, float r0, float r1) {
     float rr = r0 + t * (r1 - r0);
     return dist_sq(p0 + t * (p1 - p0), pt) < rr * rr;
 }
-DVG_DEV bool quad_within(V2 p0, V2 p1, V2 p2, V2 pt, float r0, float r1, float r2) {
+static __device__ __noinline__ bool quad_within(V2 p0, V2 p1, V2 p2, V2 pt, float r0, float r1, float r2) {
     if (dist_sq(qeval(p0, p1, p2, 0), pt) < r0 * r0) return true;
     if (dist_sq(qeval(p0, p1, p2, 1), pt) < r2 * r2) return true;
     float A = vsum((p0 - 2 * p1 + p2) * (p0 - 2 * p1 + p2));
@@ -514,52 +622,22 @@ DVG_DEV float segment_closest_lq(const DevScene &S, int s, int seg, V2 pt, V2 &c
 }
 
 // Closest point on one cubic path segment (compute_distance.h:127-280)
-DVG_DEV float cubic_closest(const DevScene &S, int seg, V2 pt, V2 &cp, float &t_root) {
-    V2 p[4];
-    int4 idx;
-    seg_load(S, seg, p, idx);
-    float dd;
-    V2 p0 = p[0], p1 = p[1], p2 = p[2], p3 = p[3];
+struct CubicClosest {
+    float dist, t;
+    V2 pt;
+};
+static __device__ __noinline__ CubicClosest cubic_closest(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
     V2 pt0 = ceval(p0, p1, p2, p3, 0), pt1 = ceval(p0, p1, p2, p3, 1);
     float d0 = dist(pt0, pt), d1 = dist(pt1, pt);
-    dd = d0;
-    cp = pt0;
-    t_root = 0;
-    if (d1 < dd) {
-        dd = d1;
-        cp = pt1;
-        t_root = 1;
-    }
-    Quintic q = cubic_quintic(p0, p1, p2, p3, pt);
-    float iv[4];
-    int niv = quintic_intervals(q, iv);
-    const float e0 = iv[0], e1 = iv[1], e2 = iv[2], e3 = iv[3];
-    float lower = 0.f;
-#pragma nounroll
-    for (int j = 0; j < niv + 1; j++) {
-        const float end = j < 2 ? (j == 0 ? e0 : e1) : (j == 2 ? e2 : e3);
-        if (j < niv && end < 0.f) continue;
-        float upper = j < niv ? fmin_r(end, 1.f) : 1.f;
-        float lb = lower, ub = upper;
-        double lbe = quintic_eval(q, lb), ube = quintic_eval(q, ub);
-        if (lbe * ube > 0) continue;
-        if (lbe > ube) {
-            float tmp = lb;
-            lb = ub;
-            ub = tmp;
-        }
-        float t = quintic_root(q, lb, ub);
+    CubicClosest r{d0, 0.f, pt0};
+    if (d1 < r.dist) r = CubicClosest{d1, 1.f, pt1};
+    quintic_search(cubic_quintic(p0, p1, p2, p3, pt), [&](float t) {
         V2 pp = ceval(p0, p1, p2, p3, t);
         float dp = dist(pp, pt);
-        if (dp < dd) {
-            dd = dp;
-            cp = pp;
-            t_root = t;
-        }
-        if (upper >= 1.f) break;
-        lower = upper;
-    }
-    return dd;
+        if (dp < r.dist) r = CubicClosest{dp, t, pp};
+        return false;
+    });
+    return r;
 }
 
 // closest_point for a path (compute_distance.h:27-300): the segments in the reference's
@@ -580,7 +658,11 @@ DVG_DEV bool closest_point_path(const DevScene &S, int s, V2 pt, float max_radiu
         float dd;
         if (S.seg_kind[seg] == 2) {
             if (cubic_farther_than(S, seg, pt, min_dist)) continue;
-            dd = cubic_closest(S, seg, pt, cp, tr);
+            const CubicPoints c = cubic_points_of(S, seg);
+            const CubicClosest r = cubic_closest(c.p0, c.p1, c.p2, c.p3, pt);
+            dd = r.dist;
+            cp = r.pt;
+            tr = r.t;
         } else {
             dd = segment_closest_lq(S, s, seg, pt, cp, tr);
         }

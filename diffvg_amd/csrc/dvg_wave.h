@@ -64,19 +64,6 @@ struct SceneRef {
 // of a kernel whose first argument is the DevScene
 DVG_DEV SceneRef scene_argument() { return SceneRef{(uint64_t)__builtin_amdgcn_kernarg_segment_ptr()}; }
 
-// The double-precision searches of the exact stage, called, not inlined: their constants and
-// intermediates then stay out of the register allocation of the loops around them.
-static __device__ __noinline__ bool wave_stroke_search(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2,
-                                                       float r3) {
-    return cubic_stroke_search(p0, p1, p2, p3, pt, r0, r1, r2, r3);
-}
-static __device__ __noinline__ int wave_winding_solve(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
-    return cubic_winding_solve(p0, p1, p2, p3, pt);
-}
-
-static __device__ __noinline__ bool wave_quad_within(V2 p0, V2 p1, V2 p2, V2 pt, float r0, float r1, float r2) {
-    return quad_within(p0, p1, p2, pt, r0, r1, r2);
-}
 // segment_within_lq for paths without the approximate quadratic distance
 DVG_DEV bool wave_within_lq(const DevScene &S, int s, int seg, int k, V2 pt, float r) {
     V2 p[4];
@@ -89,7 +76,7 @@ DVG_DEV bool wave_within_lq(const DevScene &S, int s, int seg, int k, V2 pt, flo
         if (k == 1) r2 = S.thickness[idx.z];
     }
     if (k == 0) return line_within(p[0], p[1], pt, r0, r1);
-    return wave_quad_within(p[0], p[1], p[2], pt, r0, r1, r2);
+    return quad_within(p[0], p[1], p[2], pt, r0, r1, r2);
 }
 
 // Orders the wave's LDS accesses (a wave's LDS instructions execute in order; this keeps the
@@ -143,7 +130,7 @@ DVG_DEV void wave_exact(const SceneRef &R, WaveLds<SIDES> &W, int &n2, int cnt) 
                         r3 = S.thickness[idx.w];
                     }
                     hit = dist_sq(c.p0, p) < r0 * r0 || dist_sq(c.p3, p) < r3 * r3;
-                    if (!hit) hit = wave_stroke_search(c.p0, c.p1, c.p2, c.p3, p, r0, r1, r2, r3);
+                    if (!hit) hit = cubic_stroke_search(c.p0, c.p1, c.p2, c.p3, p, r0, r1, r2, r3);
                 } else {
                     hit = wave_within_lq(S, s, seg, k, p, r);
                 }
@@ -154,7 +141,7 @@ DVG_DEV void wave_exact(const SceneRef &R, WaveLds<SIDES> &W, int &n2, int cnt) 
             if (k == 2) {
                 if (!wf::cubic_winding_test<true>(cubic_prep_of(S, seg), p.x, p.y, w)) {
                     const CubicPoints c = cubic_points_of(S, seg);
-                    w = wave_winding_solve(c.p0, c.p1, c.p2, c.p3, p);
+                    w = cubic_winding_solve(c.p0, c.p1, c.p2, c.p3, p);
                 }
             } else {
                 V2 q[4];
