@@ -50,7 +50,7 @@ constexpr int kPFragSlots = 8;
 constexpr int kPFragWords = 9;
 // Boundary adjoints of circles, ellipses and rects (three or four parameters each) are
 // combined across a wave's lanes, up to this many samples per shape of the scene: 40 shapes
-// at 333x217, 3x2 samples: k_edge 3.34 -> 0.49 ms.  Past it every lane adds its own, as
+// at 333x217, 3x2 samples: k_edge 3.34 -> 0.24 ms.  Past it every lane adds its own, as
 // before (~12 ns per sample: 10 ms for one circle and 262,144 samples, 0.9 combined),
 // because there the two forms differ by more than float rounding of one sum: adding N terms
 // of one sign one by one loses up to 2.3e-5 of the sum at 9,000 samples, 5e-5 at 32,000,
@@ -146,6 +146,10 @@ struct ColorBwdLds {
 struct EdgeLds {
     CandLds c;
     int perm[kBlock];
+};
+union EdgeWaveLds {
+    WaveLds<2> shade;
+    ScatterLds scatter;
 };
 struct SdfLds {
     CandLds c;
@@ -902,9 +906,10 @@ __global__ __launch_bounds__(kBlock) void k_edge_bin(int count, const int *edge_
 
 // Adjoint of a wave's boundary samples (render_edge_kernel, diffvg.cpp:1430-1475) from the
 // colours and edge hits of their two sides; every lane calls it, lanes without a sample pass
-// on = false.
+// on = false.  `lds`: the wave's scatter table, or null to combine in registers.
 DVG_DEV void edge_scatter(const DevScene &S, const Geom &G, bool on, const EdgeSample &es, bool in_hit, bool out_hit,
-                          V4 cin, V4 cout, const float *weight, const float *d_img, float *d_translation) {
+                          V4 cin, V4 cout, const float *weight, const float *d_img, float *d_translation,
+                          ScatterLds *lds) {
     V2 n{es.nx, es.ny};
     int bx = (int)(es.px * G.W), by = (int)(es.py * G.H);
     // every lane stays to the end: the gradient scatter combines lanes of a wave
@@ -923,8 +928,13 @@ DVG_DEV void edge_scatter(const DevScene &S, const Geom &G, bool on, const EdgeS
         contrib = dot(cin - cout, d_color) / es.pdf;
     }
     BoundaryData bd = active ? es.data : BoundaryData{0, 0, 0.f, 0};
-    accumulate_boundary_gradient_wave(S, active, active ? es.group : 0, active ? es.shape : 0, contrib,
-                                      active ? es.t : 0.f, n, bd, active ? V2{es.lx, es.ly} : V2{0, 0}, G.prim_direct != 0);
+    const int g = active ? es.group : 0, s = active ? es.shape : 0;
+    const float t = active ? es.t : 0.f;
+    const V2 lp = active ? V2{es.lx, es.ly} : V2{0, 0};
+    if (lds)
+        accumulate_boundary_gradient_lds(S, *lds, active, g, s, contrib, t, n, bd, lp, G.prim_direct != 0);
+    else
+        accumulate_boundary_gradient_wave(S, active, g, s, contrib, t, n, bd, lp, G.prim_direct != 0);
     if (active && d_translation) {
         aadd(d_translation + 2 * (by * G.W + bx) + 0, n.x * contrib);
         aadd(d_translation + 2 * (by * G.W + bx) + 1, n.y * contrib);
@@ -949,7 +959,7 @@ DVG_DEV int find_tile(const int *chunk_off, int ntiles, int chunk) {
     }
     return lo;
 }
-DVG_DEV void edge_chunk_wave(WaveLds<2> &L, const SceneRef &R, const Geom &G, int chunk, const EdgeSample *edges,
+DVG_DEV void edge_chunk_wave(EdgeWaveLds &L, const SceneRef &R, const Geom &G, int chunk, const EdgeSample *edges,
                              const int *tile_off, const int *tile_count, const int *chunk_off, int ntiles,
                              const int *sorted, const float *bg, const float *weight, const float *d_img,
                              float *d_translation) {
@@ -981,7 +991,7 @@ DVG_DEV void edge_chunk_wave(WaveLds<2> &L, const SceneRef &R, const Geom &G, in
         ci.init(has_bg, bg0);
         co.init(has_bg, bg0);
     }
-    wave_shade<2>(R, L, valid, pin, pout, pmid, 1.01e-4f * cw, 1.01e-4f * ch,
+    wave_shade<2>(R, L.shade, valid, pin, pout, pmid, 1.01e-4f * cw, 1.01e-4f * ch,
                   [&](const DevScene &S, int g, bool stroke, bool on_in, bool on_out) {
                       const int type = stroke ? S.stroke_type[g] : S.fill_type[g];
                       const int off = stroke ? S.stroke_off[g] : S.fill_off[g];
@@ -999,8 +1009,9 @@ DVG_DEV void edge_chunk_wave(WaveLds<2> &L, const SceneRef &R, const Geom &G, in
         cin = ci.result(has_bg, bgc);
         cout = co.result(has_bg, bgc);
     }
+    // the shading tables of the wave are done with
     edge_scatter(S, G, valid, es, valid && ci.edge_hit(false), valid && co.edge_hit(false), cin, cout, weight, d_img,
-                 d_translation);
+                 d_translation, &L.scatter);
 }
 
 // One workgroup per chunk of up to G.echunk boundary samples of one tile (the grid is an
@@ -1137,7 +1148,8 @@ DVG_DEV void edge_chunk(EdgeLds &L, const DevScene &S, const Geom &G, int chunk,
                 cout = co.result(has_bg, bgc);
             }
         }
-        edge_scatter(S, G, valid && side == 0, es, in_hit, out_hit, cin, cout, weight, d_img, d_translation);
+        edge_scatter(S, G, valid && side == 0, es, in_hit, out_hit, cin, cout, weight, d_img, d_translation,
+                     (ScatterLds *)nullptr);
     }
 }
 template <bool BOTH>
@@ -1153,7 +1165,7 @@ __global__ __launch_bounds__(kBlock, BOTH ? DVG_WAVES_EDGE_BOTH : DVG_WAVES_EDGE
 __global__ __launch_bounds__(64, DVG_WAVES_EDGE_WAVE) void k_edge_wave(
     DevScene S, Geom G, const EdgeSample *edges, const int *tile_off, const int *tile_count, const int *chunk_off,
     int ntiles, const int *sorted, const float *bg, const float *weight, const float *d_img, float *d_translation) {
-    __shared__ WaveLds<2> L;
+    __shared__ EdgeWaveLds L;
     edge_chunk_wave(L, scene_argument(), G, blockIdx.x, edges, tile_off, tile_count, chunk_off, ntiles, sorted, bg,
                     weight, d_img, d_translation);
 }
@@ -2269,7 +2281,7 @@ __global__ __launch_bounds__(64, DVG_WAVES_EDGE_WAVE) void kb_edge_wave(const Jo
     int j = find_job(pref, nj, blockIdx.x);
     const Job J = load_job(jobs + j);
     if (!J.d_img) return;
-    __shared__ WaveLds<2> L;
+    __shared__ EdgeWaveLds L;
     edge_chunk_wave(L, SceneRef{(uint64_t)&jobs[j].S}, J.G, blockIdx.x - pref[j], J.edges, J.tile_off, J.tile_count,
                     J.chunk_off, J.ntiles, J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr);
 }

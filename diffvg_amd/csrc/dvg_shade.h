@@ -769,6 +769,141 @@ DVG_DEV void accumulate_boundary_gradient_wave(const DevScene &S, bool active, i
     }
 }
 
+// accumulate_boundary_gradient_wave with the sums of a wave's samples gathered in LDS: lanes
+// of one (group, shape, segment) take a row of a table, each value is one LDS atomic
+// instruction whatever the number of rows, and the rows then leave as atomics 64 at a time.
+// The register form reduces 18 values across the wave once per distinct row, ~20 rows of 64
+// samples: k_edge of 2048 strokes at 512x512, 4 samples, 1.48 -> 1.30 ms; 300 paths 0.88 -> 0.79.
+constexpr int kScatterVals = 18;  // stroke width, up to 4 points or parameters (8), transform (9)
+struct ScatterLds {
+    float row[64][kScatterVals];
+    int group[64], shape[64], seg[64];
+};
+DVG_DEV void accumulate_boundary_gradient_lds(const DevScene &S, ScatterLds &L, bool active, int g, int s,
+                                              float contrib, float t, V2 normal, const BoundaryData &bd, V2 local_pt,
+                                              bool prim_direct) {
+    const int lane = threadIdx.x & 63;
+    const int type = active ? S.shape_type[s] : -1;
+    const bool path = type == 2;
+    const int seg = path ? S.seg_begin[s] + bd.base_point_id : -1;
+    // rows
+    int mine = -1, rows = 0;
+    for (uint64_t pending = __ballot(active); pending;) {
+        const int leader = __ffsll((unsigned long long)pending) - 1;
+        const int lg = __builtin_amdgcn_readlane(g, leader), ls = __builtin_amdgcn_readlane(s, leader),
+                  lseg = __builtin_amdgcn_readlane(seg, leader);
+        const bool same = active && g == lg && s == ls && seg == lseg;
+        const uint64_t m = __ballot(same);
+        if (same) mine = rows;
+        pending &= ~m;
+        rows++;
+    }
+    wave_sync();
+    for (int i = lane; i < rows * kScatterVals; i += 64) (&L.row[0][0])[i] = 0.f;
+    if (active) {  // lanes of one row write the same values
+        L.group[mine] = g;
+        L.shape[mine] = s;
+        L.seg[mine] = seg;
+    }
+    wave_sync();
+    if (active) {
+        float *row = L.row[mine];
+        auto add = [&](int i, float v) {
+            __hip_atomic_fetch_add(row + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+        };
+        if (bd.is_stroke && !(path && S.has_thick[s])) add(0, contrib);
+        if (path) {
+            const int k = S.seg_kind[seg];
+            const float tt = bd.t, o = 1 - tt;
+            float w[4] = {0.f, 0.f, 0.f, 0.f};
+            if (k == 0) {
+                w[0] = 1 - tt;
+                w[1] = tt;
+            } else if (k == 1) {
+                w[0] = (1 - tt) * (1 - tt);
+                w[1] = 2 * (1 - tt) * tt;
+                w[2] = tt * tt;
+            } else {
+                w[0] = o * o * o;
+                w[1] = 3 * (o * o) * tt;
+                w[2] = 3 * (1 - tt) * tt * tt;
+                w[3] = tt * tt * tt;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (j > k + 1) break;
+                add(1 + 2 * j, w[j] * normal.x * contrib);
+                add(2 + 2 * j, w[j] * normal.y * contrib);
+            }
+            if (bd.is_stroke && S.has_thick[s]) {  // per-point thickness (rare)
+                const int4 idx = S.seg_idx[seg];
+                const int ii[4] = {idx.x, idx.y, idx.z, idx.w};
+#pragma unroll
+                for (int j = 0; j < 4; j++)
+                    if (j <= k + 1) aadd(S.d_thickness + ii[j], w[j] * contrib);
+            }
+        } else {
+            float v[4] = {0.f, 0.f, 0.f, 0.f};
+            int n = 4;
+            if (type == 0) {
+                v[0] = contrib;
+                v[1] = normal.x * contrib;
+                v[2] = normal.y * contrib;
+                n = 3;
+            } else if (type == 1) {
+                const float tp = 2 * (float)kPi;
+                v[0] = (float)(cos((double)(tp * t)) * normal.x * contrib);
+                v[1] = (float)(sin((double)(tp * t)) * normal.y * contrib);
+                v[2] = normal.x * contrib;
+                v[3] = normal.y * contrib;
+            } else if (normal == V2{-1, 0}) {
+                v[0] = -contrib;
+            } else if (normal == V2{1, 0}) {
+                v[2] = contrib;
+            } else if (normal == V2{0, -1}) {
+                v[1] = -contrib;
+            } else if (normal == V2{0, 1}) {
+                v[3] = contrib;
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if (j >= n) break;
+                if (prim_direct)  // see kPrimDirect
+                    aadd(S.d_params + S.param_off[s] + j, v[j]);
+                else
+                    add(1 + j, v[j]);
+            }
+        }
+        const M3 s2c = m3_load(S.s2c + 9 * g);
+        M3 d_s2c;
+#pragma unroll
+        for (int i = 0; i < 9; i++) d_s2c.m[i] = 0.f;
+        V2 d_local{0, 0};
+        d_xform_pt(s2c, local_pt, normal * contrib, d_s2c, d_local);
+#pragma unroll
+        for (int i = 0; i < 9; i++) add(9 + i, d_s2c.m[i]);
+    }
+    wave_sync();
+    const int copy = grad_copy(S);
+    for (int i = lane; i < rows * kScatterVals; i += 64) {
+        const float v = (&L.row[0][0])[i];
+        if (v == 0.f) continue;  // also the values a row does not have
+        const int r = i / kScatterVals, c = i - r * kScatterVals, rs = L.shape[r], rseg = L.seg[r];
+        float *dst;
+        if (c == 0) {
+            dst = S.d_stroke_width + rs;
+        } else if (c >= 9) {
+            dst = S.d_xform + 9 * L.group[r] + (c - 9);
+        } else if (rseg >= 0) {
+            const int j = (c - 1) >> 1;
+            dst = S.d_points + 2 * reinterpret_cast<const int *>(S.seg_idx + rseg)[j] + ((c - 1) & 1);
+        } else {
+            dst = S.d_params + S.param_off[rs] + (c - 1);
+        }
+        aadd(dst + copy, v);
+    }
+}
+
 // d_sample_paint for a whole wave (every lane calls it; lanes without a paint adjoint pass
 // on = false): lanes that add to the same stops or the same gradient end points add their
 // values together before the atomics.  A drawing's gradient fill covers thousands of samples
