@@ -826,28 +826,65 @@ __global__ __launch_bounds__(kBlock, PRE ? DVG_WAVES_COLOR_BWD_PRE : DVG_WAVES_C
     color_bwd_tile<PRE>(L, S, G, blockIdx.x, bg, weight, d_img, d_bg, d_translation, err, frag, pkeep);
 }
 
-// One boundary sample and its tile; the count the atomic returns is the sample's position
-// in the tile's bin, so binning (edge_bin_one) needs no second round of atomics.
-DVG_DEV void edge_sample_one(const DevScene &S, const Geom &G, int idx, int count, EdgeSample *edges,
-                             int *edge_tile, int *edge_rank, int *tile_count) {
+// One boundary sample and its tile (-1: none).
+DVG_DEV int edge_sample_tile(const DevScene &S, const Geom &G, int idx, EdgeSample &es) {
+    if (S.num_total_shapes > 0 && make_edge_sample(S, idx, G.seed, es)) {
+        const int bx = (int)(es.px * G.W), by = (int)(es.py * G.H);
+        if (bx >= 0 && bx < G.W && by >= 0 && by < G.H) return (by / G.th) * G.tiles_x + (bx / G.tw);
+    }
+    return -1;
+}
+// The count the atomic returns is the sample's position in the tile's bin, so binning
+// (edge_bin_one) needs no second round of atomics.
+DVG_DEV void edge_sample_one(const DevScene &S, const Geom &G, int idx, int count, EdgeSample *edges, int *edge_tile,
+                             int *edge_rank, int *tile_count) {
     if (idx >= count) return;
     EdgeSample es{};
-    int tile = -1, rank = 0;
-    if (S.num_total_shapes > 0 && make_edge_sample(S, idx, G.seed, es)) {
-        int bx = (int)(es.px * G.W), by = (int)(es.py * G.H);
-        if (bx >= 0 && bx < G.W && by >= 0 && by < G.H) {
-            tile = (by / G.th) * G.tiles_x + (bx / G.tw);
-            rank = atomicAdd(tile_count + tile, 1);
-        }
-    }
+    const int tile = edge_sample_tile(S, G, idx, es);
     edges[idx] = es;
     edge_tile[idx] = tile;
-    edge_rank[idx] = rank;
+    edge_rank[idx] = tile >= 0 ? atomicAdd(&tile_count[tile], 1) : 0;
 }
-__global__ __launch_bounds__(kBlock) void k_edge_sample(DevScene S, Geom G, int count, EdgeSample *edges,
-                                                        int *edge_tile, int *edge_rank, int *tile_count) {
+// The same for a workgroup of kSampleBlock samples, counted per tile in LDS first and added to
+// a tile's count at once: a scene of few shapes sends its samples to the few tiles on their
+// boundaries, whose counters would take one atomic per sample (12.7 ns each).  2048 strokes
+// at 512x512, 4 samples: 143 -> 97 us; 24 scenes of one batch 2.8 -> 1.5 ms.  Canvases of
+// more tiles than the table holds (48 KB: two workgroups of 16 waves fill a CU) add per sample.
+constexpr int kSampleBlock = 1024;
+constexpr int kSampleTiles = 12288;
+DVG_DEV void edge_sample_block(int *s_count, const DevScene &S, const Geom &G, int block, int count, EdgeSample *edges,
+                               int *edge_tile, int *edge_rank, int *tile_count) {
+    const int ntiles = G.tiles_x * G.tiles_y;
+    const bool local = ntiles <= kSampleTiles;
+    const int idx = block * kSampleBlock + threadIdx.x;
+    if (local) {
+        for (int t = threadIdx.x; t < ntiles; t += kSampleBlock) s_count[t] = 0;
+        __syncthreads();
+    }
+    int tile = -1, rank = 0;
+    if (idx < count) {
+        EdgeSample es{};
+        tile = edge_sample_tile(S, G, idx, es);
+        edges[idx] = es;
+        if (tile >= 0) rank = local ? atomicAdd(s_count + tile, 1) : atomicAdd(tile_count + tile, 1);
+    }
+    if (local) {
+        __syncthreads();
+        for (int t = threadIdx.x; t < ntiles; t += kSampleBlock)
+            if (const int n = s_count[t]) s_count[t] = atomicAdd(tile_count + t, n);
+        __syncthreads();
+        if (tile >= 0) rank += s_count[tile];
+    }
+    if (idx < count) {
+        edge_tile[idx] = tile;
+        edge_rank[idx] = rank;
+    }
+}
+__global__ __launch_bounds__(kSampleBlock) void k_edge_sample(DevScene S, Geom G, int count, EdgeSample *edges,
+                                                              int *edge_tile, int *edge_rank, int *tile_count) {
     mark(S);
-    edge_sample_one(S, G, blockIdx.x * blockDim.x + threadIdx.x, count, edges, edge_tile, edge_rank, tile_count);
+    __shared__ int s_count[kSampleTiles];
+    edge_sample_block(s_count, S, G, blockIdx.x, count, edges, edge_tile, edge_rank, tile_count);
 }
 
 // Exclusive scans, in one workgroup, of the per-tile boundary-sample counts (-> tile
@@ -1905,7 +1942,7 @@ int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
                 DVG_CHECK(hipMemsetAsync(ws.tile_count, 0, sizeof(int) * ntiles, st));
                 {
                     DVG_PROF(st, "k_edge_sample");
-                    k_edge_sample<<<(unsigned)((nsamp + kBlock - 1) / kBlock), kBlock, 0, st>>>(
+                    k_edge_sample<<<(unsigned)((nsamp + kSampleBlock - 1) / kSampleBlock), kSampleBlock, 0, st>>>(
                         S, G, (int)nsamp, ws.edges, ws.edge_tile, ws.edge_rank, ws.tile_count);
                 }
                 {
@@ -2150,7 +2187,7 @@ struct Job {
 // kStChunk / kStChunk2: edge chunks of the jobs with one side / both sides per lane;
 // kStChunkW: of the jobs with wave-cooperative tests; kStTileF / kStTileW: tiles of the
 // colour forward of the others / of those
-enum { kStPix = 0, kStTile, kStSamp, kStChunk, kStSdf, kStZero, kStChunk2, kStChunkW, kStTileF, kStTileW, kNumStages };
+enum { kStPix = 0, kStTile, kStSamp, kStChunk, kStSdf, kStZero, kStChunk2, kStChunkW, kStTileF, kStTileW, kStEdgeSamp, kNumStages };
 
 // What the kernels read through a job is constant while they run, except the buffers that
 // one stage hands to the next (written and read by different launches of one stream, so
@@ -2241,12 +2278,13 @@ __global__ __launch_bounds__(kBlock, DVG_WAVES_BATCH_COLOR_BWD) void kb_color_bw
                         PRE ? nullptr : J.frag, PRE ? J.pkeep : nullptr);
 }
 
-__global__ __launch_bounds__(kBlock) void kb_edge_sample(const Job *jobs, const int *pref, int nj) {
+__global__ __launch_bounds__(kSampleBlock) void kb_edge_sample(const Job *jobs, const int *pref, int nj) {
     int j = find_job(pref, nj, blockIdx.x);
     const Job J = load_job(jobs + j);
     if (!J.d_img) return;
-    edge_sample_one(J.S, J.G, (blockIdx.x - pref[j]) * kBlock + threadIdx.x, J.nsamp, J.edges, J.edge_tile,
-                    J.edge_rank, J.tile_count);
+    __shared__ int s_count[kSampleTiles];
+    edge_sample_block(s_count, J.S, J.G, blockIdx.x - pref[j], J.nsamp, J.edges, J.edge_tile, J.edge_rank,
+                      J.tile_count);
 }
 
 __global__ __launch_bounds__(1024) void kb_scan(const Job *jobs, int j0) {
@@ -2643,6 +2681,7 @@ int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, i
             case kStPix: return color ? (J.npix + kBlock - 1) / kBlock : 0;
             case kStTile: return color ? J.ntiles : 0;
             case kStSamp: return edges ? (J.nsamp + kBlock - 1) / kBlock : 0;
+            case kStEdgeSamp: return edges ? (J.nsamp + kSampleBlock - 1) / kSampleBlock : 0;
             case kStTileF: return J.img && (J.pre || !J.S.wave_ok) ? J.ntiles : 0;
             case kStTileW: return J.img && !J.pre && J.S.wave_ok ? kTileWaves * J.ntiles : 0;
             case kStChunkW:
@@ -2844,7 +2883,7 @@ int batch_render(BatchHost &B, hipStream_t st) {
             if (c == 0) {
                 {
                     DVG_PROF(st, "kb_edge_sample");
-                    kb_edge_sample<<<T(kStSamp), kBlock, 0, st>>>(J, P(kStSamp), nj);
+                    kb_edge_sample<<<T(kStEdgeSamp), kSampleBlock, 0, st>>>(J, P(kStEdgeSamp), nj);
                     kb_scan<<<(unsigned)nj, 1024, 0, st>>>(jobs, j0);
                     kb_edge_bin<<<T(kStSamp), kBlock, 0, st>>>(J, P(kStSamp), nj);
                 }

@@ -65,3 +65,14 @@ def test_one_shape_many_samples(w, h, nsx, nsy):
                           stroke_color=torch.tensor([0.9, 0.2, 0.1, 0.8]))
     for pre in (False, True):
         _check([path], [group], w, h, nsx, nsy, pre)
+
+
+@pytest.mark.parametrize('h', [196592, 196608, 196624])
+def test_boundary_samples_of_canvases_around_the_count_table(h):
+    """Boundary samples are counted per tile in LDS up to 12288 tiles, one by one above."""
+    print('tall canvas', h, flush=True)
+    pts = torch.tensor([[0.2, 0.01 * h], [1.8, 0.45 * h], [0.5, 0.97 * h]])
+    path = pd.Path(num_control_points=torch.tensor([0, 0, 0]), points=pts, is_closed=True, stroke_width=torch.tensor(0.1))
+    group = pd.ShapeGroup(shape_ids=torch.tensor([0]), fill_color=torch.tensor([0.3, 0.6, 0.3, 0.7]),
+                          stroke_color=torch.tensor([0.9, 0.2, 0.1, 0.8]))
+    _check([path], [group], 2, h, 1, 1, False)
