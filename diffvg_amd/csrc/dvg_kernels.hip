@@ -40,9 +40,11 @@ constexpr int kCandCap = 2048;
 // per wave); Geom::echunk holds the one a render uses (a tuning knob)
 constexpr int kEdgeChunk = kBlock / 2;
 // fragment lists kept from a colour forward for its backward: up to kFragSlots fragments
-// per sample (a sample with more is shaded again), at most kFragCacheBytes per scene
-constexpr int kFragSlots = 16;
-constexpr size_t kFragCacheBytes = size_t(512) << 20;
+// per sample (a sample with more is shaded again), at most kFragCacheBytes per scene.  24
+// slots instead of 16: one sample of more makes its whole tile wait for the shading; 2048
+// strokes at 512x512 585 -> 316 us, with memory for as many samples as 16 slots had in 512 MiB
+constexpr int kFragSlots = 24;
+constexpr size_t kFragCacheBytes = size_t(768) << 20;
 constexpr int kFragMaxGroups = 32768;  // group ids 2 g + is_stroke are kept in 16 bits
 // prefiltered fragments keep what their adjoint needs besides the paint: group id, closest
 // shape, signed distance, closest point, path position and whether a distance was found
@@ -424,7 +426,7 @@ DVG_DEV void shade_list_record(const DevScene &S, V2 pt, const int *list, int n,
         if (st >= 0 && within_distance_local(S, g, local, nullptr)) {
             V4 c = sample_paint(S, st, S.stroke_off[g], S.stroke_ns[g], pt);
             if (comp.nf < kMaxFrags)
-                frags[comp.nf] = FragRec{V3{c.x, c.y, c.z}, c.w, comp.color, comp.alpha, 2 * g + 1};
+                frags[comp.nf] = FragRec{comp.color, comp.alpha, 2 * g + 1};
             else
                 overflow = 1;
             comp.add(c, g, -1);
@@ -433,7 +435,7 @@ DVG_DEV void shade_list_record(const DevScene &S, V2 pt, const int *list, int n,
         if (ft >= 0 && is_inside_local(S, g, local, nullptr)) {
             V4 c = sample_paint(S, ft, S.fill_off[g], S.fill_ns[g], pt);
             if (comp.nf < kMaxFrags)
-                frags[comp.nf] = FragRec{V3{c.x, c.y, c.z}, c.w, comp.color, comp.alpha, 2 * g};
+                frags[comp.nf] = FragRec{comp.color, comp.alpha, 2 * g};
             else
                 overflow = 1;
             comp.add(c, g, -1);
@@ -469,12 +471,8 @@ DVG_DEV void replay_frags(const DevScene &S, V2 pt, const uint16_t *ids, size_t 
                           Compositor &comp, FragRec *frags) {
     for (int j = 0; j < nf; j++) {
         const int gid = ids[(size_t)j * nsamp + idx];
-        const int g = gid >> 1;
-        const bool stroke = (gid & 1) != 0;
-        V4 c = stroke ? sample_paint(S, S.stroke_type[g], S.stroke_off[g], S.stroke_ns[g], pt)
-                      : sample_paint(S, S.fill_type[g], S.fill_off[g], S.fill_ns[g], pt);
-        frags[comp.nf] = FragRec{V3{c.x, c.y, c.z}, c.w, comp.color, comp.alpha, gid};
-        comp.add(c, g, -1);
+        frags[comp.nf] = FragRec{comp.color, comp.alpha, gid};
+        comp.add(frag_paint(S, gid, pt), gid >> 1, -1);
     }
 }
 
@@ -740,9 +738,10 @@ DVG_DEV void color_bwd_tile(ColorBwdLds &L, const DevScene &S, const Geom &G, in
     V4 d_color{0, 0, 0, 0}, color{0, 0, 0, 0};
     float *d_tr = nullptr;
     if (valid) {
-        d_color = gather_d_color(S.filter_type, S.filter_radius, d_img, weight, G.W, G.H, rpt);
-        d_tr = d_translation ? d_translation + 2 * (y * G.W + x) : nullptr;
         color = comp.result(has_bg, bgc);
+        d_color = gather_and_splat_adjoint(S.filter_type, S.filter_radius, d_img, weight, G.W, G.H, rpt, x, y, color,
+                                           d_radius);
+        d_tr = d_translation ? d_translation + 2 * (y * G.W + x) : nullptr;
     }
     if constexpr (PRE) {
         // all lanes: paint, stroke-width and distance adjoints are combined across the wave
@@ -761,26 +760,6 @@ DVG_DEV void color_bwd_tile(ColorBwdLds &L, const DevScene &S, const Geom &G, in
             kind = comp.nf == 0 ? 0 : 1;
             dbg_val = comp.nf == 0 ? d_color : d_back;
         }
-    }
-    if (valid) {
-        // filter-radius adjoint of the splat (diffvg.cpp:1250-1268)
-        float radius = S.filter_radius;
-        int ri = (int)ceil((double)radius);
-        for (int dy = -ri; dy <= ri; dy++)
-            for (int dx = -ri; dx <= ri; dx++) {
-                int xx = x + dx, yy = y + dy;
-                if (xx >= 0 && xx < G.W && yy >= 0 && yy < G.H) {
-                    float ws = weight[yy * G.W + xx];
-                    if (ws > 0) {
-                        float xc = xx + 0.5f, yc = yy + 0.5f;
-                        float fw = filter_weight(S.filter_type, radius, xc - rpt.x, yc - rpt.y);
-                        float4 dp = reinterpret_cast<const float4 *>(d_img)[yy * G.W + xx];
-                        float dpc = dot(V4{dp.x, dp.y, dp.z, dp.w}, color);
-                        float d_weight = (dpc * ws - fw * dpc * (ws - fw)) / (ws * ws);
-                        d_radius += d_filter_weight(S.filter_type, radius, xc - rpt.x, yc - rpt.y, d_weight);
-                    }
-                }
-            }
     }
     // workgroup reduction of the filter-radius adjoint, one atomic per tile
     float v = d_radius;

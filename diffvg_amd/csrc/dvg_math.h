@@ -356,6 +356,57 @@ DVG_DEV float d_filter_weight(int type, float radius, float dx, float dy, float 
     }
 }
 
+// filter_weight at one tap together with what d_filter_weight shares with it: the exponential
+// of the Gaussian, the cosines of the Hann window.
+struct FilterTap {
+    float w;
+    double a, b;
+};
+DVG_DEV FilterTap filter_tap(int type, float radius, float dx, float dy) {
+    FilterTap f{0.f, 0.0, 0.0};
+    const bool in = !(fabs((double)dx) > radius || fabs((double)dy) > radius);
+    if (type == kHann) {
+        const float tp = (float)(2 * kPi);
+        f.a = 1.0 - cos((double)(tp * ((dx / (2 * radius)) + 0.5f)));
+        f.b = 1.0 - cos((double)(tp * ((dy / (2 * radius)) + 0.5f)));
+        if (in) f.w = (float)(0.5f * f.a * 0.5f * f.b / (double)(radius * radius));
+    } else if (type == kGaussian) {
+        const double s = (double)radius / 3.0;
+        const double d2 = (double)dx * dx + (double)dy * dy;
+        const double w = exp(-d2 / (2.0 * s * s)) / (2.0 * kPi * s * s);
+        if (in) f.w = (float)w;
+        f.a = w * (d2 / (s * s * s) - 2.0 / s);
+    } else {
+        f.w = filter_weight(type, radius, dx, dy);
+    }
+    return f;
+}
+// d_filter_weight from the tap; r5 = radius^5 (used by the tent).
+DVG_DEV float filter_tap_adjoint(const FilterTap &f, int type, float radius, double r5, float dx, float dy,
+                                 float d_return) {
+    if (type == kTent) {
+        const double fx = (double)radius - fabs((double)dx), fy = (double)radius - fabs((double)dy);
+        const float norm = 1 / (radius * radius);
+        const double d_norm = (double)d_return * fx * fy;
+        return (float)((double)d_return * fy * norm + (double)d_return * fx * norm + (-4) * d_norm / r5);
+    } else if (type == kHann) {
+        const float ndx = (dx / (2 * radius)) + 0.5f, ndy = (dy / (2 * radius)) + 0.5f;
+        const float tp = (float)(2 * kPi);
+        const double fx = 0.5f * f.a, fy = 0.5f * f.b;
+        const float norm = 1 / (radius * radius);
+        const double d_fx = (double)d_return * fy * norm, d_fy = (double)d_return * fx * norm;
+        const double d_norm = (double)d_return * fx * fy;
+        const double d_ndx = d_fx * 0.5f * sin((double)(tp * ndx)) * (double)tp;
+        const double d_ndy = d_fy * 0.5f * sin((double)(tp * ndy)) * (double)tp;
+        const float tr = 2 * radius;
+        return (float)(d_ndx * (double)(-2 * dx / (tr * tr)) + d_ndy * (double)(-2 * dy / (tr * tr)) +
+                       (-2) * d_norm / (double)(radius * radius * radius));
+    } else if (type == kGaussian) {
+        return (float)((double)d_return * f.a / 3.0);
+    }
+    return d_filter_weight(type, radius, dx, dy, d_return);
+}
+
 DVG_DEV float smoothstep(float d) {
     float t = (d + 1.f) / 2.f;
     t = t < 0.f ? 0.f : (t > 1.f ? 1.f : t);

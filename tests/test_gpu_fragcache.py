@@ -67,6 +67,20 @@ def test_replayed_backward_equals_shading_backward(case, prefilter):
     assert np.array_equal(a.render(w, h, 2, 2, 5, prefilter=prefilter)['image'], fwd['image'])
 
 
+@pytest.mark.parametrize('n', [23, 24, 25, 27])
+def test_fills_around_the_kept_count(n):
+    """Without strokes the centre samples have n fragments; a forward keeps 24."""
+    print('fragcache fills', n, flush=True)
+    f = scenes.flat_case(layers(n=n, strokes=False))
+    w, h = f['canvas_width'], f['canvas_height']
+    d = np.random.default_rng(6).uniform(-1, 1, (h, w, 4)).astype(np.float32)
+    a = GpuRunner(f)
+    a.render(w, h, 2, 2, 5)
+    kept = a.render(w, h, 2, 2, 5, d_image=d, translation=True)
+    fresh = GpuRunner(f).render(w, h, 2, 2, 5, d_image=d, translation=True)
+    _same(kept, fresh, n)
+
+
 def test_lists_of_another_seed_are_not_used():
     print('fragcache seed', flush=True)
     f = _flat('layers')
