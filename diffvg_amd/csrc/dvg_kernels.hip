@@ -6,9 +6,11 @@
 //   k_color       one 256-lane workgroup (four wave64) per pixel tile: the workgroup
 //                 bins the groups whose inflated top-level box meets the tile into LDS,
 //                 in increasing group id, then every lane shades one sample against
-//                 that list, compositing fragments as they are found
+//                 that list, compositing fragments as they are found.  Scenes of one shape
+//                 per group run k_color_wave / k_edge_wave instead: a wave per workgroup
+//                 whose lanes share out the coverage tests (dvg_wave.h)
 //   k_resolve     per pixel: filter-weighted gather of the sample colours
-//   k_color_bwd   per tile: recompute fragments, reverse compositing sweep, paint
+//   k_color_bwd   per tile: replay the fragments the forward kept, reverse compositing sweep, paint
 //                 adjoints, filter-radius adjoint reduced per workgroup
 //   k_edge_sample / k_edge_bin / k_edge   boundary samples binned by pixel tile, both
 //                 sides of each boundary shaded against the tile's candidate list
@@ -827,7 +829,8 @@ DVG_DEV void edge_sample_one(const DevScene &S, const Geom &G, int idx, int coun
 // The same for a workgroup of kSampleBlock samples, counted per tile in LDS first and added to
 // a tile's count at once: a scene of few shapes sends its samples to the few tiles on their
 // boundaries, whose counters would take one atomic per sample (12.7 ns each).  2048 strokes
-// at 512x512, 4 samples: 143 -> 97 us; 24 scenes of one batch 2.8 -> 1.5 ms.  Canvases of
+// at 512x512, 4 samples: 143 -> 97 us; a batch of 256 scenes of up to 512 paths at 28 to 256
+// pixels 2.8 -> 1.5 ms.  Canvases of
 // more tiles than the table holds (48 KB: two workgroups of 16 waves fill a CU) add per sample.
 constexpr int kSampleBlock = 1024;
 constexpr int kSampleTiles = 12288;

@@ -11,8 +11,8 @@
 //     (one lane per segment); for each that is left, the lanes whose point its box holds push
 //     (segment, slot, lane);
 //   * screen: one item per lane, the float test (dvg_winding_fast.h) that decides most of them;
-//   * exact: what the screen left open, one item per lane: the reference's arithmetic
-//     (segment_winding, segment_within).
+//   * exact: what the screen left open, one item per lane: the reference's decision
+//     (cubic_winding_libm and cubic_roots_cr, cubic_stroke_search, quad_within).
 // Results come back through LDS: winding sums (added; their order does not matter) and
 // stroke hits (or-ed) per lane and slot.  kWaveSlots candidates are in flight at once; then
 // their fragments are composited in the list's order.

@@ -162,8 +162,10 @@ int dvg_scene_set_mode(dvg_scene *scene, int mode);
 int dvg_scene_set_tiling(dvg_scene *scene, int tile_width);
 /* Boundary samples per wavefront of the TILED edge kernel for later renders and batches
  * of this scene: 32 (each lane shades one of the two colour queries of a sample; the
- * default, also chosen by 0) or 64 (each lane shades both).  Picked by the autotuner;
- * results do not depend on it beyond float summation order.  No reference counterpart. */
+ * default, also chosen by 0) or 64 (each lane shades both).  Scenes whose groups hold one
+ * shape each run a wave-cooperative edge kernel instead (64 samples per wave, both points
+ * tested at once), which it does not change.  Picked by the autotuner; results do not
+ * depend on it beyond float summation order.  No reference counterpart. */
 int dvg_scene_set_samples_per_wave(dvg_scene *scene, int edge_samples_per_wave);
 
 /* Device-resident parameter values of a scene: DEVICE pointers on the scene's GPU, in the
