@@ -617,6 +617,8 @@ int build_scene(const dvg_scene_desc &d, int gpu_index, SceneHost &sc) {
     if (int e = clear_device(sc.device, sc.grad, reps * sc.grad_floats * sizeof(float))) return e;
     D.wave_ok = nseg <= kWaveMaxSegs;
     for (int g = 0; g < ng; g++) D.wave_ok &= d.group_num_shapes[g] == 1;
+    sc.round_shapes = false;
+    for (int s = 0; s < ns; s++) sc.round_shapes |= shape_type[s] == 0 || shape_type[s] == 1;
     for (int s = 0; s < ns; s++)
         if (shape_type[s] == 2) D.wave_ok &= !approx[s] && d.path_num_base_points[s] <= kWaveMaxPathSegs;
     D.rep_mask = reps - 1;

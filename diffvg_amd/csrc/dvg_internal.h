@@ -93,6 +93,7 @@ struct SceneHost {
     int tile_w = 0;               // pixel tile width of the TILED schedule (0 = square default)
     int edge_spw = 32;            // boundary samples per wave of the edge kernel: 32 or 64
     int cw = 0, ch = 0, num_shapes = 0, num_groups = 0;
+    bool round_shapes = false;  // circles or ellipses among them
     int num_shape_params = 0, num_points_total = 0, num_color_params = 0;
     void *block = nullptr;        // scene arrays
     size_t block_bytes = 0, block_granted = 0;

@@ -41,6 +41,7 @@ constexpr int kCandCap = 2048;
 // sample (32 samples per wave, the default), kBlock when each lane shades both sides (64
 // per wave); Geom::echunk holds the one a render uses (a tuning knob)
 constexpr int kEdgeChunk = kBlock / 2;
+constexpr int kWaveChunk = 64;  // of the wave-cooperative kernel, one wave
 // fragment lists kept from a colour forward for its backward: up to kFragSlots fragments
 // per sample (a sample with more is shaded again), at most kFragCacheBytes per scene.  24
 // slots instead of 16: one sample of more makes its whole tile wait for the shading; 2048
@@ -130,7 +131,7 @@ struct Geom {
     int tw, th, tiles_x, tiles_y;
     float sx_scale, sy_scale;  // canvas / render
     float margin;
-    int echunk;  // boundary samples per edge workgroup: 64 (wave-cooperative), kEdgeChunk or kBlock
+    int echunk;  // boundary samples per edge workgroup: kWaveChunk, kEdgeChunk or kBlock
     int prim_direct;  // primitives' boundary adjoints are added sample by sample (kPrimDirect)
 };
 
@@ -961,7 +962,7 @@ DVG_DEV void edge_scatter(const DevScene &S, const Geom &G, bool on, const EdgeS
 }
 
 // edge_chunk with the wave-cooperative coverage tests (dvg_wave.h), which test both points of
-// a sample at once where one decision holds for both: one wave, G.echunk = 64 samples of one
+// a sample at once where one decision holds for both: one wave, kWaveChunk samples of one
 // tile.  A chunk of 256 left a third of the lanes without a sample (a tile of the 300-path
 // scene holds 256 on average, so its second chunk is mostly empty).  A group of one shape
 // whose shape is hit also adds a fragment, so the hits that the coverage tests raise
@@ -985,7 +986,7 @@ DVG_DEV void edge_chunk_wave(EdgeWaveLds &L, const SceneRef &R, const Geom &G, i
     if (chunk >= chunk_off[ntiles]) return;
     const int lane = threadIdx.x;
     const int tile = find_tile(chunk_off, ntiles, chunk);
-    const int b0 = (chunk - chunk_off[tile]) * 64, cnt = min(64, tile_count[tile] - b0);
+    const int b0 = (chunk - chunk_off[tile]) * kWaveChunk, cnt = min(kWaveChunk, tile_count[tile] - b0);
     const bool valid = lane < cnt;
     const int eidx = valid ? sorted[tile_off[tile] + b0 + lane] : 0;
     const bool has_bg = bg != nullptr;
@@ -1739,8 +1740,13 @@ static Geom make_geom(const SceneHost &sc, const dvg_render_args &a) {
     if (th < 1) th = 1;
     G.tw = tw;
     G.th = th;
-    G.echunk = sc.dev.wave_ok ? 64 : (sc.edge_spw == 64 ? kBlock : kEdgeChunk);
     G.prim_direct = (int64_t)G.W * G.H * G.spp > kPrimDirect * sc.num_shapes;
+    // Circles and ellipses past kPrimDirect keep the per-lane kernel: their adds one by one are
+    // its time (one circle at 256x256, 4 samples: 10.0 ms either way), and the order in which
+    // its workgroups make them is what those sums of up to 10^5 and more terms of both signs
+    // round to (the wave kernel's order moves them by up to 9e-5, two runs of this one by 2e-5).
+    const bool wave = sc.dev.wave_ok && !(G.prim_direct && sc.round_shapes);
+    G.echunk = wave ? kWaveChunk : (sc.edge_spw == 64 ? kBlock : kEdgeChunk);
     G.tiles_x = (G.W + tw - 1) / tw;
     G.tiles_y = (G.H + th - 1) / th;
     G.sx_scale = (float)sc.cw / (float)G.W;
@@ -1937,7 +1943,7 @@ int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
                     DVG_PROF(st, "k_edge");
                     // at most one partial chunk per tile plus nsamp / echunk full ones
                     unsigned grid = (unsigned)(ntiles + (nsamp + G.echunk - 1) / G.echunk);
-                    if (S.wave_ok)
+                    if (G.echunk == kWaveChunk)
                         k_edge_wave<<<grid, 64, 0, st>>>(S, G, ws.edges, ws.tile_off, ws.tile_count, ws.chunk_off,
                                                              ntiles, ws.edge_sorted, a.background_image, ws.weight,
                                                              a.d_render_image, a.d_translation);
@@ -2667,11 +2673,11 @@ int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, i
             case kStTileF: return J.img && (J.pre || !J.S.wave_ok) ? J.ntiles : 0;
             case kStTileW: return J.img && !J.pre && J.S.wave_ok ? kTileWaves * J.ntiles : 0;
             case kStChunkW:
-                return edges && J.S.wave_ok ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
+                return edges && J.G.echunk == kWaveChunk ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
             case kStChunk:
                 return edges && J.G.echunk == kEdgeChunk ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
             case kStChunk2:
-                return edges && J.G.echunk == kBlock && !J.S.wave_ok ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
+                return edges && J.G.echunk == kBlock ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
             case kStSdf: return sdf ? (J.eval ? (J.num_eval + kBlock - 1) / kBlock : J.ntiles) : 0;
             default: return std::max(1, std::min(64, (std::max(J.grad_n, J.ntiles) + kBlock - 1) / kBlock));
         }
