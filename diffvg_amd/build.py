@@ -7,7 +7,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, 'csrc')
 LIB = os.path.join(HERE, 'libdiffvg_amd.so')
 SOURCES = ['dvg_host.cpp', 'dvg_kernels.hip']
-HEADERS = ['dvg_scene.h', 'dvg_math.h', 'dvg_crmath.h', 'dvg_query.h', 'dvg_winding_fast.h', 'dvg_shade.h', 'dvg_wave.h', 'dvg_memory.h',
+HEADERS = ['dvg_scene.h', 'dvg_math.h', 'dvg_crmath.h', 'dvg_quintic.h', 'dvg_query.h', 'dvg_winding_fast.h', 'dvg_shade.h', 'dvg_wave.h', 'dvg_memory.h',
            'dvg_internal.h', 'dvg_build.h', 'dvg_sort.h']
 
 # -ffp-contract=off keeps every multiply and add separately rounded, as the reference's

@@ -77,8 +77,11 @@ constexpr int64_t kPrimDirect = 12288;
 #ifndef DVG_WAVES_EDGE_WAVE
 #define DVG_WAVES_EDGE_WAVE 5
 #endif
-// the per-lane tests (scenes with groups of several shapes): as measured before the
-// double-precision searches were called rather than inlined
+// the per-lane tests (scenes with groups of several shapes).  k_edge: 300 paths in groups of two,
+// 600 strokes in groups of three and 2,048 strokes in groups of two, all at 512x512: backward
+// 1.96 / 2.88 / 6.95 ms at 5 waves, 2.15 / 3.14 / 7.64 at 4; at 6 it spills in the loop over the
+// segments (strokes 7.6).  The others as measured before the double-precision searches were
+// called rather than inlined.
 #ifndef DVG_WAVES_COLOR
 #define DVG_WAVES_COLOR 5
 #endif
@@ -86,7 +89,7 @@ constexpr int64_t kPrimDirect = 12288;
 #define DVG_WAVES_BATCH_COLOR 3
 #endif
 #ifndef DVG_WAVES_EDGE
-#define DVG_WAVES_EDGE 6
+#define DVG_WAVES_EDGE 5
 #endif
 #ifndef DVG_WAVES_BATCH_EDGE
 #define DVG_WAVES_BATCH_EDGE 5

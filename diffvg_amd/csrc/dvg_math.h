@@ -13,13 +13,11 @@
 
 #include <cstdint>
 
-#include "dvg_crmath.h"
+#include "dvg_quintic.h"
 
 namespace dvg {
 
 #define DVG_DEV __device__ __forceinline__
-
-constexpr double kPi = 3.14159265358979323846;
 
 struct V2 {
     float x, y;
@@ -212,21 +210,6 @@ DVG_DEV bool solve_quadratic_f(float a, float b, float c, float *t0, float *t1) 
     *t1 = r1;
     return true;
 }
-DVG_DEV bool solve_quadratic_d(double a, double b, double c, double *t0, double *t1) {
-    double discrim = b * b - 4 * a * c;
-    if (discrim < 0) return false;
-    double root_discrim = __builtin_sqrt(discrim);
-    double q = b < 0 ? -0.5f * (b - root_discrim) : -0.5f * (b + root_discrim);
-    double r0 = q / a, r1 = c / q;
-    if (r0 > r1) {
-        double tmp = r0;
-        r0 = r1;
-        r1 = tmp;
-    }
-    *t0 = r0;
-    *t1 = r1;
-    return true;
-}
 // solve_cubic<float>: sqrt/acos/cos/pow are evaluated in double, as in the reference.
 DVG_DEV int solve_cubic_f(float a, float b, float c, float d, float t[3]) {
     if (fabs((double)a) < 1e-6f) {
@@ -252,37 +235,6 @@ DVG_DEV int solve_cubic_f(float a, float b, float c, float d, float t[3]) {
         float A = R > 0 ? (float)-pow((double)R + disc, third) : (float)pow((double)-R + disc, third);
         float B = fabs((double)A) > 1e-6f ? Q / A : 0.f;
         t[0] = (A + B) - b / 3.f;
-        return 1;
-    }
-}
-// solve_cubic<double> (solve.h:29-64).  CR selects the correctly rounded acos, cos and
-// pow; the default uses the device libm.
-template <bool CR = false>
-DVG_DEV int solve_cubic_d(double a, double b, double c, double d, double t[3]) {
-    if (fabs(a) < 1e-6f) {
-        if (solve_quadratic_d(b, c, d, &t[0], &t[1])) return 2;
-        return 0;
-    }
-    b /= a;
-    c /= a;
-    d /= a;
-    double Q = (b * b - 3 * c) / 9.f;
-    double R = (2 * b * b * b - 9 * b * c + 27 * d) / 54.f;
-    if (R * R < Q * Q * Q) {
-        double x = R / sqrt(Q * Q * Q);
-        double theta = CR ? cr::acos_cr(x) : acos(x);
-        double sq = sqrt(Q);
-        double a0 = theta / 3.f, a1 = (theta + 2.f * kPi) / 3.f, a2 = (theta - 2.f * kPi) / 3.f;
-        t[0] = -2.f * sq * (CR ? cr::cos_cr(a0) : cos(a0)) - b / 3.f;
-        t[1] = -2.f * sq * (CR ? cr::cos_cr(a1) : cos(a1)) - b / 3.f;
-        t[2] = -2.f * sq * (CR ? cr::cos_cr(a2) : cos(a2)) - b / 3.f;
-        return 3;
-    } else {
-        double base = R > 0 ? R + sqrt(R * R - Q * Q * Q) : -R + sqrt(R * R - Q * Q * Q);
-        double root = CR ? cr::pow_cr(base, 1. / 3.) : pow(base, 1. / 3.);
-        double A = R > 0 ? -root : root;
-        double B = fabs(A) > 1e-6f ? Q / A : 0.0;
-        t[0] = (A + B) - b / 3.0;
         return 1;
     }
 }

@@ -64,11 +64,14 @@ DVG_DEV wf::StrokePrep stroke_prep_of(const DevScene &S, int seg) {
 struct CubicPoints {
     V2 p0, p1, p2, p3;
 };
-DVG_DEV CubicPoints cubic_points_of(const DevScene &S, int seg) {
-    const float4 *src = S.seg_wf + kSegPrep * (size_t)seg + kSegPoints;
+DVG_DEV const float4 *cubic_points_at(const DevScene &S, int seg) {
+    return S.seg_wf + kSegPrep * (size_t)seg + kSegPoints;
+}
+DVG_DEV CubicPoints cubic_points(const float4 *src) {
     const float4 a = src[0], b = src[1];
     return CubicPoints{V2{a.x, a.y}, V2{a.z, a.w}, V2{b.x, b.y}, V2{b.z, b.w}};
 }
+DVG_DEV CubicPoints cubic_points_of(const DevScene &S, int seg) { return cubic_points(cubic_points_at(S, seg)); }
 
 DVG_DEV V2 qeval(V2 p0, V2 p1, V2 p2, float t) {
     float tt = 1 - t;
@@ -245,183 +248,6 @@ DVG_DEV V2 quadratic_closest_pt_approx(V2 b0, V2 b1, V2 b2, V2 pt, float *t_ = n
     return (tt * tt) * b0 + (2 * tt * t) * b1 + (t * t) * b2 + pt;
 }
 
-// The stationary points of the distance to a cubic: roots of a quintic, isolated by the roots
-// of a cubic and a linear factor (within_distance.h:119-272, compute_distance.h:127-280).  The
-// arithmetic is double; next to the reference's, divisions by one number are products with
-// its reciprocal, polynomials are evaluated by Horner's rule with fused multiply-adds and the
-// trigonometric roots come from one sine and cosine: roundings of the last bit or two, in
-// interval ends and iterates that are then stored as floats.  (A point's coverage by its 2,048
-// strokes took half of the edge kernel: 17 double divisions, three cosines, a power and 45
-// double operations a Newton step for each.)
-struct Quintic {
-    double A, B, C, D, E, F;  // leading coefficient, and the others divided by it
-};
-DVG_DEV Quintic cubic_quintic(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
-    V2 a = -p0 + 3 * p1 - 3 * p2 + p3;
-    V2 b = 3 * p0 - 6 * p1 + 3 * p2;
-    V2 c = -3 * p0 + 3 * p1;
-    V2 d = p0 - pt;
-    Quintic q;
-    q.A = 3 * vsum(a * a);
-    const double inv = 1.0 / q.A;
-    q.B = (double)(5 * vsum(a * b)) * inv;
-    q.C = (double)(4 * vsum(a * c) + 2 * vsum(b * b)) * inv;
-    q.D = (double)(3 * (vsum(b * c) + vsum(a * d))) * inv;
-    q.E = (double)(vsum(c * c) + 2 * vsum(d * b)) * inv;
-    q.F = (double)vsum(d * c) * inv;
-    return q;
-}
-DVG_DEV double quintic_eval(const Quintic &q, double t) {
-    return __builtin_fma(__builtin_fma(__builtin_fma(__builtin_fma(t + q.B, t, q.C), t, q.D), t, q.E), t, q.F);
-}
-DVG_DEV double quintic_deriv(const Quintic &q, double t) {
-    return __builtin_fma(__builtin_fma(__builtin_fma(__builtin_fma(5.0, t, 4 * q.B), t, 3 * q.C), t, 2 * q.D), t, q.E);
-}
-// sin and cos of x in [0, pi / 3] by their Taylor series (to x^21 and x^20; the next terms are
-// below 1e-20)
-DVG_DEV void sincos_third(double x, double &s, double &c) {
-    const double z = x * x;
-    double p = 1.0 / 51090942171709440000.0, r = 1.0 / 2432902008176640000.0;
-    p = __builtin_fma(p, z, -1.0 / 121645100408832000.0);
-    r = __builtin_fma(r, z, -1.0 / 6402373705728000.0);
-    p = __builtin_fma(p, z, 1.0 / 355687428096000.0);
-    r = __builtin_fma(r, z, 1.0 / 20922789888000.0);
-    p = __builtin_fma(p, z, -1.0 / 1307674368000.0);
-    r = __builtin_fma(r, z, -1.0 / 87178291200.0);
-    p = __builtin_fma(p, z, 1.0 / 6227020800.0);
-    r = __builtin_fma(r, z, 1.0 / 479001600.0);
-    p = __builtin_fma(p, z, -1.0 / 39916800.0);
-    r = __builtin_fma(r, z, -1.0 / 3628800.0);
-    p = __builtin_fma(p, z, 1.0 / 362880.0);
-    r = __builtin_fma(r, z, 1.0 / 40320.0);
-    p = __builtin_fma(p, z, -1.0 / 5040.0);
-    r = __builtin_fma(r, z, -1.0 / 720.0);
-    p = __builtin_fma(p, z, 1.0 / 120.0);
-    r = __builtin_fma(r, z, 1.0 / 24.0);
-    p = __builtin_fma(p, z, -1.0 / 6.0);
-    r = __builtin_fma(r, z, -0.5);
-    s = __builtin_fma(p * z, x, x);
-    c = __builtin_fma(r, z, 1.0);
-}
-// Roots of a t^3 + b t^2 + c t + d as solve_cubic_d returns them (solve.h:29-64).
-DVG_DEV int isolating_cubic(double a, double b, double c, double d, double (&t)[3]) {
-    if (fabs(a) < 1e-6f) return solve_quadratic_d(b, c, d, &t[0], &t[1]) ? 2 : 0;
-    const double inv = 1.0 / a, third = 1.0 / 3.0;
-    b *= inv;
-    c *= inv;
-    d *= inv;
-    const double Q = (b * b - 3 * c) * (1.0 / 9.0);
-    const double R = (2 * b * b * b - 9 * b * c + 27 * d) * (1.0 / 54.0);
-    const double Q3 = Q * Q * Q, b3 = b * third;
-    if (R * R < Q3) {
-        double s, co;
-        sincos_third(acos(R / sqrt(Q3)) * third, s, co);
-        const double h = 0.86602540378443864676 * s, m = -2.0 * __builtin_sqrt(Q);
-        t[0] = m * co - b3;
-        t[1] = m * (-0.5 * co - h) - b3;
-        t[2] = m * (-0.5 * co + h) - b3;
-        return 3;
-    }
-    const double root = cbrt(fabs(R) + __builtin_sqrt(R * R - Q3));
-    const double A = R > 0 ? -root : root;
-    const double B = fabs(A) > 1e-6f ? Q / A : 0.0;
-    t[0] = (A + B) - b3;
-    return 1;
-}
-// Isolating intervals (within_distance.h:195-216); the reference's uninitialised
-// intervals[0] (isolator root outside [0, 1]) is treated as absent.
-// All indices are compile-time constants (slots past n are not read as such), so the array
-// stays in registers.
-DVG_DEV int quintic_intervals(const Quintic &q, float (&iv)[4]) {
-    // the reference's float fractions
-    const double p1A = (2 / 5.f) * q.C - (4 / 25.f) * q.B * q.B;
-    const double p1B = (3 / 5.f) * q.D - (3 / 25.f) * q.B * q.C;
-    const double p1C = (4 / 5.f) * q.E - (2 / 25.f) * q.B * q.D;
-    const double p1D = q.F - q.B * q.E * (1.0 / 25.0);
-    const double q_root = q.B * -0.2;
-    double pr[3] = {0.0, 0.0, 0.0};
-    const int num_sol = isolating_cubic(p1A, p1B, p1C, p1D, pr);
-    const bool first = q_root >= 0 && q_root <= 1;
-    const int n = num_sol + (first ? 1 : 0);
-    iv[0] = first ? (float)q_root : (float)pr[0];
-    iv[1] = first ? (float)pr[0] : (float)pr[1];
-    iv[2] = first ? (float)pr[1] : (float)pr[2];
-    iv[3] = (float)pr[2];
-    // insertion sort of the first n
-#pragma unroll
-    for (int j = 1; j < 4; j++) {
-        bool go = j < n;
-#pragma unroll
-        for (int k = j; k > 0; k--) {
-            go = go && iv[k - 1] > iv[k];
-            const float lo = go ? iv[k] : iv[k - 1], hi = go ? iv[k - 1] : iv[k];
-            iv[k - 1] = lo;
-            iv[k] = hi;
-        }
-    }
-    return n;
-}
-// Newton's iteration kept in its bracket (within_distance.h:232-262)
-DVG_DEV float quintic_root(const Quintic &q, float lb, float ub) {
-    float t = 0.5f * (lb + ub);
-#pragma nounroll
-    for (int it = 0; it < 20; it++) {
-        if (!(t >= lb && t <= ub)) t = 0.5f * (lb + ub);
-        const double td = t;
-        const double value = quintic_eval(q, td);
-        if (fabs(value) < 1e-5f || it == 19) break;
-        if (value > 0.f)
-            ub = t;
-        else
-            lb = t;
-        const double deriv = quintic_deriv(q, td);
-        double r = __builtin_amdgcn_rcp(deriv);
-        r = __builtin_fma(__builtin_fma(-deriv, r, 1.0), r, r);
-        r = __builtin_fma(__builtin_fma(-deriv, r, 1.0), r, r);
-        t = (float)__builtin_fma(-value, r, td);
-    }
-    return t;
-}
-// Calls visit(t) for the root in each interval with a sign change, in order, until it
-// returns true.  The brackets are found first, so that the lanes of a wave run their first
-// searches together, then their second ones, whichever intervals those are.
-template <class Visit>
-DVG_DEV void quintic_search(const Quintic &q, const Visit &visit) {
-    float iv[4];
-    const int n = quintic_intervals(q, iv);
-    float lo[5], hi[5];
-    unsigned found = 0;
-    float lower = 0.f;
-    double at_lower = quintic_eval(q, 0.0);
-    bool more = true;
-#pragma unroll
-    for (int j = 0; j < 5; j++) {
-        const bool inner = j < 4 && j < n;
-        const float end = j < 4 ? iv[j < 4 ? j : 3] : 1.f;
-        const bool use = more && j <= n && !(inner && end < 0.f);
-        const float upper = inner ? fmin_r(end, 1.f) : 1.f;
-        const double at_upper = quintic_eval(q, upper);
-        const bool change = use && !(at_lower * at_upper > 0);
-        const bool falls = at_lower > at_upper;
-        lo[j] = falls ? upper : lower;
-        hi[j] = falls ? lower : upper;
-        if (change) {
-            found |= 1u << j;
-            more = !(upper >= 1.f);
-            lower = upper;
-            at_lower = at_upper;
-        }
-    }
-#pragma nounroll
-    while (found) {
-        const int j = __ffs(found) - 1;
-        found &= found - 1;
-        const float lb = j < 2 ? (j == 0 ? lo[0] : lo[1]) : (j == 2 ? lo[2] : (j == 3 ? lo[3] : lo[4]));
-        const float ub = j < 2 ? (j == 0 ? hi[0] : hi[1]) : (j == 2 ? hi[2] : (j == 3 ? hi[3] : hi[4]));
-        if (visit(quintic_root(q, lb, ub))) break;
-    }
-}
-
 // Every point of cubic segment `seg` is certainly farther than r from pt (the chords of an
 // 8-step polyline, the chords' deviation bound and a rounding margin, from the segment's
 // prep); false for r = inf.
@@ -429,18 +255,60 @@ DVG_DEV bool cubic_farther_than(const DevScene &S, int seg, V2 pt, float r) {
     return wf::stroke_farther(stroke_prep_of(S, seg), pt.x, pt.y, r);
 }
 
+DVG_DEV QuinticSums quintic_sums(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
+    return cubic_quintic_sums(p0.x, p0.y, p1.x, p1.y, p2.x, p2.y, p3.x, p3.y, pt.x, pt.y);
+}
+// The plain search's intervals, in a call of their own, and the points read again after it (the
+// laundered address keeps the first ones from staying live): with both in one function the
+// kernels would need more registers than they are compiled for.
+struct PlainIntervals {
+    float a, b, c, d;
+    int n;
+};
+static __device__ __noinline__ PlainIntervals plain_intervals(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
+    float iv[4];
+    const int n = quintic_intervals_plain(cubic_quintic_plain(quintic_sums(p0, p1, p2, p3, pt)), iv);
+    return PlainIntervals{iv[0], iv[1], iv[2], iv[3], n};
+}
+// plain(p0..p3) visits the roots of quintic_search_plain of the segment whose points lie at src
+template <class Visit>
+DVG_DEV void plain_search(const float4 *src, V2 pt, const Visit &visit) {
+    const CubicPoints c = cubic_points(src);
+    const PlainIntervals v = plain_intervals(c.p0, c.p1, c.p2, c.p3, pt);
+    asm volatile("" : "+v"(src));
+    const CubicPoints p = cubic_points(src);
+    const float iv[4] = {v.a, v.b, v.c, v.d};
+    quintic_search_plain(cubic_quintic_plain(quintic_sums(p.p0, p.p1, p.p2, p.p3, pt)), iv, v.n,
+                         [&](float t) { return visit(p, t); });
+}
 // Whether one of the stationary points of the distance to a cubic that the quintic search
 // finds lies within the stroke's radius there (within_distance.h:119-272 past its end tests).
-static __device__ __noinline__ bool cubic_stroke_search(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2,
-                                                        float r3) {
+DVG_DEV bool within_at(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float t, float r0, float r1, float r2, float r3) {
+    float tt = 1 - t;
+    float rr = (tt * tt * tt) * r0 + (3 * tt * tt * t) * r1 + (3 * tt * t * t) * r2 + (t * t * t) * r3;
+    return dist_sq(ceval(p0, p1, p2, p3, t), pt) < rr * rr;
+}
+// 0 or 1; 2: the coefficients are large and the plain search decides
+static __device__ __noinline__ int cubic_stroke_fast(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2,
+                                                     float r3) {
+    const Quintic q = cubic_quintic(quintic_sums(p0, p1, p2, p3, pt));
+    if (quintic_large(q)) return 2;
     bool hit = false;
-    quintic_search(cubic_quintic(p0, p1, p2, p3, pt), [&](float t) {
-        float tt = 1 - t;
-        float rr = (tt * tt * tt) * r0 + (3 * tt * tt * t) * r1 + (3 * tt * t * t) * r2 + (t * t * t) * r3;
-        hit = dist_sq(ceval(p0, p1, p2, p3, t), pt) < rr * rr;
-        return hit;
+    quintic_search(q, [&](float t) { return hit = within_at(p0, p1, p2, p3, pt, t, r0, r1, r2, r3); });
+    return hit;
+}
+static __device__ __noinline__ bool cubic_stroke_plain(const float4 *src, V2 pt, float r0, float r1, float r2, float r3) {
+    bool hit = false;
+    plain_search(src, pt, [&](const CubicPoints &p, float t) {
+        return hit = within_at(p.p0, p.p1, p.p2, p.p3, pt, t, r0, r1, r2, r3);
     });
     return hit;
+}
+// of the segment whose points, p0 to p3, lie at src
+DVG_DEV bool cubic_stroke_search(const float4 *src, V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2,
+                                 float r3) {
+    const int hit = cubic_stroke_fast(p0, p1, p2, p3, pt, r0, r1, r2, r3);
+    return hit != 2 ? hit : cubic_stroke_plain(src, pt, r0, r1, r2, r3);
 }
 
 // Stroke test of a line and of a quadratic segment (within_distance.h:32-118), radius r0, r1
@@ -508,7 +376,7 @@ DVG_DEV int segment_within(const DevScene &S, int s, int seg, V2 pt, float r) {
     // every curve point certainly farther than the largest radius magnitude (the radius
     // at t is a convex combination of r0..r3): the quintic search below would find nothing
     if (cubic_farther_than(S, seg, pt, fmaxf(fmaxf(fabsf(r0), fabsf(r1)), fmaxf(fabsf(r2), fabsf(r3))))) return 0;
-    return cubic_stroke_search(p0, p1, p2, p3, pt, r0, r1, r2, r3);
+    return cubic_stroke_search(cubic_points_at(S, seg), p0, p1, p2, p3, pt, r0, r1, r2, r3);
 }
 
 DVG_DEV bool within_distance_path(const DevScene &S, int s, V2 pt, float r) {
@@ -626,18 +494,41 @@ struct CubicClosest {
     float dist, t;
     V2 pt;
 };
-static __device__ __noinline__ CubicClosest cubic_closest(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
+DVG_DEV CubicClosest closest_end(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
     V2 pt0 = ceval(p0, p1, p2, p3, 0), pt1 = ceval(p0, p1, p2, p3, 1);
     float d0 = dist(pt0, pt), d1 = dist(pt1, pt);
-    CubicClosest r{d0, 0.f, pt0};
-    if (d1 < r.dist) r = CubicClosest{d1, 1.f, pt1};
-    quintic_search(cubic_quintic(p0, p1, p2, p3, pt), [&](float t) {
-        V2 pp = ceval(p0, p1, p2, p3, t);
-        float dp = dist(pp, pt);
-        if (dp < r.dist) r = CubicClosest{dp, t, pp};
-        return false;
-    });
+    return d1 < d0 ? CubicClosest{d1, 1.f, pt1} : CubicClosest{d0, 0.f, pt0};
+}
+DVG_DEV bool closer_at(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float t, CubicClosest &r) {
+    V2 pp = ceval(p0, p1, p2, p3, t);
+    float dp = dist(pp, pt);
+    if (dp < r.dist) r = CubicClosest{dp, t, pp};
+    return false;
+}
+// t = -1: the coefficients are large and the plain search decides
+static __device__ __noinline__ CubicClosest cubic_closest_fast(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
+    const Quintic q = cubic_quintic(quintic_sums(p0, p1, p2, p3, pt));
+    if (quintic_large(q)) return CubicClosest{0.f, -1.f, pt};
+    CubicClosest r = closest_end(p0, p1, p2, p3, pt);
+    quintic_search(q, [&](float t) { return closer_at(p0, p1, p2, p3, pt, t, r); });
     return r;
+}
+static __device__ __noinline__ CubicClosest cubic_closest_plain(const float4 *src, V2 pt) {
+    CubicClosest r{0.f, -1.f, pt};
+    plain_search(src, pt, [&](const CubicPoints &p, float t) {
+        if (r.t < 0.f) r = closest_end(p.p0, p.p1, p.p2, p.p3, pt);
+        return closer_at(p.p0, p.p1, p.p2, p.p3, pt, t, r);
+    });
+    if (r.t < 0.f) {
+        const CubicPoints p = cubic_points(src);
+        r = closest_end(p.p0, p.p1, p.p2, p.p3, pt);
+    }
+    return r;
+}
+DVG_DEV CubicClosest cubic_closest(const float4 *src, V2 pt) {
+    const CubicPoints c = cubic_points(src);
+    const CubicClosest r = cubic_closest_fast(c.p0, c.p1, c.p2, c.p3, pt);
+    return r.t >= 0.f ? r : cubic_closest_plain(src, pt);
 }
 
 // closest_point for a path (compute_distance.h:27-300): the segments in the reference's
@@ -658,8 +549,7 @@ DVG_DEV bool closest_point_path(const DevScene &S, int s, V2 pt, float max_radiu
         float dd;
         if (S.seg_kind[seg] == 2) {
             if (cubic_farther_than(S, seg, pt, min_dist)) continue;
-            const CubicPoints c = cubic_points_of(S, seg);
-            const CubicClosest r = cubic_closest(c.p0, c.p1, c.p2, c.p3, pt);
+            const CubicClosest r = cubic_closest(cubic_points_at(S, seg), pt);
             dd = r.dist;
             cp = r.pt;
             tr = r.t;
@@ -830,7 +720,7 @@ DVG_DEV int d_closest_point_path_vals(const DevScene &S, int s, V2 pt, V2 d_cp, 
         } else if (t == 1) {
             d_p3 += d_cp;
         } else {
-            Quintic q = cubic_quintic(p0, p1, p2, p3, pt);
+            Quintic q = cubic_quintic_plain(quintic_sums(p0, p1, p2, p3, pt));
             double A = q.A;
             V2 d_p = d_cp;
             float tt = 1 - t;
@@ -840,7 +730,7 @@ DVG_DEV int d_closest_point_path_vals(const DevScene &S, int s, V2 pt, V2 d_cp, 
             d_p1 += d_p * (3 * tt * tt * t);
             d_p2 += d_p * (3 * tt * t * t);
             d_p3 += d_p * (t * t * t);
-            double poly_deriv_t = quintic_deriv(q, t);
+            double poly_deriv_t = quintic_deriv_plain(q, t);
             if (fabs(poly_deriv_t) > 1e-10f) {
                 double r = d_t / poly_deriv_t;
                 double d_B = -r * t * t * t * t;

@@ -12,7 +12,8 @@
 //     (segment, slot, lane);
 //   * screen: one item per lane, the float test (dvg_winding_fast.h) that decides most of them;
 //   * exact: what the screen left open, one item per lane: the reference's decision
-//     (cubic_winding_libm and cubic_roots_cr, cubic_stroke_search, quad_within).
+//     (cubic_winding_libm and cubic_roots_cr, quad_within; cubic_stroke_search, which keeps the
+//     reference's operations only where their last bits decide: kQuinticLarge).
 // Results come back through LDS: winding sums (added; their order does not matter) and
 // stroke hits (or-ed) per lane and slot.  kWaveSlots candidates are in flight at once; then
 // their fragments are composited in the list's order.
@@ -130,7 +131,8 @@ DVG_DEV void wave_exact(const SceneRef &R, WaveLds<SIDES> &W, int &n2, int cnt) 
                         r3 = S.thickness[idx.w];
                     }
                     hit = dist_sq(c.p0, p) < r0 * r0 || dist_sq(c.p3, p) < r3 * r3;
-                    if (!hit) hit = cubic_stroke_search(c.p0, c.p1, c.p2, c.p3, p, r0, r1, r2, r3);
+                    if (!hit)
+                        hit = cubic_stroke_search(cubic_points_at(S, seg), c.p0, c.p1, c.p2, c.p3, p, r0, r1, r2, r3);
                 } else {
                     hit = wave_within_lq(S, s, seg, k, p, r);
                 }
