@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -99,6 +100,11 @@ struct SceneHost {
     size_t block_bytes = 0, block_granted = 0;
     float *grad = nullptr;        // gradient arrays
     size_t grad_floats = 0, grad_granted = 0;  // floats of one copy (DevScene::rep_mask)
+    // the stream whose backwards may add to the gradient copies (take_copies); the mutex is
+    // held from the choice to the fold's launch
+    std::mutex copies_mu;
+    bool copies_owned = false;
+    hipStream_t copies_stream = nullptr;
     size_t g_params = 0, g_points = 0, g_thick = 0, g_sw = 0, g_color = 0, g_xform = 0, g_filter = 0;
     // [0] render conditions, [1] conditions found by dvg_scene_update, [2] parameter
     // version on the device (advanced by every update), [4..9] and [10..15] the key of the

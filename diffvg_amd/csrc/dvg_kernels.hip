@@ -1194,8 +1194,9 @@ __global__ __launch_bounds__(64, DVG_WAVES_EDGE_WAVE) void k_edge_wave(
 }
 
 // Adds the gradient copies 1..rep_mask to the block and clears them (DevScene::rep_mask).
-// Exchanges and atomic adds: another render of the scene on another stream may be adding to
-// the copies, and what it adds after the exchange is folded by its own backward.
+// Only one stream's backwards add to a scene's copies and fold them (take_copies): between the
+// exchange and the add a sum is in neither place, and a backward of another stream would end
+// without it in the block.
 // A workgroup folds 64 floats: wave w exchanges copies 1 + w, 5 + w, ... with all exchanges in
 // flight at once (one after another they would cost a memory round trip each), and the four
 // partial sums meet in LDS.
@@ -1822,6 +1823,37 @@ static bool keep_buffer(SceneHost &sc, void *&ptr, size_t &granted, hipStream_t 
     return ptr != nullptr;
 }
 
+static bool is_capturing(hipStream_t st) {
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    return st && (hipStreamIsCapturing(st, &c) != hipSuccess || c != hipStreamCaptureStatusNone);
+}
+
+// Whether a backward on stream `st` may add to the scene's gradient copies; one that may not
+// adds to the block itself, which any number of streams may do at once.  The copies belong to
+// one stream, and pass to another only when the first is idle (its folds are done).  A backward
+// captured into a graph never uses them: its replays may run beside any stream.
+static bool take_copies(SceneHost &sc, hipStream_t st) {
+    if (is_capturing(st)) return false;
+    if (!sc.copies_owned || sc.copies_stream == st) {
+        sc.copies_owned = true;
+        sc.copies_stream = st;
+        return true;
+    }
+    if (is_capturing(sc.copies_stream)) return false;  // not to be queried
+    hipError_t e = hipStreamQuery(sc.copies_stream);
+    if (e != hipSuccess) (void)hipGetLastError();
+    if (e == hipErrorNotReady) return false;
+    if (e != hipSuccess) {  // a stream that is no more
+        e = hipDeviceSynchronize();
+        if (e != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+    }
+    sc.copies_stream = st;
+    return true;
+}
+
 int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
     hipStream_t st = (hipStream_t)a.stream;
     Geom G = make_geom(sc, a);
@@ -1836,6 +1868,15 @@ int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
     const bool color_out = a.render_image || a.d_render_image;
     const bool sdf_out = a.render_sdf || a.d_render_sdf;
     int ntiles = G.tiles_x * G.tiles_y;
+    // the copies are added to by the colour backward and the tiled SDF's
+    std::unique_lock<std::mutex> copies(sc.copies_mu, std::defer_lock);
+    if (S.rep_mask && (a.d_render_image || (a.d_render_sdf && !eval_mode))) {
+        copies.lock();
+        if (!take_copies(sc, st)) {
+            S.rep_mask = 0;
+            copies.unlock();
+        }
+    }
     if (color_out) {
         Workspace &ws = fixed ? *fixed : acquire_workspace(sc.device, st);
         struct Release {
@@ -1974,7 +2015,7 @@ int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed) {
             k_sdf_tiled<<<ntiles, kBlock, 0, st>>>(S, G, a.render_sdf, a.d_render_sdf, a.d_translation);
         }
     }
-    if ((a.d_render_image || a.d_render_sdf) && S.rep_mask)
+    if (copies.owns_lock())
         k_fold_grads<<<(unsigned)((S.rep_stride + 63) / 64), kBlock, 0, st>>>(S, sc.grad);
     DVG_CHECK(hipGetLastError());
     // nothing waits here: conditions the kernels flag are reported by scene_status

@@ -128,7 +128,8 @@ int dvg_scene_destroy(dvg_scene *scene);
  * scene's gradient buffers.  Asynchronous on args->stream in DVG_MODE_TILED (conditions
  * the reference asserts on -- fragment overflow, prefiltered circle strokes -- are then
  * reported by dvg_scene_status and dvg_scene_get_grads); synchronous in DVG_MODE_PLAIN,
- * like the reference. */
+ * like the reference.  Backwards of one scene on several streams at once add up; when the
+ * work enqueued on one of them ends, its sums are in the gradient buffers. */
 int dvg_render(dvg_scene *scene, const dvg_render_args *args);
 
 /* dvg_render in DVG_MODE_TILED (whatever the scene's mode) that allocates no device
@@ -151,7 +152,8 @@ int dvg_scene_grad_layout(dvg_scene *scene, int64_t *offsets, int64_t *total_flo
 /* Copies the gradient block to device memory `dst` (total_floats floats), stream-ordered
  * on `stream`: the device-resident counterpart of dvg_scene_get_grads. */
 int dvg_scene_copy_grads(dvg_scene *scene, float *dst, void *stream);
-/* Clears the gradient buffers (stream-ordered on `stream`). */
+/* Clears the gradient buffers (stream-ordered on `stream`).  A backward that is running on
+ * another stream meanwhile may leave any part of its sums behind. */
 int dvg_scene_zero_grads(dvg_scene *scene, void *stream);
 /* Selects DVG_MODE_TILED (default) or DVG_MODE_PLAIN for later renders. */
 int dvg_scene_set_mode(dvg_scene *scene, int mode);
