@@ -2258,12 +2258,14 @@ __global__ __launch_bounds__(kBlock) void kb_zero(const Job *jobs, const int *pr
         for (int i = b * kBlock + threadIdx.x; i < J.grad_n; i += nb * kBlock) J.grad[i] = 0.f;
 }
 
-// one row of workgroups per job; a workgroup strides over the job's gradient block
+// kFoldBlocks workgroups per job, which stride over the job's gradient block; one dimension,
+// as a grid's second one ends at 65,535 and a batch may hold more jobs
+constexpr int kFoldBlocks = 8;
 __global__ __launch_bounds__(kBlock) void kb_fold_grads(const Job *jobs) {
-    const Job J = load_job(jobs + blockIdx.y);
+    const Job J = load_job(jobs + blockIdx.x / kFoldBlocks);
     if (!(J.d_img || J.d_sdf) || !J.S.rep_mask) return;
     __shared__ float part[4][64];
-    for (int base = blockIdx.x * 64; base < J.S.rep_stride; base += gridDim.x * 64)
+    for (int base = (blockIdx.x % kFoldBlocks) * 64; base < J.S.rep_stride; base += kFoldBlocks * 64)
         fold_grads(J.S, J.grad, base, part);
 }
 
@@ -2886,7 +2888,7 @@ int batch_render(BatchHost &B, hipStream_t st) {
         if (c == 2) {
             DVG_PROF(st, "kb_sdf");
             kb_sdf<<<T(kStSdf), kBlock, 0, st>>>(J, P(kStSdf), nj);
-            if (B.fold[c]) kb_fold_grads<<<dim3(8, (unsigned)nj), kBlock, 0, st>>>(J);
+            if (B.fold[c]) kb_fold_grads<<<kFoldBlocks * (unsigned)nj, kBlock, 0, st>>>(J);
             continue;
         }
         {
@@ -2926,7 +2928,7 @@ int batch_render(BatchHost &B, hipStream_t st) {
                     if (T(kStChunkW)) kb_edge_wave<<<T(kStChunkW), 64, 0, st>>>(J, P(kStChunkW), nj);
                 }
             }
-            if (B.fold[c]) kb_fold_grads<<<dim3(8, (unsigned)nj), kBlock, 0, st>>>(J);
+            if (B.fold[c]) kb_fold_grads<<<kFoldBlocks * (unsigned)nj, kBlock, 0, st>>>(J);
         }
     }
     hipError_t e = hipGetLastError();

@@ -428,3 +428,23 @@ def test_uneven_scenes_256_graph():
         for k in GRAD_KEYS:
             if gw[k].size:
                 assert _rel(g0[i][k], gw[k]) <= 1e-3, (i, k)
+
+
+def test_backward_batch_of_more_jobs_than_a_grid_has_rows():
+    """66,000 backward jobs (of one scene): past 65,535, where a grid's second dimension ends.
+    Each adds the same terms; 2,000 of them land in one of the 32 copies of a gradient, whose
+    float sum loses up to 2,000 x 2^-24."""
+    print('batch of 66000 jobs', flush=True)
+    f = scenes.flat_case('curve_fill')
+    sc = _lib.DeviceScene(f, 0)
+    d = torch.from_numpy(np.random.default_rng(4).uniform(0.5, 1, (4, 4, 4)).astype(np.float32)).to(DEV)
+    job = dict(width=4, height=4, nsx=2, nsy=2, seed=3, d_render_image=d)
+    sc.zero_grads(None)
+    sc.render(**job)
+    one = sc.grads()
+    n = 66000
+    Batch([(sc, job)] * n).render(None)
+    many = sc.grads()
+    for k in ('points', 'color_params'):
+        assert np.abs(one[k]).max() > 0
+        assert _rel(many[k] / n, one[k]) <= 2e-4, k
