@@ -20,9 +20,9 @@ PERSISTENT = 2
 
 
 class Batch:
-    """`persistent`: the whole render is one kernel launch whose workgroups take the
-    batch's work items from a device queue (DVG_BATCH_PERSISTENT), instead of one launch
-    per stage."""
+    """`persistent` asks for one kernel launch whose workgroups take the batch's work items
+    from a device queue (DVG_BATCH_PERSISTENT) instead of one launch per stage; this build
+    refuses it with a RuntimeError."""
 
     def __init__(self, jobs, zero_grads=True, persistent=False):
         L = _lib.lib()

@@ -137,7 +137,7 @@ struct SceneHost {
 
 // Batched renders (one kernel per stage over the jobs of many scenes).
 struct BatchHost;
-// flags: DVG_BATCH_ZERO_GRADS, DVG_BATCH_PERSISTENT
+// flags: DVG_BATCH_ZERO_GRADS (DVG_BATCH_PERSISTENT is refused)
 int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, int flags, BatchHost **out);
 int batch_render(BatchHost &b, hipStream_t st);
 int batch_status(BatchHost &b);

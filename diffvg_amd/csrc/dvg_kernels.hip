@@ -122,10 +122,6 @@ constexpr int64_t kPrimDirect = 12288;
 #ifndef DVG_WAVES_SDF
 #define DVG_WAVES_SDF 4
 #endif
-// the persistent batch kernel runs every stage in one launch, so one setting for all
-#ifndef DVG_WAVES_PERSIST
-#define DVG_WAVES_PERSIST 4
-#endif
 
 // Render geometry shared by the kernels.
 struct Geom {
@@ -138,9 +134,8 @@ struct Geom {
     int prim_direct;  // primitives' boundary adjoints are added sample by sample (kPrimDirect)
 };
 
-// Workgroup-shared storage of the tiled stages.  Each stage function takes its own
-// struct from the caller: the single-stage kernels declare one, the persistent batch
-// kernel overlays all of them in one union.
+// Workgroup-shared storage of the tiled stages, declared by the kernels and handed to the
+// stage functions.
 struct CandLds {
     int list[kCandCap];
     int w[kBlock / 64];
@@ -819,23 +814,13 @@ DVG_DEV int edge_sample_tile(const DevScene &S, const Geom &G, int idx, EdgeSamp
     }
     return -1;
 }
-// The count the atomic returns is the sample's position in the tile's bin, so binning
-// (edge_bin_one) needs no second round of atomics.
-DVG_DEV void edge_sample_one(const DevScene &S, const Geom &G, int idx, int count, EdgeSample *edges, int *edge_tile,
-                             int *edge_rank, int *tile_count) {
-    if (idx >= count) return;
-    EdgeSample es{};
-    const int tile = edge_sample_tile(S, G, idx, es);
-    edges[idx] = es;
-    edge_tile[idx] = tile;
-    edge_rank[idx] = tile >= 0 ? atomicAdd(&tile_count[tile], 1) : 0;
-}
-// The same for a workgroup of kSampleBlock samples, counted per tile in LDS first and added to
-// a tile's count at once: a scene of few shapes sends its samples to the few tiles on their
-// boundaries, whose counters would take one atomic per sample (12.7 ns each).  2048 strokes
-// at 512x512, 4 samples: 143 -> 97 us; a batch of 256 scenes of up to 512 paths at 28 to 256
-// pixels 2.8 -> 1.5 ms.  Canvases of
-// more tiles than the table holds (48 KB: two workgroups of 16 waves fill a CU) add per sample.
+// The boundary samples of a workgroup of kSampleBlock, their tiles and their positions in the
+// tiles' bins, so that binning (edge_bin_one) needs no second round of atomics.  They are counted
+// per tile in LDS first and added to a tile's count at once: a scene of few shapes sends its
+// samples to the few tiles on their boundaries, whose counters would take one atomic per sample
+// (12.7 ns each).  2048 strokes at 512x512, 4 samples: 143 -> 97 us; a batch of 256 scenes of up
+// to 512 paths at 28 to 256 pixels 2.8 -> 1.5 ms.  Canvases of more tiles than the table holds
+// (48 KB: two workgroups of 16 waves fill a CU) add per sample.
 constexpr int kSampleBlock = 1024;
 constexpr int kSampleTiles = 12288;
 DVG_DEV void edge_sample_block(int *s_count, const DevScene &S, const Geom &G, int block, int count, EdgeSample *edges,
@@ -2369,190 +2354,6 @@ __global__ __launch_bounds__(kBlock, DVG_WAVES_SDF) void kb_sdf(const Job *jobs,
         sdf_tile(L, J.S, J.G, blockIdx.x - pref[j], J.sdf, J.d_sdf, J.d_tr);
 }
 
-// ------------------------------------------------------------------ persistent batch kernel
-// One launch per batch render: a fixed grid of workgroups (as many as the device holds at
-// once) takes tasks -- (stage, job, workgroup of that stage) -- from a counter in HBM, in
-// a fixed order: stage by stage over all jobs, in the order of kPStage.  A task first
-// waits until the stages it depends on are done for its own job (per-job counters of
-// finished tasks), so a scene's resolve can start while other scenes still shade, and a
-// small scene's edge pass overlaps the colour passes of large ones.  Every dependency is
-// on a task earlier in the order, and a task is taken only by a running workgroup, so
-// every wait ends: the earliest unfinished task waits for nothing.  As a safeguard a wait
-// gives up after a time budget (the host reports it as an error); the results of such a
-// render are not defined.  The last workgroup to leave resets the counters for the next
-// launch, so the launch can be replayed from a HIP graph.
-//
-// DISABLED (batch_create refuses DVG_BATCH_PERSISTENT): the first GPU run of this kernel
-// (a batch of ten small mixed jobs) did not finish within three minutes, and neither its
-// dependency waits nor their time budget explain that on reading; the kernel is kept
-// for reference, not launched.
-enum PStage {
-    kPZero = 0,
-    kPWeight,
-    kPColor0,
-    kPColor1,
-    kPResolve,
-    kPColorBwd0,
-    kPColorBwd1,
-    kPEdgeSample,
-    kPScan,
-    kPEdgeBin,
-    kPEdge,
-    kPSdf,
-    kNumPStages
-};
-
-// stages whose tasks of the same job must be done first (bit masks of PStage)
-DVG_DEV uint32_t pstage_deps(int s) {
-    switch (s) {
-        case kPResolve: return (1u << kPWeight) | (1u << kPColor0) | (1u << kPColor1);
-        // gradients cleared; weights; the fragment lists the job's forward keeps
-        case kPColorBwd0: return (1u << kPZero) | (1u << kPWeight) | (1u << kPColor0);
-        case kPColorBwd1: return (1u << kPZero) | (1u << kPWeight) | (1u << kPColor1);
-        case kPEdgeSample: return 1u << kPZero;  // tile counts cleared
-        case kPScan: return 1u << kPEdgeSample;
-        case kPEdgeBin: return 1u << kPScan;
-        case kPEdge: return (1u << kPEdgeBin) | (1u << kPWeight) | (1u << kPZero);
-        case kPSdf: return 1u << kPZero;
-        default: return 0u;
-    }
-}
-
-// words of the task state ahead of the per-job counters
-enum { kPNext = 0, kPExited, kPAbort, kPStateInts = 4 };
-
-union PLds {
-    CandLds color;
-    ColorBwdLds bwd;
-    EdgeLds edge;
-    SdfLds sdf;
-    ScanLds<kBlock> scan;
-};
-
-// One lane waits for the task's prerequisites (`done` = the job's counters); false when
-// the render was given up (this or another wait exceeded the budget).
-DVG_DEV bool pstage_wait(const int *ppref, int nj, int j, int s, int *done, int *state, uint64_t budget) {
-    uint32_t deps = pstage_deps(s);
-    uint64_t t0 = 0;
-    while (deps) {
-        const int d = __builtin_ctz(deps);
-        deps &= deps - 1;
-        const int *pf = ppref + d * (nj + 1);
-        const int need = pf[j + 1] - pf[j];
-        while (need > 0 && __hip_atomic_load(done + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < need) {
-            if (__hip_atomic_load(state + kPAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) return false;
-            const uint64_t now = wall_clock64();
-            if (t0 == 0) {
-                t0 = now;
-            } else if (now - t0 > budget) {
-                atomicOr(state + kPAbort, 1);
-                return false;
-            }
-            __builtin_amdgcn_s_sleep(8);
-        }
-    }
-    __threadfence();  // acquire: what the finished tasks wrote is visible from here on
-    return __hip_atomic_load(state + kPAbort, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0;
-}
-
-DVG_DEV void run_pstage(PLds &L, const Job &J, int s, int b, int nb, int zero_grads) {
-    switch (s) {
-        case kPZero:
-            if (J.d_img && J.tile_count)
-                for (int i = b * kBlock + threadIdx.x; i < J.ntiles; i += nb * kBlock) J.tile_count[i] = 0;
-            if (zero_grads && (J.d_img || J.d_sdf))
-                for (int i = b * kBlock + threadIdx.x; i < J.grad_n; i += nb * kBlock) J.grad[i] = 0.f;
-            break;
-        case kPWeight: weight_pixel(J.S, J.G, b * kBlock + threadIdx.x, J.weight); break;
-        case kPColor0: color_tile<0>(L.color, J.S, J.G, b, J.bg, J.colors, J.err, J.frag, nullptr); break;
-        case kPColor1: color_tile<1>(L.color, J.S, J.G, b, J.bg, J.colors, J.err, nullptr, J.pkeep); break;
-        case kPResolve:
-            resolve_pixel(J.S, J.G, b * kBlock + threadIdx.x, J.pre, J.weight, J.colors, J.img);
-            break;
-        case kPColorBwd0:
-            color_bwd_tile<0>(L.bwd, J.S, J.G, b, J.bg, J.weight, J.d_img, J.d_bg, J.d_tr, J.err, J.frag, nullptr);
-            break;
-        case kPColorBwd1:
-            color_bwd_tile<1>(L.bwd, J.S, J.G, b, J.bg, J.weight, J.d_img, J.d_bg, J.d_tr, J.err, nullptr, J.pkeep);
-            break;
-        case kPEdgeSample:
-            edge_sample_one(J.S, J.G, b * kBlock + threadIdx.x, J.nsamp, J.edges, J.edge_tile, J.edge_rank,
-                            J.tile_count);
-            break;
-        case kPScan:
-            scan_tiles<kBlock>(L.scan, J.tile_count, J.tile_off, J.chunk_off, J.ntiles, J.G.echunk);
-            break;
-        case kPEdgeBin:
-            edge_bin_one(b * kBlock + threadIdx.x, J.nsamp, J.edge_tile, J.edge_rank, J.tile_off, J.edge_sorted);
-            break;
-        case kPEdge:
-            if (J.G.echunk == kBlock)
-                edge_chunk<true>(L.edge, J.S, J.G, b, J.edges, J.tile_off, J.tile_count, J.chunk_off, J.ntiles,
-                                 J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr);
-            else
-                edge_chunk<false>(L.edge, J.S, J.G, b, J.edges, J.tile_off, J.tile_count, J.chunk_off, J.ntiles,
-                                  J.edge_sorted, J.bg, J.weight, J.d_img, J.d_tr);
-            break;
-        case kPSdf:
-            if (J.eval)
-                sdf_sample(J.S, J.G, b * kBlock + threadIdx.x, J.eval, J.num_eval, J.sdf, J.d_sdf, J.d_tr);
-            else
-                sdf_tile(L.sdf, J.S, J.G, b, J.sdf, J.d_sdf, J.d_tr);
-            break;
-        default: break;
-    }
-}
-
-// ppref[s * (nj + 1) + k]: first task of job k within stage s; pbase[s]: first task of
-// stage s (pbase[kNumPStages] = all tasks); state: kPStateInts words, then the
-// per-job counters done[j * kNumPStages + s].
-__global__ __launch_bounds__(kBlock, DVG_WAVES_PERSIST) void kb_persist(const Job *jobs, int nj, const int *ppref,
-                                                                       const int *pbase, int *state, int zero_grads,
-                                                                       uint64_t budget) {
-    __shared__ PLds L;
-    __shared__ int s_task;
-    __shared__ int s_go;
-    __shared__ int s_last;
-    int *done = state + kPStateInts;
-    const int total = pbase[kNumPStages];
-    for (;;) {
-        if (threadIdx.x == 0) s_task = atomicAdd(state + kPNext, 1);
-        __syncthreads();
-        const int t = __builtin_amdgcn_readfirstlane(s_task);
-        if (t >= total) break;
-        int s = 0;
-        while (pbase[s + 1] <= t) s++;
-        const int *pf = ppref + s * (nj + 1);
-        const int local = t - pbase[s];
-        const int j = __builtin_amdgcn_readfirstlane(find_job(pf, nj, local));
-        const int b = local - pf[j], nb = pf[j + 1] - pf[j];
-        // a render given up skips its remaining tasks (their inputs may not be there)
-        if (threadIdx.x == 0) s_go = pstage_wait(ppref, nj, j, s, done + j * kNumPStages, state, budget) ? 1 : 0;
-        __syncthreads();
-        if (__builtin_amdgcn_readfirstlane(s_go)) run_pstage(L, jobs[j], s, b, nb, zero_grads);
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            __threadfence();  // release: this task's writes before its count
-            atomicAdd(done + j * kNumPStages + s, 1);
-        }
-    }
-    // the last workgroup out clears the counters for the next launch
-    if (threadIdx.x == 0) {
-        __threadfence();
-        s_last = atomicAdd(state + kPExited, 1) == (int)gridDim.x - 1;
-    }
-    __syncthreads();
-    if (s_last) {
-        __threadfence();
-        for (int i = threadIdx.x; i < nj * kNumPStages; i += blockDim.x) done[i] = 0;
-        if (threadIdx.x == 0) {
-            state[kPNext] = 0;
-            state[kPExited] = 0;
-        }
-        __threadfence();
-    }
-}
-
 struct BatchHost {
     int device = 0;
     int n = 0;
@@ -2573,11 +2374,6 @@ struct BatchHost {
     size_t ws_bytes = 0, ws_granted = 0;
     hipStream_t last_stream = nullptr;
     std::vector<SceneHost *> keep_holds;  // one entry per job holding its scene's kept lists
-    // persistent launch (DVG_BATCH_PERSISTENT): task prefix arrays and state in dev_block
-    bool persistent = false;
-    size_t ppref_off = 0, pbase_off = 0, pstate_off = 0;
-    int ptotal = 0, pgrid = 0;
-    uint64_t pbudget = 0;
 };
 
 static size_t al256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -2589,10 +2385,9 @@ int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, i
     std::unique_ptr<BatchHost> guard(B);
     B->n = n;
     B->zero_grads = (flags & DVG_BATCH_ZERO_GRADS) ? 1 : 0;
-    B->persistent = (flags & DVG_BATCH_PERSISTENT) != 0;
-    // Switched off: its first GPU run did not finish (see kb_persist); the cause is not
-    // known, so the launch is refused rather than risked.
-    if (B->persistent)
+    // One launch whose workgroups took the items from a device queue: its first GPU run did not
+    // finish, the cause is not known, and it is no longer here.
+    if (flags & DVG_BATCH_PERSISTENT)
         return set_error("DVG_BATCH_PERSISTENT is disabled in this build: the persistent batch kernel did not "
                          "finish on the GPU and the cause is not known; use the one-launch-per-stage batch");
     B->device = scenes[0]->device;
@@ -2749,42 +2544,6 @@ int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, i
             B->total[c * kNumStages + st] = acc;
         }
     }
-    // persistent launch: task counts per (stage, job) over all jobs
-    std::vector<int> ppref, pbase;
-    if (B->persistent) {
-        auto ptasks = [&](const Job &J, int stage) -> int {
-            bool color = J.img || J.d_img, edges = J.d_img && !J.pre, sdf = J.sdf || J.d_sdf;
-            switch (stage) {
-                case kPZero: return blocks(J, kStZero);
-                case kPWeight: return color ? (J.npix + kBlock - 1) / kBlock : 0;
-                case kPColor0: return J.img && !J.pre ? J.ntiles : 0;
-                case kPColor1: return J.img && J.pre ? J.ntiles : 0;
-                case kPResolve: return J.img ? (J.npix + kBlock - 1) / kBlock : 0;
-                case kPColorBwd0: return J.d_img && !J.pre ? J.ntiles : 0;
-                case kPColorBwd1: return J.d_img && J.pre ? J.ntiles : 0;
-                case kPEdgeSample:
-                case kPEdgeBin: return edges ? (J.nsamp + kBlock - 1) / kBlock : 0;
-                case kPScan: return edges ? 1 : 0;
-                case kPEdge: return edges ? J.ntiles + (J.nsamp + J.G.echunk - 1) / J.G.echunk : 0;
-                case kPSdf: return sdf ? (J.eval ? (J.num_eval + kBlock - 1) / kBlock : J.ntiles) : 0;
-                default: return 0;
-            }
-        };
-        int64_t acc_all = 0;
-        for (int st = 0; st < kNumPStages; st++) {
-            pbase.push_back((int)acc_all);
-            int acc = 0;
-            for (int k = 0; k < n; k++) {
-                ppref.push_back(acc);
-                acc += ptasks(B->jobs[k], st);
-            }
-            ppref.push_back(acc);
-            acc_all += acc;
-        }
-        if (acc_all > (int64_t)0x7fffffff - 4 * 65536) return set_error("too many tasks for one persistent batch");
-        pbase.push_back((int)acc_all);
-        B->ptotal = (int)acc_all;
-    }
     B->scenes.assign(scenes, scenes + n);
     int prev = -1;
     (void)hipGetDevice(&prev);
@@ -2797,24 +2556,6 @@ int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, i
     // whole device)
     size_t jbytes = al256(sizeof(Job) * n);
     B->dev_bytes = jbytes + al256(B->pref.size() * sizeof(int));
-    if (B->persistent) {
-        B->ppref_off = B->dev_bytes;
-        B->dev_bytes += al256(ppref.size() * sizeof(int));
-        B->pbase_off = B->dev_bytes;
-        B->dev_bytes += al256(pbase.size() * sizeof(int));
-        B->pstate_off = B->dev_bytes;  // zeroed below with the rest of the block
-        B->dev_bytes += al256((size_t)(kPStateInts + n * kNumPStages) * sizeof(int));
-        int per_cu = 0, cus = 0, rate_khz = 0;
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kb_persist, kBlock, 0) != hipSuccess ||
-            hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, B->device) != hipSuccess ||
-            hipDeviceGetAttribute(&rate_khz, hipDeviceAttributeWallClockRate, B->device) != hipSuccess) {
-            if (prev >= 0 && prev != B->device) (void)hipSetDevice(prev);
-            return set_error("persistent batch: device query failed");
-        }
-        B->pgrid = std::max(1, std::min(B->ptotal, std::max(1, per_cu) * std::max(1, cus)));
-        // a dependency wait gives up after 20 s of wall clock (a render takes milliseconds)
-        B->pbudget = (uint64_t)std::max(rate_khz, 1) * 1000ull * 20ull;
-    }
     B->dev_block = cache_alloc(B->device, B->dev_bytes, &B->dev_granted);
     if (!B->dev_block) {
         restore();
@@ -2848,10 +2589,6 @@ int batch_create(SceneHost *const *scenes, const dvg_render_args *args, int n, i
     std::vector<uint8_t> host(B->dev_bytes, 0);
     std::memcpy(host.data(), B->jobs.data(), sizeof(Job) * n);
     std::memcpy(host.data() + jbytes, B->pref.data(), B->pref.size() * sizeof(int));
-    if (B->persistent) {
-        std::memcpy(host.data() + B->ppref_off, ppref.data(), ppref.size() * sizeof(int));
-        std::memcpy(host.data() + B->pbase_off, pbase.data(), pbase.size() * sizeof(int));
-    }
     int rc = upload(B->device, B->dev_block, host.data(), B->dev_bytes);
     restore();
     if (rc) {
@@ -2869,15 +2606,6 @@ int batch_render(BatchHost &B, hipStream_t st) {
     if (prev != B.device) (void)hipSetDevice(B.device);
     const Job *jobs = (const Job *)B.dev_block;
     const int *pref_base = (const int *)((uint8_t *)B.dev_block + al256(sizeof(Job) * B.n));
-    if (B.persistent) {
-        if (B.ptotal > 0) {
-            DVG_PROF(st, "kb_persist");
-            uint8_t *base = (uint8_t *)B.dev_block;
-            kb_persist<<<(unsigned)B.pgrid, kBlock, 0, st>>>(jobs, B.n, (const int *)(base + B.ppref_off),
-                                                             (const int *)(base + B.pbase_off),
-                                                             (int *)(base + B.pstate_off), B.zero_grads, B.pbudget);
-        }
-    } else
     for (int c = 0; c < 3; c++) {
         int j0 = B.cls_begin[c], nj = B.cls_begin[c + 1] - j0;
         if (nj == 0) continue;
@@ -2946,20 +2674,6 @@ int batch_status(BatchHost &B) {
     // render conditions accumulate in each scene's word until read: read and clear them,
     // as dvg_scene_status does (a forward batch's findings are still there when its
     // backward batch has run)
-    if (B.persistent) {
-        int abort_word = 0;
-        int *state = (int *)((uint8_t *)B.dev_block + B.pstate_off);
-        DVG_CHECK(hipMemcpyAsync(&abort_word, state + kPAbort, sizeof(int), hipMemcpyDeviceToHost, B.last_stream));
-        DVG_CHECK(hipStreamSynchronize(B.last_stream));
-        if (abort_word) {
-            // the launch's last workgroup reset the task counters; clear the flag too
-            DVG_CHECK(hipMemsetAsync(state + kPAbort, 0, sizeof(int), B.last_stream));
-            DVG_CHECK(hipStreamSynchronize(B.last_stream));
-            if (prev >= 0 && prev != B.device) (void)hipSetDevice(prev);
-            return set_error("persistent batch: a task waited longer than its time limit for the tasks it depends "
-                             "on; the batch's results are not defined");
-        }
-    }
     int flags[2] = {0, 0};
     for (auto *sc : B.scenes) {
         int h[2] = {0, 0};
