@@ -83,6 +83,7 @@ def lib():
     L.dvg_render_noalloc.argtypes = [ctypes.c_void_p, ctypes.POINTER(RenderArgs)]
     L.dvg_scene_get_grads.argtypes = [ctypes.c_void_p, ctypes.POINTER(Grads)]
     L.dvg_scene_zero_grads.argtypes = [ctypes.c_void_p, ctypes.c_void_p]
+    L.dvg_scene_samples_per_wave_matters.argtypes = [ctypes.c_void_p] + [ctypes.c_int] * 4 + [ctypes.POINTER(ctypes.c_int)]
     L.dvg_scene_set_mode.argtypes = [ctypes.c_void_p, ctypes.c_int]
     L.dvg_scene_set_tiling.argtypes = [ctypes.c_void_p, ctypes.c_int]
     L.dvg_scene_set_samples_per_wave.argtypes = [ctypes.c_void_p, ctypes.c_int]
@@ -153,6 +154,12 @@ class DeviceScene:
 
     def set_samples_per_wave(self, edge_samples_per_wave):
         check(self._lib.dvg_scene_set_samples_per_wave(self.handle, int(edge_samples_per_wave)))
+
+    def samples_per_wave_matters(self, width, height, nsx, nsy):
+        out = ctypes.c_int()
+        check(self._lib.dvg_scene_samples_per_wave_matters(self.handle, int(width), int(height), int(nsx), int(nsy),
+                                                           ctypes.byref(out)))
+        return bool(out.value)
 
     @staticmethod
     def make_args(width, height, nsx, nsy, seed, background=None, render_image=None, render_sdf=None,

@@ -7,14 +7,15 @@ order:
   aspect and how the four wavefronts of a workgroup cover it (pixel rows in order).
   Wider tiles keep a wave's samples in fewer rows, narrower ones in fewer columns; which
   candidate lists are shortest and which waves diverge least depends on the scene;
-* the boundary samples per wave of the edge kernel: 32 (each lane shades one of the
-  two colour queries of a sample, so a lane keeps one compositor live) or 64 (each lane
-  shades both, with twice the state but half the lanes).
+* the boundary samples per wave of the per-lane edge kernel: 32 (each lane shades one of
+  the two colour queries of a sample, so a lane keeps one compositor live) or 64 (each lane
+  shades both, with twice the state but half the lanes).  Renders that take the
+  wave-cooperative edge kernel have no such choice, and only the widths are timed.
 
 `tune` times one forward + backward per (width, samples per wave) on the caller's scene
 (HIP events on the current stream) and remembers the fastest per workload signature --
-render size bucket, samples per pixel, group-count bucket, prefiltering -- so later
-scenes of the same kind reuse it without timing.
+render size bucket, samples per pixel, group-count bucket, prefiltering, edge kernel -- so
+later scenes of the same kind reuse it without timing.
 
 Per batch (`Tuner.tune_batch`): one launch per stage or one persistent launch
 (`Batch(persistent=...)`), timed on the caller's batches; a structure the library
@@ -57,9 +58,10 @@ class Tuner:
         self.timings = {}
         self.batch_timings = {}
 
-    def candidates(self, spp, prefilter=False):
+    def candidates(self, spp, prefilter=False, edge_choice=True):
         """(tile width, edge samples per wave) pairs to time.  Prefiltered renders have no
-        edge pass, so only the width varies for them."""
+        edge pass, and the wave-cooperative edge kernel (edge_choice False) no such setting, so
+        only the width varies for them."""
         px = max(1, 256 // spp)
         out, tw = [], 1
         while tw <= px:
@@ -68,7 +70,7 @@ class Tuner:
             tw *= 2
         # drop the extreme slivers
         widths = [t for t in out if px // t >= 2 or t == out[-1]][-6:]
-        spws = (32,) if prefilter else EDGE_SAMPLES_PER_WAVE
+        spws = EDGE_SAMPLES_PER_WAVE if edge_choice and not prefilter else (32,)
         return [(tw, spw) for tw in widths for spw in spws]
 
     @staticmethod
@@ -77,11 +79,18 @@ class Tuner:
         scene.set_tiling(tw)
         scene.set_samples_per_wave(spw)
 
+    @staticmethod
+    def _key(scene, width, height, nsx, nsy, num_groups, prefilter):
+        """(key of `best`, whether the edge samples per wave matter)"""
+        choice = scene.samples_per_wave_matters(width, height, nsx, nsy)
+        key = signature(width, height, nsx, nsy, num_groups, prefilter)
+        return (key if choice else key + ('wave',)), choice
+
     def tune(self, scene, width, height, nsx, nsy, seed=0, prefilter=False, num_groups=None):
         """Times each candidate on `scene` (one forward + backward each), sets the fastest
         and returns it as (tile width, edge samples per wave)."""
         ng = num_groups if num_groups is not None else scene.flat['num_groups']
-        key = signature(width, height, nsx, nsy, ng, prefilter)
+        key, edge_choice = self._key(scene, width, height, nsx, nsy, ng, prefilter)
         if key in self.best:
             self._set(scene, self.best[key])
             return self.best[key]
@@ -97,7 +106,7 @@ class Tuner:
             scene.render(width, height, nsx, nsy, seed, d_render_image=d_img, use_prefiltering=prefilter, stream=st)
 
         res = {}
-        for choice in self.candidates(nsx * nsy, prefilter):
+        for choice in self.candidates(nsx * nsy, prefilter, edge_choice):
             self._set(scene, choice)
             res[choice] = _time_ms(step, self.reps)
         best = min(res, key=res.get)
@@ -108,7 +117,7 @@ class Tuner:
 
     def apply(self, scene, width, height, nsx, nsy, prefilter=False):
         """Sets the remembered choice for this workload signature, if any."""
-        key = signature(width, height, nsx, nsy, scene.flat['num_groups'], prefilter)
+        key, _ = self._key(scene, width, height, nsx, nsy, scene.flat['num_groups'], prefilter)
         if key in self.best:
             self._set(scene, self.best[key])
             return self.best[key]

@@ -741,6 +741,15 @@ int dvg_scene_set_samples_per_wave(dvg_scene *scene, int edge_samples_per_wave) 
     return 0;
 }
 
+int dvg_scene_samples_per_wave_matters(dvg_scene *scene, int width, int height, int num_samples_x, int num_samples_y,
+                                       int *matters) {
+    if (!scene || !matters) return set_error("null argument");
+    if (width <= 0 || height <= 0 || num_samples_x <= 0 || num_samples_y <= 0)
+        return set_error("width, height and sample counts must be positive");
+    *matters = !edge_by_wave(scene->h, (int64_t)width * height * num_samples_x * num_samples_y);
+    return 0;
+}
+
 int dvg_scene_set_mode(dvg_scene *scene, int mode) {
     if (!scene) return set_error("null scene");
     if (mode != DVG_MODE_TILED && mode != DVG_MODE_PLAIN) return set_error("unknown render mode");

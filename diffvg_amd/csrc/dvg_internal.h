@@ -148,6 +148,8 @@ int build_scene(const dvg_scene_desc &d, int gpu_index, SceneHost &sc);
 int update_scene(SceneHost &sc, const dvg_scene_params &p, float filter_radius, hipStream_t st);
 int scene_status(SceneHost &sc);
 void free_scene(SceneHost &sc);
+// whether a TILED render of this size takes the wave-cooperative edge kernel
+bool edge_by_wave(const SceneHost &sc, int64_t samples);
 // `fixed`: a workspace the caller carved (the allocation-free entry point); the render
 // then neither grows a workspace nor keeps fragment lists for its backward.
 int render_tiled(SceneHost &sc, const dvg_render_args &a, Workspace *fixed = nullptr);

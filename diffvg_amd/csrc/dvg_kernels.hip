@@ -1711,6 +1711,15 @@ void Workspace::release() {
     npix_cap = nsamp_cap = ntiles_cap = 0;
 }
 
+static bool prim_direct(const SceneHost &sc, int64_t samples) { return samples > kPrimDirect * sc.num_shapes; }
+// Circles and ellipses past kPrimDirect keep the per-lane kernel: their adds one by one are
+// its time (one circle at 256x256, 4 samples: 10.0 ms either way), and the order in which
+// its workgroups make them is what those sums of up to 10^5 and more terms of both signs
+// round to (the wave kernel's order moves them by up to 9e-5, two runs of this one by 2e-5).
+bool edge_by_wave(const SceneHost &sc, int64_t samples) {
+    return sc.dev.wave_ok && !(sc.round_shapes && prim_direct(sc, samples));
+}
+
 static Geom make_geom(const SceneHost &sc, const dvg_render_args &a) {
     Geom G;
     G.W = a.width;
@@ -1729,13 +1738,8 @@ static Geom make_geom(const SceneHost &sc, const dvg_render_args &a) {
     if (th < 1) th = 1;
     G.tw = tw;
     G.th = th;
-    G.prim_direct = (int64_t)G.W * G.H * G.spp > kPrimDirect * sc.num_shapes;
-    // Circles and ellipses past kPrimDirect keep the per-lane kernel: their adds one by one are
-    // its time (one circle at 256x256, 4 samples: 10.0 ms either way), and the order in which
-    // its workgroups make them is what those sums of up to 10^5 and more terms of both signs
-    // round to (the wave kernel's order moves them by up to 9e-5, two runs of this one by 2e-5).
-    const bool wave = sc.dev.wave_ok && !(G.prim_direct && sc.round_shapes);
-    G.echunk = wave ? kWaveChunk : (sc.edge_spw == 64 ? kBlock : kEdgeChunk);
+    G.prim_direct = prim_direct(sc, (int64_t)G.W * G.H * G.spp);
+    G.echunk = edge_by_wave(sc, (int64_t)G.W * G.H * G.spp) ? kWaveChunk : (sc.edge_spw == 64 ? kBlock : kEdgeChunk);
     G.tiles_x = (G.W + tw - 1) / tw;
     G.tiles_y = (G.H + th - 1) / th;
     G.sx_scale = (float)sc.cw / (float)G.W;

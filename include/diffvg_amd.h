@@ -169,6 +169,10 @@ int dvg_scene_set_tiling(dvg_scene *scene, int tile_width);
  * tested at once), which it does not change.  Picked by the autotuner; results do not
  * depend on it beyond float summation order.  No reference counterpart. */
 int dvg_scene_set_samples_per_wave(dvg_scene *scene, int edge_samples_per_wave);
+/* Whether that setting changes the edge kernel of a TILED render of this size: `matters`
+ * receives 1, or 0 when the render takes the wave-cooperative kernel. */
+int dvg_scene_samples_per_wave_matters(dvg_scene *scene, int width, int height, int num_samples_x, int num_samples_y,
+                                       int *matters);
 
 /* Device-resident parameter values of a scene: DEVICE pointers on the scene's GPU, in the
  * layout of the float arrays of dvg_scene_desc (points as x,y pairs; thickness 0 where a

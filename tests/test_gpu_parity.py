@@ -415,3 +415,21 @@ def test_autotuner_picks_a_candidate():
     assert best in t.candidates(4)
     assert {spw for _, spw in t.candidates(4)} == {32, 64}
     assert t.apply(_lib.DeviceScene(f, 0), 64, 64, 2, 2) == best
+
+
+@pytest.mark.parametrize('case, spws', [('overlap_eo', {32}), ('transformed', {32, 64}), ('quad_approx', {32, 64}),
+                                        ('single_circle_64', {32, 64})])
+def test_autotuner_times_only_what_the_scene_takes(case, spws):
+    """Scenes of one shape per group run the wave-cooperative edge kernel, which has no samples
+    per wave to choose; two shapes in a group, approximated quadratics and a circle of many
+    samples do.  Neither kind uses the other's choice."""
+    from diffvg_amd.autotune import Tuner
+    print('autotuner', case, flush=True)
+    sc = _lib.DeviceScene(scenes.flat_case(case), 0)
+    t = Tuner(reps=1)
+    t.tune(sc, 64, 64, 2, 2, num_groups=4)
+    (timed,) = t.timings.values()
+    assert {spw for _, spw in timed} == spws
+    other = _lib.DeviceScene(scenes.flat_case('strokes' if spws == {32, 64} else 'transformed'), 0)
+    t.tune(other, 64, 64, 2, 2, num_groups=4)
+    assert len(t.best) == 2
