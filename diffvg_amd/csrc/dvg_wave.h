@@ -187,17 +187,13 @@ DVG_DEV void wave_screen(const SceneRef &R, WaveLds<SIDES> &W, int &n1, int &n2,
                         rmax = fmaxf(fmaxf(fabsf(r0), fabsf(S.thickness[idx.y])),
                                      fmaxf(fabsf(S.thickness[idx.z]), fabsf(r3)));
                     }
-                    const V2 p0{q.x[0], q.y[0]}, p3{q.x[8], q.y[8]};
                     bool hit;
                     float reach = 0.f;
                     if constexpr (SIDES == 2) {
-                        // within both points' reach of an end of the curve, with a margin for
-                        // rounding
                         reach = hx + hy;
-                        const float less = reach + 1e-4f * (fmaxf(q.mc, fmaxf(fabsf(pt.x), fabsf(pt.y))) + 1.f);
-                        const float c0 = r0 - less, c3 = r3 - less;
-                        hit = (c0 > 0.f && dist_sq(p0, pt) < c0 * c0) || (c3 > 0.f && dist_sq(p3, pt) < c3 * c3);
+                        hit = wf::stroke_ends_within(q, pt.x, pt.y, r0, r3, reach);
                     } else {
+                        const V2 p0{q.x[0], q.y[0]}, p3{q.x[8], q.y[8]};
                         hit = dist_sq(p0, pt) < r0 * r0 || dist_sq(p3, pt) < r3 * r3;
                     }
                     if (hit) {

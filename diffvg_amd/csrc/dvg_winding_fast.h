@@ -277,6 +277,15 @@ DVG_WF bool stroke_farther(const StrokePrep &q, float ptx, float pty, float rmax
     return far;
 }
 
+// Every point within `reach` of pt lies within the stroke's radius (r0, r3) of one and the same end
+// of the curve, with a margin for rounding (the other half of a decision for a whole box).
+DVG_WF bool stroke_ends_within(const StrokePrep &q, float ptx, float pty, float r0, float r3, float reach) {
+    const float less = reach + 1e-4f * (fmaxf(q.mc, fmaxf(fabsf(ptx), fabsf(pty))) + 1.f);
+    const float c0 = r0 - less, c3 = r3 - less;
+    const float ux = ptx - q.x[0], uy = pty - q.y[0], vx = ptx - q.x[8], vy = pty - q.y[8];
+    return (c0 > 0.f && ux * ux + uy * uy < c0 * c0) || (c3 > 0.f && vx * vx + vy * vy < c3 * c3);
+}
+
 DVG_WF bool cubic_certainly_farther(float p0x, float p0y, float p1x, float p1y, float p2x, float p2y, float p3x,
                                     float p3y, float ptx, float pty, float rmax) {
     return stroke_farther(stroke_prep(p0x, p0y, p1x, p1y, p2x, p2y, p3x, p3y), ptx, pty, rmax);

@@ -45,17 +45,34 @@ def test_fast_cubic_stroke_rejection_never_disagrees(mode, min_decided):
     assert out[0] / out[2] >= min_decided
 
 
-@pytest.mark.parametrize('near, min_decided', [(0, 0.9), (1, 0.25)])
-def test_fast_cubic_winding_holds_over_a_box(near, min_decided):
+@pytest.mark.parametrize('near, full, min_decided', [(0, 0, 0.9), (1, 0, 0.05), (0, 1, 0.9), (1, 1, 0.25)])
+def test_fast_cubic_winding_holds_over_a_box(near, full, min_decided):
     """With half widths the test decides for every point of a box at once (the two sides of a
-    boundary sample): the oracle agrees at the box's corners and at points inside it."""
+    boundary sample): the oracle agrees at the box's corners and at points inside it.  The
+    renderer takes the short form (full 0) for boxes."""
     if not os.path.exists(SO):
         pytest.skip('tests/csrc not built (make -C tests/csrc)')
     L = ctypes.CDLL(SO)
-    L.wf_fuzz_box.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_uint64, ctypes.POINTER(ctypes.c_int64),
-                              ctypes.POINTER(ctypes.c_float)]
+    L.wf_fuzz_box.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_uint64,
+                              ctypes.POINTER(ctypes.c_int64), ctypes.POINTER(ctypes.c_float)]
     out = (ctypes.c_int64 * 3)()
     bad = (ctypes.c_float * 10)()
-    L.wf_fuzz_box(near, 300000, 500 + near, out, bad)
+    L.wf_fuzz_box(near, full, 300000, 500 + near, out, bad)
     assert out[1] == 0, ('mismatch', list(bad))
     assert out[0] / out[2] >= min_decided
+
+
+@pytest.mark.parametrize('mode', [0, 1, 2, 3])
+def test_fast_stroke_decisions_hold_over_a_box(mode):
+    """The decisions that a stroke covers, or does not, every point of a box: the oracle's
+    within-distance test agrees at its corners and inside it."""
+    if not os.path.exists(SO):
+        pytest.skip('tests/csrc not built (make -C tests/csrc)')
+    L = ctypes.CDLL(SO)
+    L.wf_stroke_box_fuzz.argtypes = [ctypes.c_int, ctypes.c_int64, ctypes.c_uint64, ctypes.POINTER(ctypes.c_int64),
+                                     ctypes.POINTER(ctypes.c_float)]
+    out = (ctypes.c_int64 * 4)()
+    bad = (ctypes.c_float * 10)()
+    L.wf_stroke_box_fuzz(mode, 150000, 900 + mode, out, bad)
+    assert out[2] == 0, ('mismatch', list(bad))
+    assert min(out[0], out[1]) >= 0.05 * out[3], list(out)
