@@ -76,3 +76,19 @@ def test_boundary_samples_of_canvases_around_the_count_table(h):
     group = pd.ShapeGroup(shape_ids=torch.tensor([0]), fill_color=torch.tensor([0.3, 0.6, 0.3, 0.7]),
                           stroke_color=torch.tensor([0.9, 0.2, 0.1, 0.8]))
     _check([path], [group], 2, h, 1, 1, False)
+
+
+@pytest.mark.parametrize('h, direct', [(96, False), (97, True)])
+def test_primitives_on_both_sides_of_the_direct_line(h, direct):
+    """Boundary adjoints of primitives are combined up to 12,288 samples per shape, added one by
+    one past it: 3 shapes, 4 samples a pixel, 96 x 96 (the line) and 96 x 97."""
+    print('primitives at the line', h, flush=True)
+    shapes = [pd.Circle(radius=torch.tensor(20.0), center=torch.tensor([30.0, 34.0]), stroke_width=torch.tensor(2.0)),
+              pd.Ellipse(radius=torch.tensor([24.0, 12.0]), center=torch.tensor([60.0, 60.0])),
+              pd.Rect(p_min=torch.tensor([40.0, 10.0]), p_max=torch.tensor([80.0, 44.0]),
+                      stroke_width=torch.tensor(1.5))]
+    groups = [pd.ShapeGroup(shape_ids=torch.tensor([i]), fill_color=torch.tensor([0.2 + 0.3 * i, 0.7, 0.4, 0.6]),
+                            stroke_color=None if i == 1 else torch.tensor([0.1, 0.2, 0.9, 0.8])) for i in range(3)]
+    f = flatten(96, h, shapes, groups, 0, 0.5)
+    assert GpuRunner(f).scene.samples_per_wave_matters(96, h, 2, 2) == direct
+    _check(shapes, groups, 96, h, 2, 2, False)

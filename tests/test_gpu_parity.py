@@ -384,11 +384,14 @@ def test_gpu_tile_shape_does_not_change_results(case):
             assert _rel(gg[k], ref_g[k]) <= 1e-4, (tw, k)
 
 
-@pytest.mark.parametrize('case', ['strokes', 'overlap_nz', 'gradients'])
+@pytest.mark.parametrize('case', ['strokes', 'overlap_nz', 'gradients', 'transformed', 'quad_approx',
+                                  'single_circle_64'])
 def test_gpu_edge_samples_per_wave_does_not_change_results(case):
     """The autotuner's second knob (boundary samples per wave of the edge kernel: one or
     both colour queries of a sample per lane) changes only float summation order, also
-    combined with non-square tiles; forward images are untouched by it."""
+    combined with non-square tiles; forward images are untouched by it.  It acts on the last
+    three cases (two shapes in a group, approximated quadratics, a circle of many samples);
+    the others take the wave-cooperative kernel whatever it says."""
     f = scenes.flat_case(case)
     w, h = f['canvas_width'], f['canvas_height']
     d = np.random.default_rng(7).uniform(-1, 1, (h, w, 4)).astype(np.float32)
@@ -433,3 +436,32 @@ def test_autotuner_times_only_what_the_scene_takes(case, spws):
     other = _lib.DeviceScene(scenes.flat_case('strokes' if spws == {32, 64} else 'transformed'), 0)
     t.tune(other, 64, 64, 2, 2, num_groups=4)
     assert len(t.best) == 2
+
+
+@pytest.mark.parametrize('spw', [32, 64])
+def test_batched_per_lane_edge_kernels_match_oracle(spw):
+    """kb_edge in both forms: the scenes that do not take the wave-cooperative kernel, in one
+    batch."""
+    from diffvg_amd.batch import Batch
+    print('batched edge kernels', spw, flush=True)
+    cases = ['transformed', 'quad_approx', 'single_circle_64']
+    rng = np.random.default_rng(8)
+    jobs, want, scs = [], [], []
+    for k, case in enumerate(cases):
+        f = scenes.flat_case(case)
+        w, h = f['canvas_width'], f['canvas_height']
+        d = rng.uniform(-1, 1, (h, w, 4)).astype(np.float32)
+        want.append(OracleRunner(f).render(w, h, 2, 2, 3 + k, d_image=d)['grads'])
+        sc = _lib.DeviceScene(f, 0)
+        assert sc.samples_per_wave_matters(w, h, 2, 2)
+        sc.set_samples_per_wave(spw)
+        scs.append(sc)
+        jobs.append((sc, dict(width=w, height=h, nsx=2, nsy=2, seed=3 + k,
+                              d_render_image=torch.from_numpy(d).to('cuda:0'))))
+    b = Batch(jobs)
+    b.render(None)
+    b.status()
+    for case, sc, o in zip(cases, scs, want):
+        g = sc.grads()
+        for k in GRAD_KEYS:
+            assert _rel(g[k], o[k]) <= 1e-3, (case, k)
