@@ -291,10 +291,10 @@ DVG_DEV bool within_at(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float t, float r0, flo
 // 0 or 1; 2: the coefficients are large and the plain search decides
 static __device__ __noinline__ int cubic_stroke_fast(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2,
                                                      float r3) {
-    const Quintic q = cubic_quintic(quintic_sums(p0, p1, p2, p3, pt));
-    if (quintic_large(q)) return 2;
+    const QuinticSums u = quintic_sums(p0, p1, p2, p3, pt);
+    if (quintic_large(u)) return 2;
     bool hit = false;
-    quintic_search(q, [&](float t) { return hit = within_at(p0, p1, p2, p3, pt, t, r0, r1, r2, r3); });
+    quintic_search(cubic_quintic(u), [&](float t) { return hit = within_at(p0, p1, p2, p3, pt, t, r0, r1, r2, r3); });
     return hit;
 }
 static __device__ __noinline__ bool cubic_stroke_plain(const float4 *src, V2 pt, float r0, float r1, float r2, float r3) {
@@ -494,41 +494,58 @@ struct CubicClosest {
     float dist, t;
     V2 pt;
 };
-DVG_DEV CubicClosest closest_end(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
-    V2 pt0 = ceval(p0, p1, p2, p3, 0), pt1 = ceval(p0, p1, p2, p3, 1);
+DVG_DEV CubicClosest closest_end(const CubicPoints &p, V2 pt) {
+    V2 pt0 = ceval(p.p0, p.p1, p.p2, p.p3, 0), pt1 = ceval(p.p0, p.p1, p.p2, p.p3, 1);
     float d0 = dist(pt0, pt), d1 = dist(pt1, pt);
     return d1 < d0 ? CubicClosest{d1, 1.f, pt1} : CubicClosest{d0, 0.f, pt0};
 }
-DVG_DEV bool closer_at(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float t, CubicClosest &r) {
-    V2 pp = ceval(p0, p1, p2, p3, t);
-    float dp = dist(pp, pt);
-    if (dp < r.dist) r = CubicClosest{dp, t, pp};
-    return false;
-}
 // t = -1: the coefficients are large and the plain search decides
-static __device__ __noinline__ CubicClosest cubic_closest_fast(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt) {
-    const Quintic q = cubic_quintic(quintic_sums(p0, p1, p2, p3, pt));
-    if (quintic_large(q)) return CubicClosest{0.f, -1.f, pt};
-    CubicClosest r = closest_end(p0, p1, p2, p3, pt);
-    quintic_search(q, [&](float t) { return closer_at(p0, p1, p2, p3, pt, t, r); });
+static __device__ __noinline__ CubicClosest cubic_closest_fast(const float4 *src, V2 pt) {
+    const CubicPoints p = cubic_points(src);
+    const QuinticSums u = quintic_sums(p.p0, p.p1, p.p2, p.p3, pt);
+    CubicClosest r = closest_end(p, pt);
+    if (quintic_large(u))
+        r.t = -1.f;
+    else
+        quintic_search(cubic_quintic(u), [&](float t) {
+            V2 pp = ceval(p.p0, p.p1, p.p2, p.p3, t);
+            float dp = dist(pp, pt);
+            if (dp < r.dist) r = CubicClosest{dp, t, pp};
+            return false;
+        });
     return r;
 }
-static __device__ __noinline__ CubicClosest cubic_closest_plain(const float4 *src, V2 pt) {
-    CubicClosest r{0.f, -1.f, pt};
-    plain_search(src, pt, [&](const CubicPoints &p, float t) {
-        if (r.t < 0.f) r = closest_end(p.p0, p.p1, p.p2, p.p3, pt);
-        return closer_at(p.p0, p.p1, p.p2, p.p3, pt, t, r);
+// the closest point's t
+static __device__ __noinline__ float cubic_closest_plain(const float4 *src, V2 pt) {
+    float t = -1.f, d = 0.f;
+    plain_search(src, pt, [&](const CubicPoints &p, float tj) {
+        if (t < 0.f) {
+            const CubicClosest r = closest_end(p, pt);
+            t = r.t;
+            d = r.dist;
+        }
+        const float dj = dist(ceval(p.p0, p.p1, p.p2, p.p3, tj), pt);
+        if (dj < d) {
+            d = dj;
+            t = tj;
+        }
+        return false;
     });
-    if (r.t < 0.f) {
-        const CubicPoints p = cubic_points(src);
-        r = closest_end(p.p0, p.p1, p.p2, p.p3, pt);
-    }
-    return r;
+    return t;
 }
 DVG_DEV CubicClosest cubic_closest(const float4 *src, V2 pt) {
-    const CubicPoints c = cubic_points(src);
-    const CubicClosest r = cubic_closest_fast(c.p0, c.p1, c.p2, c.p3, pt);
-    return r.t >= 0.f ? r : cubic_closest_plain(src, pt);
+    CubicClosest r = cubic_closest_fast(src, pt);
+    if (r.t < 0.f) {
+        r.t = cubic_closest_plain(src, pt);
+        const CubicPoints p = cubic_points(src);
+        if (r.t < 0.f) {  // no root: an end
+            r = closest_end(p, pt);
+        } else {
+            r.pt = ceval(p.p0, p.p1, p.p2, p.p3, r.t);
+            r.dist = dist(r.pt, pt);
+        }
+    }
+    return r;
 }
 
 // closest_point for a path (compute_distance.h:27-300): the segments in the reference's

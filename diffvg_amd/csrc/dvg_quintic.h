@@ -113,9 +113,11 @@ DVG_Q Quintic cubic_quintic(const QuinticSums &u) {
     const double A = u.A, inv = 1.0 / A;
     return Quintic{A, u.B * inv, u.C * inv, u.D * inv, u.E * inv, u.F * inv};
 }
-constexpr double kQuinticLarge = 1e6;
-DVG_Q bool quintic_large(const Quintic &q) {  // also when a coefficient is not a number
-    return !(fmax(fmax(fabs(q.B), fabs(q.C)), fmax(fmax(fabs(q.D), fabs(q.E)), fabs(q.F))) < kQuinticLarge);
+constexpr float kQuinticLarge = 1e6f;
+// also when the leading coefficient is 0 or one is not a number
+DVG_Q bool quintic_large(const QuinticSums &u) {
+    const float m = fmaxf(fmaxf(fabsf(u.B), fabsf(u.C)), fmaxf(fmaxf(fabsf(u.D), fabsf(u.E)), fabsf(u.F)));
+    return !(m < kQuinticLarge * u.A);
 }
 DVG_Q double quintic_eval(const Quintic &q, double t) {
     return __builtin_fma(__builtin_fma(__builtin_fma(__builtin_fma(t + q.B, t, q.C), t, q.D), t, q.E), t, q.F);

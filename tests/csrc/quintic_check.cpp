@@ -47,15 +47,14 @@ float renderer_distance(const V2 *p, V2 pt, int64_t &large) {
         best = std::fmin(best, at(p, pt, t));
         return false;
     };
-    const Quintic q = cubic_quintic(u);
-    if (quintic_large(q)) {
+    if (quintic_large(u)) {
         const Quintic v = cubic_quintic_plain(u);
         float iv[4];
         const int n = quintic_intervals_plain(v, iv);
         quintic_search_plain(v, iv, n, visit);
         large++;
     } else {
-        quintic_search(q, visit);
+        quintic_search(cubic_quintic(u), visit);
     }
     return std::sqrt(best);
 }
