@@ -44,8 +44,11 @@ constexpr int kEdgeChunk = kBlock / 2;
 constexpr int kWaveChunk = 64;  // of the wave-cooperative kernel, one wave
 // fragment lists kept from a colour forward for its backward: up to kFragSlots fragments
 // per sample (a sample with more is shaded again), at most kFragCacheBytes per scene.  24
-// slots instead of 16: one sample of more makes its whole tile wait for the shading; 2048
-// strokes at 512x512 585 -> 316 us, with memory for as many samples as 16 slots had in 512 MiB
+// slots instead of 16, 50 bytes a sample instead of 34: one sample of more makes its whole tile
+// wait for the shading.  Colour backward of 2048 strokes at 512x512 547 -> 314 us, of 256 uneven
+// scenes as a batch 4.70 -> 3.73 ms, of 300 paths and smaller drawings the same.  768 MiB hold
+// the lists of as many samples (16 million) as 512 MiB did with 16 slots; prefiltered lists
+// (292 bytes a sample) share the limit and are kept up to 2.76 million samples.
 constexpr int kFragSlots = 24;
 constexpr size_t kFragCacheBytes = size_t(768) << 20;
 constexpr int kFragMaxGroups = 32768;  // group ids 2 g + is_stroke are kept in 16 bits
@@ -54,13 +57,14 @@ constexpr int kFragMaxGroups = 32768;  // group ids 2 g + is_stroke are kept in 
 constexpr int kPFragSlots = 8;
 constexpr int kPFragWords = 9;
 // Boundary adjoints of circles, ellipses and rects (three or four parameters each) are
-// combined across a wave's lanes, up to this many samples per shape of the scene: 40 shapes
-// at 333x217, 3x2 samples: k_edge 3.34 -> 0.24 ms.  Past it every lane adds its own, as
-// before (~12 ns per sample: 10 ms for one circle and 262,144 samples, 0.9 combined),
-// because there the two forms differ by more than float rounding of one sum: adding N terms
-// of one sign one by one loses up to 2.3e-5 of the sum at 9,000 samples, 5e-5 at 32,000,
-// 3.4e-4 at 262,144 (12-60 seeds), and results of large few-primitive renders are kept as
-// they were.
+// combined across a wave's lanes while a render has at most this many boundary samples per
+// shape, on average over the scene's shapes (samples are drawn by boundary length: one long
+// circle among many short paths may get more than that and is still combined): 40 shapes at
+// 333x217, 3x2 samples: k_edge 3.34 -> 0.24 ms.  Past it every lane adds its own, ~12 ns per
+// sample (10 ms for one circle and 262,144 samples, 0.9 combined).  The line is not one of
+// accuracy: the combined sum is the nearer one, adding N terms of one sign one by one loses up
+// to 2.3e-5 of the sum at 9,000 samples, 5e-5 at 32,000 and 3.4e-4 at 262,144 (12-60 seeds).  It
+// keeps the results of large renders of few primitives what they have been.
 constexpr int64_t kPrimDirect = 12288;
 // Waves per SIMD each heavy shading kernel is compiled for, i.e. its register budget
 // (512 / waves VGPRs per lane; beyond it the compiler spills to scratch), chosen by
@@ -77,11 +81,13 @@ constexpr int64_t kPrimDirect = 12288;
 #ifndef DVG_WAVES_EDGE_WAVE
 #define DVG_WAVES_EDGE_WAVE 5
 #endif
-// the per-lane tests (scenes with groups of several shapes).  k_edge: 300 paths in groups of two,
-// 600 strokes in groups of three and 2,048 strokes in groups of two, all at 512x512: backward
-// 1.96 / 2.88 / 6.95 ms at 5 waves, 2.15 / 3.14 / 7.64 at 4; at 6 it spills in the loop over the
-// segments (strokes 7.6).  The others as measured before the double-precision searches were
-// called rather than inlined.
+// the per-lane tests (scenes with groups of several shapes).  300 paths in groups of two, 600
+// strokes in groups of three and 2,048 strokes in groups of two, all at 512x512: backward (k_edge
+// most of it) 1.95 / 2.86 / 6.89 ms at 5 waves, 2.15 / 3.14 / 7.64 at 4, at 6 it spills in the
+// loop over the segments (600 strokes: 7.6); forward (k_color) 0.60 / 0.95 / 2.31 at 5, 0.66 /
+// 1.02 / 2.49 at 3 and 4, 0.87 / 3.96 / 10.9 at 6.  64 scenes of 2 to 65 paths in groups of two
+// at 96x96 as a batch: kb_color 0.69 at 2, 3 and 4, 0.66 at 5 (0.39 to 0.40 at each with half of
+// the scenes on the wave-cooperative kernels), backward 2.30 at 5, 2.46 at 4, 2.68 at 6
 #ifndef DVG_WAVES_COLOR
 #define DVG_WAVES_COLOR 5
 #endif
@@ -117,8 +123,7 @@ constexpr int64_t kPrimDirect = 12288;
 #ifndef DVG_WAVES_COLOR_BWD_PRE
 #define DVG_WAVES_COLOR_BWD_PRE 3
 #endif
-// distance field of 300 paths at 256x256, forward + backward: 1.31 ms at 4 waves, 1.34 at 5,
-// 1.43 at 6
+// distance field of 300 paths in groups of two at 256x256, forward: 2.20 ms at 4 waves, 2.29 at 5
 #ifndef DVG_WAVES_SDF
 #define DVG_WAVES_SDF 4
 #endif
