@@ -288,14 +288,20 @@ DVG_DEV bool within_at(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float t, float r0, flo
     float rr = (tt * tt * tt) * r0 + (3 * tt * tt * t) * r1 + (3 * tt * t * t) * r2 + (t * t * t) * r3;
     return dist_sq(ceval(p0, p1, p2, p3, t), pt) < rr * rr;
 }
-// 0 or 1; 2: the coefficients are large and the plain search decides
-static __device__ __noinline__ int cubic_stroke_fast(V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2,
-                                                     float r3) {
-    const QuinticSums u = quintic_sums(p0, p1, p2, p3, pt);
-    if (quintic_large(u)) return 2;
+// 0 or 1; 2: the roots hang on rounding and the plain search decides.  The points are read again
+// where the roots are tested, as in plain_search.
+static __device__ __noinline__ int cubic_stroke_fast(const float4 *src, V2 pt, float r0, float r1, float r2, float r3) {
+    const CubicPoints c = cubic_points(src);
+    const QuinticSums u = quintic_sums(c.p0, c.p1, c.p2, c.p3, pt);
+    const QuinticScale scale = quintic_scale(u);
+    if (scale.large(u.A)) return 2;
+    asm volatile("" : "+v"(src));
     bool hit = false;
-    quintic_search(cubic_quintic(u), [&](float t) { return hit = within_at(p0, p1, p2, p3, pt, t, r0, r1, r2, r3); });
-    return hit;
+    const bool done = quintic_search(cubic_quintic(u), scale, [&](float t) {
+        const CubicPoints p = cubic_points(src);
+        return hit = within_at(p.p0, p.p1, p.p2, p.p3, pt, t, r0, r1, r2, r3);
+    });
+    return done ? hit : 2;
 }
 static __device__ __noinline__ bool cubic_stroke_plain(const float4 *src, V2 pt, float r0, float r1, float r2, float r3) {
     bool hit = false;
@@ -304,10 +310,9 @@ static __device__ __noinline__ bool cubic_stroke_plain(const float4 *src, V2 pt,
     });
     return hit;
 }
-// of the segment whose points, p0 to p3, lie at src
-DVG_DEV bool cubic_stroke_search(const float4 *src, V2 p0, V2 p1, V2 p2, V2 p3, V2 pt, float r0, float r1, float r2,
-                                 float r3) {
-    const int hit = cubic_stroke_fast(p0, p1, p2, p3, pt, r0, r1, r2, r3);
+// of the segment whose points lie at src
+DVG_DEV bool cubic_stroke_search(const float4 *src, V2 pt, float r0, float r1, float r2, float r3) {
+    const int hit = cubic_stroke_fast(src, pt, r0, r1, r2, r3);
     return hit != 2 ? hit : cubic_stroke_plain(src, pt, r0, r1, r2, r3);
 }
 
@@ -376,7 +381,7 @@ DVG_DEV int segment_within(const DevScene &S, int s, int seg, V2 pt, float r) {
     // every curve point certainly farther than the largest radius magnitude (the radius
     // at t is a convex combination of r0..r3): the quintic search below would find nothing
     if (cubic_farther_than(S, seg, pt, fmaxf(fmaxf(fabsf(r0), fabsf(r1)), fmaxf(fabsf(r2), fabsf(r3))))) return 0;
-    return cubic_stroke_search(cubic_points_at(S, seg), p0, p1, p2, p3, pt, r0, r1, r2, r3);
+    return cubic_stroke_search(cubic_points_at(S, seg), pt, r0, r1, r2, r3);
 }
 
 DVG_DEV bool within_distance_path(const DevScene &S, int s, V2 pt, float r) {
@@ -499,31 +504,28 @@ DVG_DEV CubicClosest closest_end(const CubicPoints &p, V2 pt) {
     float d0 = dist(pt0, pt), d1 = dist(pt1, pt);
     return d1 < d0 ? CubicClosest{d1, 1.f, pt1} : CubicClosest{d0, 0.f, pt0};
 }
-// t = -1: the coefficients are large and the plain search decides
+// t = -1: the roots hang on rounding and the plain search decides
 static __device__ __noinline__ CubicClosest cubic_closest_fast(const float4 *src, V2 pt) {
-    const CubicPoints p = cubic_points(src);
-    const QuinticSums u = quintic_sums(p.p0, p.p1, p.p2, p.p3, pt);
-    CubicClosest r = closest_end(p, pt);
-    if (quintic_large(u))
-        r.t = -1.f;
-    else
-        quintic_search(cubic_quintic(u), [&](float t) {
-            V2 pp = ceval(p.p0, p.p1, p.p2, p.p3, t);
-            float dp = dist(pp, pt);
-            if (dp < r.dist) r = CubicClosest{dp, t, pp};
-            return false;
-        });
+    const CubicPoints c = cubic_points(src);
+    const QuinticSums u = quintic_sums(c.p0, c.p1, c.p2, c.p3, pt);
+    const QuinticScale scale = quintic_scale(u);
+    CubicClosest r = closest_end(c, pt);
+    asm volatile("" : "+v"(src));
+    const auto visit = [&](float t) {
+        const CubicPoints p = cubic_points(src);
+        V2 pp = ceval(p.p0, p.p1, p.p2, p.p3, t);
+        float dp = dist(pp, pt);
+        if (dp < r.dist) r = CubicClosest{dp, t, pp};
+        return false;
+    };
+    if (scale.large(u.A) || !quintic_search(cubic_quintic(u), scale, visit)) r.t = -1.f;
     return r;
 }
 // the closest point's t
 static __device__ __noinline__ float cubic_closest_plain(const float4 *src, V2 pt) {
-    float t = -1.f, d = 0.f;
+    const CubicClosest end = closest_end(cubic_points(src), pt);
+    float d = end.dist, t = end.t;
     plain_search(src, pt, [&](const CubicPoints &p, float tj) {
-        if (t < 0.f) {
-            const CubicClosest r = closest_end(p, pt);
-            t = r.t;
-            d = r.dist;
-        }
         const float dj = dist(ceval(p.p0, p.p1, p.p2, p.p3, tj), pt);
         if (dj < d) {
             d = dj;
@@ -538,12 +540,8 @@ DVG_DEV CubicClosest cubic_closest(const float4 *src, V2 pt) {
     if (r.t < 0.f) {
         r.t = cubic_closest_plain(src, pt);
         const CubicPoints p = cubic_points(src);
-        if (r.t < 0.f) {  // no root: an end
-            r = closest_end(p, pt);
-        } else {
-            r.pt = ceval(p.p0, p.p1, p.p2, p.p3, r.t);
-            r.dist = dist(r.pt, pt);
-        }
+        r.pt = ceval(p.p0, p.p1, p.p2, p.p3, r.t);
+        r.dist = dist(r.pt, pt);
     }
     return r;
 }

@@ -6,6 +6,7 @@
 #pragma once
 
 #include <cmath>
+#include <cstdint>
 
 #if defined(__HIPCC__)
 #include <hip/hip_runtime.h>
@@ -78,14 +79,20 @@ DVG_Q int solve_cubic_d(double a, double b, double c, double d, double t[3]) {
 // strokes took half of the edge kernel: 17 double divisions, three cosines, a power and 45
 // double operations a Newton step for each.)
 //
-// Where the normalised coefficients are large those roundings decide: the curve is nearly a
-// quadratic or a line (a quadratic written as a cubic has coefficients of 1e9 to 1e17, made of
-// the rounding of its float coordinates), its quintic cancels at the interval ends, and whether
-// two ends have the same sign, so whether the reference finds the closest point at all, is a
-// matter of the last bit.  1.4e-4 of the points near such strokes were covered otherwise than
-// in the reference; none in 4 million up to coefficients of 1e7.  From kQuinticLarge on the
-// reference's own operations are used (quintic_search_plain): 300 strokes of three such segments
-// at 256x256, 4 samples, take 0.21 ms forward and 0.44 backward, 0.14 and 0.30 without them.
+// Whether the reference finds a root, so perhaps the closest point at all, can hang on those last
+// bits, and then its own operations are used (quintic_search_plain):
+//   * where the normalised coefficients are large (kQuinticLarge).  The curve is nearly a quadratic
+//     or a line -- a quadratic written as a cubic has coefficients of 1e9 to 1e17, made of the
+//     rounding of its float coordinates -- and the interval ends are rounding too.  1.4e-4 of the
+//     points near such strokes were covered otherwise; none in 4 million up to coefficients of 1e7;
+//   * where the quintic at an interval end is zero to rounding, or the cubic's roots are double
+//     (kQuinticOpen): curves through points A and B only, as A B B B (handles on an end), have
+//     multiple roots in both polynomials.  2.9e-3 of the points near A B B B were covered
+//     otherwise.  Of ordinary curves 3e-5 of the points come here.
+// With both, no decision differs over 30 million cases of 30 families of curves.  Looking for them
+// costs 2% of a pass over 2,048 strokes and 5% of a distance field; 300 strokes of three
+// quadratics written as cubics at 256x256, 4 samples, take 0.21 ms forward and 0.43 backward
+// instead of 0.14 and 0.30.
 struct Quintic {
     double A, B, C, D, E, F;  // leading coefficient, and the others divided by it
 };
@@ -114,10 +121,17 @@ DVG_Q Quintic cubic_quintic(const QuinticSums &u) {
     return Quintic{A, u.B * inv, u.C * inv, u.D * inv, u.E * inv, u.F * inv};
 }
 constexpr float kQuinticLarge = 1e6f;
-// also when the leading coefficient is 0 or one is not a number
-DVG_Q bool quintic_large(const QuinticSums &u) {
-    const float m = fmaxf(fmaxf(fabsf(u.B), fabsf(u.C)), fmaxf(fmaxf(fabsf(u.D), fabsf(u.E)), fabsf(u.F)));
-    return !(m < kQuinticLarge * u.A);
+constexpr float kQuinticOpen = 1e-9f;
+// What tells that the roots of a quintic hang on rounding, from its sums: the sum of the
+// coefficients' magnitudes and whether the derivative vanishes at 1 beside it.
+struct QuinticScale {
+    float size;
+    bool flat_end;
+    DVG_Q bool large(float A) const { return !(size < kQuinticLarge * A); }  // also for A = 0, not a number
+};
+DVG_Q QuinticScale quintic_scale(const QuinticSums &u) {
+    const float size = u.A + (fabsf(u.B) + fabsf(u.C)) + (fabsf(u.D) + fabsf(u.E)) + fabsf(u.F);
+    return QuinticScale{size, fabsf(5 * u.A + 4 * u.B + 3 * u.C + 2 * u.D + u.E) < 1e-4f * size};
 }
 DVG_Q double quintic_eval(const Quintic &q, double t) {
     return __builtin_fma(__builtin_fma(__builtin_fma(__builtin_fma(t + q.B, t, q.C), t, q.D), t, q.E), t, q.F);
@@ -151,17 +165,22 @@ DVG_Q void sincos_third(double x, double &s, double &c) {
     s = __builtin_fma(p * z, x, x);
     c = __builtin_fma(r, z, 1.0);
 }
-// Roots of a t^3 + b t^2 + c t + d as solve_cubic_d returns them (solve.h:29-64).
-DVG_Q int isolating_cubic(double a, double b, double c, double d, double (&t)[3]) {
-    if (fabs(a) < 1e-6f) return solve_quadratic_d(b, c, d, &t[0], &t[1]) ? 2 : 0;
+// Roots of a t^3 + b t^2 + c t + d as solve_cubic_d returns them (solve.h:29-64).  `open` is set
+// when two of them are so close that the number found hangs on rounding.
+DVG_Q int isolating_cubic(double a, double b, double c, double d, double (&t)[3], bool &open) {
+    if (fabs(a) < 1e-6f) {
+        open = !(fabs(c * c - 4 * b * d) > kQuinticOpen * (c * c));
+        return solve_quadratic_d(b, c, d, &t[0], &t[1]) ? 2 : 0;
+    }
     const double inv = 1.0 / a, third = 1.0 / 3.0;
     b *= inv;
     c *= inv;
     d *= inv;
     const double Q = (b * b - 3 * c) * (1.0 / 9.0);
     const double R = (2 * b * b * b - 9 * b * c + 27 * d) * (1.0 / 54.0);
-    const double Q3 = Q * Q * Q, b3 = b * third;
-    if (R * R < Q3) {
+    const double Q3 = Q * Q * Q, R2 = R * R, b3 = b * third;
+    open = !(fabs(R2 - Q3) > kQuinticOpen * R2);
+    if (R2 < Q3) {
         double s, co;
         sincos_third(acos(R / sqrt(Q3)) * third, s, co);
         const double h = 0.86602540378443864676 * s, m = -2.0 * __builtin_sqrt(Q);
@@ -170,7 +189,7 @@ DVG_Q int isolating_cubic(double a, double b, double c, double d, double (&t)[3]
         t[2] = m * (-0.5 * co + h) - b3;
         return 3;
     }
-    const double root = cbrt(fabs(R) + __builtin_sqrt(R * R - Q3));
+    const double root = cbrt(fabs(R) + __builtin_sqrt(R2 - Q3));
     const double A = R > 0 ? -root : root;
     const double B = fabs(A) > 1e-6f ? Q / A : 0.0;
     t[0] = (A + B) - b3;
@@ -201,7 +220,7 @@ DVG_Q int sort_intervals(bool first, float q_root, int num_sol, const double (&p
     return n;
 }
 // Isolating intervals (within_distance.h:195-216)
-DVG_Q int quintic_intervals(const Quintic &q, float (&iv)[4]) {
+DVG_Q int quintic_intervals(const Quintic &q, float (&iv)[4], bool &open) {
     // the reference's float fractions
     const double p1A = (2 / 5.f) * q.C - (4 / 25.f) * q.B * q.B;
     const double p1B = (3 / 5.f) * q.D - (3 / 25.f) * q.B * q.C;
@@ -209,7 +228,7 @@ DVG_Q int quintic_intervals(const Quintic &q, float (&iv)[4]) {
     const double p1D = q.F - q.B * q.E * (1.0 / 25.0);
     const double q_root = q.B * -0.2;
     double pr[3] = {0.0, 0.0, 0.0};
-    const int num_sol = isolating_cubic(p1A, p1B, p1C, p1D, pr);
+    const int num_sol = isolating_cubic(p1A, p1B, p1C, p1D, pr, open);
     return sort_intervals(q_root >= 0 && q_root <= 1, (float)q_root, num_sol, pr, iv);
 }
 // A first reciprocal, correct to about a float's precision
@@ -241,16 +260,23 @@ DVG_Q float quintic_root(const Quintic &q, float lb, float ub) {
     }
     return t;
 }
+// |x| by its upper half: enough to compare magnitudes, in one register
+DVG_Q uint32_t high_word(double x) {
+    uint64_t v;
+    __builtin_memcpy(&v, &x, sizeof(v));
+    return (uint32_t)(v >> 32) & 0x7fffffffu;
+}
 // Calls visit(t) for the root in each interval with a sign change, in order, until it
 // returns true.  The brackets are found first, so that the lanes of a wave run their first
-// searches together, then their second ones, whichever intervals those are.
+// searches together, then their second ones, whichever intervals those are.  False, and nothing
+// visited, when the signs at the interval ends hang on rounding.
 template <class Visit>
-DVG_Q void quintic_search(const Quintic &q, const Visit &visit) {
+DVG_Q bool quintic_search(const Quintic &q, const QuinticScale &scale, const Visit &visit) {
     float iv[4];
-    const int n = quintic_intervals(q, iv);
-    float lo[5], hi[5];
-    unsigned found = 0;
-    float lower = 0.f;
+    bool open = false;
+    const int n = quintic_intervals(q, iv, open);
+    const uint32_t small = high_word((double)(kQuinticOpen * scale.size) * (1.0 / q.A));
+    unsigned found = 0, falls = 0;  // intervals with a sign change, and those where it is downward
     double at_lower = quintic_eval(q, 0.0);
     bool more = true;
 #pragma unroll
@@ -260,25 +286,31 @@ DVG_Q void quintic_search(const Quintic &q, const Visit &visit) {
         const bool use = more && j <= n && !(inner && end < 0.f);
         const float upper = inner ? (end < 1.f ? end : 1.f) : 1.f;
         const double at_upper = quintic_eval(q, upper);
+        // at 1 a root of its own does no harm (a handle of no length has one)
+        const bool counts = j < 4 ? inner && end > -1e-5f && end < 1.00001f : scale.flat_end;
+        open = open || (counts && high_word(at_upper) < small);
         const bool change = use && !(at_lower * at_upper > 0);
-        const bool falls = at_lower > at_upper;
-        lo[j] = falls ? upper : lower;
-        hi[j] = falls ? lower : upper;
+        if (at_lower > at_upper) falls |= 1u << j;
         if (change) {
             found |= 1u << j;
             more = !(upper >= 1.f);
-            lower = upper;
             at_lower = at_upper;
         }
     }
+    if (open) return false;
+    float lower = 0.f;
 #pragma nounroll
     while (found) {
         const int j = __builtin_ctz(found);
         found &= found - 1;
-        const float lb = j < 2 ? (j == 0 ? lo[0] : lo[1]) : (j == 2 ? lo[2] : (j == 3 ? lo[3] : lo[4]));
-        const float ub = j < 2 ? (j == 0 ? hi[0] : hi[1]) : (j == 2 ? hi[2] : (j == 3 ? hi[3] : hi[4]));
+        const float end = j < 2 ? (j == 0 ? iv[0] : iv[1]) : (j == 2 ? iv[2] : iv[3]);
+        const float upper = j < 4 && j < n && end < 1.f ? end : 1.f;
+        const bool down = (falls >> j) & 1u;
+        const float lb = down ? upper : lower, ub = down ? lower : upper;
+        lower = upper;
         if (visit(quintic_root(q, lb, ub))) break;
     }
+    return true;
 }
 
 // The same with the reference's operations in the reference's order (within_distance.h:187-262)

@@ -131,8 +131,7 @@ DVG_DEV void wave_exact(const SceneRef &R, WaveLds<SIDES> &W, int &n2, int cnt) 
                         r3 = S.thickness[idx.w];
                     }
                     hit = dist_sq(c.p0, p) < r0 * r0 || dist_sq(c.p3, p) < r3 * r3;
-                    if (!hit)
-                        hit = cubic_stroke_search(cubic_points_at(S, seg), c.p0, c.p1, c.p2, c.p3, p, r0, r1, r2, r3);
+                    if (!hit) hit = cubic_stroke_search(cubic_points_at(S, seg), p, r0, r1, r2, r3);
                 } else {
                     hit = wave_within_lq(S, s, seg, k, p, r);
                 }

@@ -47,14 +47,13 @@ float renderer_distance(const V2 *p, V2 pt, int64_t &large) {
         best = std::fmin(best, at(p, pt, t));
         return false;
     };
-    if (quintic_large(u)) {
+    const QuinticScale scale = quintic_scale(u);
+    if (scale.large(u.A) || !quintic_search(cubic_quintic(u), scale, visit)) {
         const Quintic v = cubic_quintic_plain(u);
         float iv[4];
         const int n = quintic_intervals_plain(v, iv);
         quintic_search_plain(v, iv, n, visit);
         large++;
-    } else {
-        quintic_search(cubic_quintic(u), visit);
     }
     return std::sqrt(best);
 }
@@ -64,7 +63,8 @@ extern "C" {
 // mode 0: random; 1: straight, control points at thirds; 2: a quadratic written as a cubic;
 // 3: first handle of no length; 4: both handles of no length; 5: closed loop; 6: horizontal; 7:
 // large coordinates; 8: tiny; 9: a quadratic written as a cubic and moved by 1e-6 to 1; 10: an
-// arc as four-point circles have it, on whole coordinates, and its centre.
+// arc as four-point circles have it, on whole coordinates, and its centre; 11 to 15: with points
+// A and B only, A A A B, A B B B, A B A B, A B B A and one point; 16: second handle of no length.
 // Half of the points lie about one stroke radius from the curve.  out: cases, cases that take
 // the plain search, cases whose distances differ by more than 1e-3, cases that a stroke of that
 // radius covers in one but not in the other; worst: the largest difference of the distances.
@@ -90,6 +90,12 @@ void quintic_fuzz(int mode, int64_t n, uint64_t seed, int64_t *out, float *worst
         if (mode == 3 || mode == 4) p[1] = p[0];
         if (mode == 4) p[2] = p[3];
         if (mode == 5) p[3] = p[0];
+        if (mode >= 11 && mode <= 15) {
+            static const int order[5][4] = {{0, 0, 0, 1}, {0, 1, 1, 1}, {0, 1, 0, 1}, {0, 1, 1, 0}, {0, 0, 0, 0}};
+            const V2 ab[2] = {p[0], p[3]};
+            for (int k = 0; k < 4; k++) p[k] = ab[order[mode - 11][k]];
+        }
+        if (mode == 16) p[2] = p[3];
         for (V2 &x : p) {
             if (mode == 6) x = V2{cx + 3.f * (x.x - cx), cy};
             if (mode == 7) x = V2{40.f * x.x, 40.f * x.y};
