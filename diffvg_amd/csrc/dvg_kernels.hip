@@ -1819,7 +1819,10 @@ static bool keep_buffer(SceneHost &sc, void *&ptr, size_t &granted, hipStream_t 
 
 static bool is_capturing(hipStream_t st) {
     hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
-    return st && (hipStreamIsCapturing(st, &c) != hipSuccess || c != hipStreamCaptureStatusNone);
+    if (!st) return false;
+    if (hipStreamIsCapturing(st, &c) == hipSuccess) return c != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();  // a stream that is no more
+    return false;
 }
 
 // Whether a backward on stream `st` may add to the scene's gradient copies; one that may not
